@@ -307,6 +307,48 @@ def test_linear_gemms_bf16_operands(shape):
         assert e < 1e-5, name
 
 
+@pytest.mark.parametrize("form", ["fp32", "mixed", "bf16"])
+@pytest.mark.parametrize("shape,skew", [((1, 9, 17), 0), ((65, 129, 63), 0), ((130, 257, 1001), 0),
+                                        ((128, 64, 72), 1), ((2048, 264, 520), 1)])
+def test_linear_products_of_any_width_and_alignment(form, shape, skew):
+    """The three contractions on operands that need a packed copy (rows that are
+    not whole 16-byte chunks, addresses off by one element, fp32 operands in bf16
+    products) against float64 on the rounded operands.  Products of bf16 values are
+    exact in fp32, so only fp32 summation differs: with |terms| of one size, a sum
+    of n terms is off by at most n 2^-24 of its norm, and by about sqrt(n) 2^-24;
+    1e-6 + 4 sqrt(n) 2^-24 bounds every contraction here."""
+    from valkyr_amd import kernels as K
+
+    M, N, Kd = shape
+    note(f"linear {form} M={M} N={N} K={Kd} skew={skew}")
+    rng = np.random.default_rng(M + N + Kd)
+    host64, ptr, keep = {}, {}, []
+    for name, n in (("x", M * Kd), ("w", N * Kd), ("dy", M * N)):
+        a = rng.standard_normal(n + skew, dtype=np.float32)
+        if form == "bf16":
+            buf, a = bf16_dev(a)
+        else:
+            buf = dev(a)
+        if form == "mixed":
+            a = O.round_bf16(a)
+        keep.append(buf)
+        ptr[name] = buf.offset(skew * (2 if form == "bf16" else 4))
+        host64[name] = a[skew:].astype(np.float64)
+    x, w, dy = host64["x"].reshape(M, Kd), host64["w"].reshape(N, Kd), host64["dy"].reshape(M, N)
+    y, dx, dw = zeros(M * N), zeros(M * Kd), zeros(N * Kd)
+    if form == "bf16":
+        K.matmul_nt_bf16(ptr["x"], ptr["w"], y, M, N, Kd)
+        K.linear_backward_dx_bf16(ptr["dy"], ptr["w"], dx, M, N, Kd)
+        K.linear_backward_dw_bf16(ptr["dy"], ptr["x"], dw, M, N, Kd)
+    else:
+        p = 0 if form == "fp32" else 1
+        K.matmul_nt(ptr["x"], ptr["w"], y, M, N, Kd, p)
+        K.linear_backward_dx(ptr["dy"], ptr["w"], dx, M, N, Kd, p)
+        K.linear_backward_dw(ptr["dy"], ptr["x"], dw, M, N, Kd, p)
+    for n, ref, got in ((Kd, x @ w.T, y), (N, dy @ w, dx), (M, dy.T @ x, dw)):
+        assert rel_l2(ref, host(got)) < 1e-6 + 4 * math.sqrt(n) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("shape", [(2048, 3072, 1024), (2000, 3072, 1000), (256, 192, 128),
                                    (130, 100, 72)])
 def test_gate_up_swiglu_matches_two_passes(shape):

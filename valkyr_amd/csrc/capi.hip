@@ -356,70 +356,86 @@ vkh_status vkh_fa_backward_from_o(const vkh_attn_params *p, const void *q, const
 
 // ── GEMMs ──────────────────────────────────────────────────────────────
 
-// Split-K workspace for one call (stream-ordered allocation), if the plan wants one.
+// Workspace for one call.  Up to kLeaseMax it is the stream's kept scratch; more
+// is allocated in stream order and freed after the call's work.
+constexpr size_t kLeaseMax = 256ull << 20;
 extern "C++" {
 template <class F>
 static vkh_status with_ws(size_t bytes, hipStream_t st, const char *what, F &&f) {
     GemmWs ws{nullptr, bytes};
     ScratchLease lease;
-    if (ws.bytes) VKH_TRY(lease.acquire(ws.bytes, st, &ws.p));
+    const bool own = bytes > kLeaseMax;
+    if (own) {
+        note_allocation();
+        VKH_HIP(hipMallocAsync(&ws.p, bytes, st));
+    } else if (bytes) {
+        VKH_TRY(lease.acquire(bytes, st, &ws.p));
+    }
     const hipError_t e = f(ws);
+    if (own) (void)hipFreeAsync(ws.p, st);
     if (e != hipSuccess) return hip_fail(e, what);
     return VKH_OK;
 }
-template <class F>
-static vkh_status with_g16_ws(int M, int N, int K, hipStream_t st, const char *what, F &&f) {
-    return with_ws(g16_ws_bytes_for(M, N, K), st, what, f);
-}
 }
 
-// Precision FP32: the DMA-staged fp32 MFMA kernels (g32_*), which take the
-// generic kernel for operands outside their layout rules; BF16: operands
-// rounded to bf16 on their way into the generic kernel's LDS tiles.
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return cs != hipStreamCaptureStatusNone;
+}
+
+// One contraction of a linear layer.  Operands that need a packed copy (fp32
+// operands in the bf16 precision; rows that are not whole 16-byte chunks) go
+// through the workspace to the DMA-staged kernels; while the stream is being
+// captured they take the generic kernel, which needs none.  Against the generic
+// kernel, forward / dx / dW: 2048 tokens, 2560 x 2560, fp32 operands in bf16
+// products 55 / 55 / 63 us (645 / 443 / 351); bf16 operands of 2000 x 4100 x 4099
+// 156 / 143 / 117 us (455 / 638 / 533); fp32 of 1000 x 1500 x 3001 131 / 130 /
+// 117 us (205 / 156 / 211); 16 tokens, 1024 x 1024 mixed 15 / 15 / 8 us (41 / 29 / 7).
+static vkh_status linear(LinOp op, LinForm f, const void *a, const void *b, float *out, uint32_t M,
+                         uint32_t N, uint32_t K, const char *what, hipStream_t st) {
+    if (!M || !N || !K || (lin_packs(op, f, a, b, M, N, K) && capturing(st))) {
+        const Precision pr = f == LinForm::F32 ? Precision::FP32 : Precision::BF16;
+        const DType dt = f == LinForm::BF16 ? DType::BF16 : DType::F32;
+        const Mat ma{a, (long)(op == LinOp::NT ? K : N), dt}, mb{b, (long)K, dt};
+        if (op == LinOp::NT) VKH_HIP(gemm_nt(pr, ma, mb, out, N, M, N, K, nullptr, 0, 1.f, 0.f, st));
+        else if (op == LinOp::NN) VKH_HIP(gemm_nn(pr, ma, mb, out, K, M, N, K, 1.f, 0.f, st));
+        else VKH_HIP(gemm_tn(pr, ma, mb, out, K, M, N, K, 1.f, 0.f, st));
+        return VKH_OK;
+    }
+    return with_ws(lin_ws_bytes(op, f, a, b, M, N, K), st, what, [&](const GemmWs &ws) {
+        return lin_run(op, f, a, b, out, M, N, K, ws, st);
+    });
+}
+static inline LinForm form_of(uint32_t precision) {
+    return PR(precision) == Precision::FP32 ? LinForm::F32 : LinForm::MIXED;
+}
+
 vkh_status vkh_matmul_nt(const float *x, const float *w, float *y, uint32_t M, uint32_t N,
                          uint32_t K, uint32_t precision, vkh_stream stream) {
     CHECK_ARG(x && w && y, "null pointer");
-    hipStream_t st = S(stream);
-    if (PR(precision) == Precision::FP32)
-        return with_ws(g32_ws_bytes_for(M, N, K), st, "matmul_nt", [&](const GemmWs &ws) {
-            return g32_nt(x, K, w, K, y, N, M, N, K, nullptr, 0, 1.f, 0.f, ws, st);
-        });
-    VKH_HIP(gemm_nt(PR(precision), matf(x, K), matf(w, K), y, N, M, N, K, nullptr, 0, 1.f, 0.f, st));
-    return VKH_OK;
+    return linear(LinOp::NT, form_of(precision), x, w, y, M, N, K, "matmul_nt", S(stream));
 }
 
 vkh_status vkh_linear_backward_dx(const float *dy, const float *w, float *dx, uint32_t M,
                                   uint32_t N, uint32_t K, uint32_t precision, vkh_stream stream) {
     CHECK_ARG(dy && w && dx, "null pointer");
-    hipStream_t st = S(stream);
-    if (PR(precision) == Precision::FP32)
-        return with_ws(g32_ws_bytes_for(M, K, N), st, "linear_backward_dx", [&](const GemmWs &ws) {
-            return g32_nn(dy, N, w, K, dx, K, M, N, K, 1.f, 0.f, ws, st);
-        });
-    VKH_HIP(gemm_nn(PR(precision), matf(dy, N), matf(w, K), dx, K, M, N, K, 1.f, 0.f, st));
-    return VKH_OK;
+    return linear(LinOp::NN, form_of(precision), dy, w, dx, M, N, K, "linear_backward_dx", S(stream));
 }
 
 vkh_status vkh_linear_backward_dw(const float *dy, const float *x, float *dw, uint32_t M,
                                   uint32_t N, uint32_t K, uint32_t precision, vkh_stream stream) {
     CHECK_ARG(dy && x && dw, "null pointer");
-    hipStream_t st = S(stream);
-    if (PR(precision) == Precision::FP32)
-        return with_ws(g32_ws_bytes_for(N, K, M), st, "linear_backward_dw", [&](const GemmWs &ws) {
-            return g32_tn(dy, N, x, K, dw, K, M, N, K, 1.f, 0.f, ws, st);
-        });
-    VKH_HIP(gemm_tn(PR(precision), matf(dy, N), matf(x, K), dw, K, M, N, K, 1.f, 0.f, st));
-    return VKH_OK;
+    return linear(LinOp::TN, form_of(precision), dy, x, dw, M, N, K, "linear_backward_dw", S(stream));
 }
 
 vkh_status vkh_matmul_nt_bf16(const void *x, const void *w, float *y, uint32_t M, uint32_t N,
                               uint32_t K, vkh_stream stream) {
     CHECK_ARG(x && w && y, "null pointer");
-    hipStream_t st = S(stream);
-    return with_g16_ws(M, N, K, st, "matmul_nt_bf16", [&](const GemmWs &ws) {
-        return g16_nt((const bf16 *)x, K, (const bf16 *)w, K, y, N, M, N, K, nullptr, 0, 1.f, 0.f,
-                      ws, st);
-    });
+    return linear(LinOp::NT, LinForm::BF16, x, w, y, M, N, K, "matmul_nt_bf16", S(stream));
 }
 
 vkh_status vkh_gate_up_swiglu_bf16(const void *x, const void *w_gu, float *gu, void *gated,
@@ -462,19 +478,13 @@ vkh_status vkh_gate_up_swiglu(const float *x, const float *w_gu, float *gu, floa
 vkh_status vkh_linear_backward_dx_bf16(const void *dy, const void *w, float *dx, uint32_t M,
                                        uint32_t N, uint32_t K, vkh_stream stream) {
     CHECK_ARG(dy && w && dx, "null pointer");
-    hipStream_t st = S(stream);
-    return with_g16_ws(M, K, N, st, "linear_backward_dx_bf16", [&](const GemmWs &ws) {
-        return g16_nn((const bf16 *)dy, N, (const bf16 *)w, K, dx, K, M, N, K, 1.f, 0.f, ws, st);
-    });
+    return linear(LinOp::NN, LinForm::BF16, dy, w, dx, M, N, K, "linear_backward_dx_bf16", S(stream));
 }
 
 vkh_status vkh_linear_backward_dw_bf16(const void *dy, const void *x, float *dw, uint32_t M,
                                        uint32_t N, uint32_t K, vkh_stream stream) {
     CHECK_ARG(dy && x && dw, "null pointer");
-    hipStream_t st = S(stream);
-    return with_g16_ws(N, K, M, st, "linear_backward_dw_bf16", [&](const GemmWs &ws) {
-        return g16_tn((const bf16 *)dy, N, (const bf16 *)x, K, dw, K, M, N, K, 1.f, 0.f, ws, st);
-    });
+    return linear(LinOp::TN, LinForm::BF16, dy, x, dw, M, N, K, "linear_backward_dw_bf16", S(stream));
 }
 
 vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, const float *b,
@@ -484,7 +494,7 @@ vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, cons
     CHECK_ARG(r > 0, "rank 0");
     const Precision pr = PR(precision);
     hipStream_t st = S(stream);
-    VKH_HIP(gemm_nt(pr, matf(x, K), matf(w, K), y, N, M, N, K, nullptr, 0, 1.f, 0.f, st));
+    VKH_TRY(linear(LinOp::NT, form_of(precision), x, w, y, M, N, K, "lora_forward", st));
     // rank-r kernels (fp32 factors and products) where the shape allows
     LoraSegs sa, sb;
     sa.n = sb.n = 1;
@@ -509,6 +519,7 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
     const Precision pr = PR(precision);
     hipStream_t st = S(stream);
     float *dyB = nullptr;
+    vkh_status base = VKH_OK;  // of the base product
     note_allocation();
     VKH_HIP(hipMallocAsync((void **)&dyB, (size_t)M * r * 4 + 256, st));
     LoraSegs sb, sa, sdA, sdB;
@@ -521,20 +532,22 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
         lora_fast_ok(DType::F32, dy, N, (int)r, sdB) && (!dx || lora_update_ok(dx, K, (int)r, sa))) {
         // rank-r kernels (fp32 factors and products)
         hipError_t e = lora_rows(DType::F32, dy, N, (int)M, (int)r, sb, 1.f, st);
-        if (e == hipSuccess && dx) e = gemm_nn(pr, matf(dy, N), matf(w, K), dx, K, M, N, K, 1.f, 0.f, st);
-        if (e == hipSuccess && dx) e = lora_update(dx, K, (int)M, (int)r, sa, aor, st);
+        if (e == hipSuccess && dx) base = linear(LinOp::NN, form_of(precision), dy, w, dx, M, N, K, "lora_backward", st);
+        if (e == hipSuccess && base == VKH_OK && dx) e = lora_update(dx, K, (int)M, (int)r, sa, aor, st);
         if (e == hipSuccess) e = lora_cols(DType::F32, x, K, (int)M, (int)r, sdA, aor, st);
         if (e == hipSuccess) e = lora_cols(DType::F32, dy, N, (int)M, (int)r, sdB, aor, st);
         (void)hipFreeAsync(dyB, st);
+        if (base != VKH_OK) return base;
         if (e != hipSuccess) return hip_fail(e, "lora_backward");
         return VKH_OK;
     }
     hipError_t e = gemm_nn(pr, matf(dy, N), matf(b, r), dyB, r, M, N, r, 1.f, 0.f, st);
-    if (e == hipSuccess && dx) e = gemm_nn(pr, matf(dy, N), matf(w, K), dx, K, M, N, K, 1.f, 0.f, st);
-    if (e == hipSuccess && dx) e = gemm_nn(pr, matf(dyB, r), matf(a, K), dx, K, M, r, K, aor, 1.f, st);
+    if (e == hipSuccess && dx) base = linear(LinOp::NN, form_of(precision), dy, w, dx, M, N, K, "lora_backward", st);
+    if (e == hipSuccess && base == VKH_OK && dx) e = gemm_nn(pr, matf(dyB, r), matf(a, K), dx, K, M, r, K, aor, 1.f, st);
     if (e == hipSuccess) e = gemm_tn(pr, matf(dyB, r), matf(x, K), dA, K, M, r, K, aor, 0.f, st);
     if (e == hipSuccess) e = gemm_tn(pr, matf(dy, N), matf(inter, r), dB, r, M, N, r, aor, 0.f, st);
     (void)hipFreeAsync(dyB, st);
+    if (base != VKH_OK) return base;
     if (e != hipSuccess) return hip_fail(e, "lora_backward");
     return VKH_OK;
 }

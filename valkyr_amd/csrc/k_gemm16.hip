@@ -586,6 +586,152 @@ hipError_t g32_tn(const float *dy, long lddy, const float *x, long ldx, float *d
     return run32<Lay::MN, Lay::MN>(a, b, GemmShape{N, K, M}, e, ws, st);
 }
 
+// ── linear products of any operand form ────────────────────────────────
+namespace {
+
+// One operand's packed copy: dst[r][0 .. V chunks) = src[r][0 .. run), then zeros.
+struct PackSeg {
+    const void *src;
+    void *dst;
+    size_t n;         // 16-byte chunks of dst
+    unsigned chunks;  // ... per row
+    int run;
+};
+
+// Copies of one or two operands whose rows become whole 16-byte chunks of TD.
+// One 16-byte store per thread; the source is read in vector loads at its
+// element alignment (global loads need no more on gfx950).  Bound by HBM: a
+// [151936, 1024] fp32 -> bf16 pack takes 190 us (933 MB, 4.9 TB/s).  Both
+// operands go in one launch: a launch costs more than a small pack (64 x 256:
+// 10.4 us for a product with two pack launches before it, 8.7 with one).
+template <typename TS, typename TD>
+__global__ __launch_bounds__(256) void pack_rows_k(PackSeg s0, PackSeg s1) {
+    constexpr int V = 16 / sizeof(TD);
+    typedef TD vec_t __attribute__((ext_vector_type(V)));
+    const size_t stride = (size_t)gridDim.x * 256, n = s0.n + s1.n;
+    for (size_t j = (size_t)blockIdx.x * 256 + threadIdx.x; j < n; j += stride) {
+        const bool second = j >= s0.n;
+        const PackSeg &s = second ? s1 : s0;
+        const size_t i = second ? j - s0.n : j, r = i / s.chunks;
+        const int c = (int)(i - r * s.chunks) * V;
+        const TS *p = (const TS *)s.src + r * s.run + c;
+        TS t[V];
+        if (c + V <= s.run) {
+            __builtin_memcpy(t, p, sizeof(t));
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e) t[e] = c + e < s.run ? p[e] : (TS)0.f;
+        }
+        vec_t v;
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = (TD)(float)t[e];
+        reinterpret_cast<vec_t *>(s.dst)[i] = v;
+    }
+}
+
+template <typename TS, typename TD>
+hipError_t pack_rows(const PackSeg &s0, const PackSeg &s1, hipStream_t st) {
+    const size_t n = s0.n + s1.n;
+    if (!n) return hipSuccess;
+    hipLaunchKernelGGL((pack_rows_k<TS, TD>), dim3((unsigned)std::min<size_t>((n + 255) / 256, 65536)),
+                       dim3(256), 0, st, s0, s1);
+    return hipGetLastError();
+}
+
+int chunk_elems(LinForm f) { return f == LinForm::F32 ? 4 : 8; }
+size_t packed_bytes(LinForm f, long rows, long run) {
+    const size_t v = chunk_elems(f), b = (run + v - 1) / v * 16 * (size_t)rows;
+    return (b + 255) / 256 * 256;
+}
+bool needs_pack(LinForm f, const void *p, long run) {
+    return f == LinForm::MIXED || ((uintptr_t)p & 15u) || run % chunk_elems(f);
+}
+
+struct LinDims {
+    long ra, ca, rb, cb;  // rows and contiguous run of the two operands
+    GemmShape s;          // the product
+};
+LinDims lin_dims(LinOp op, int M, int N, int K) {
+    if (op == LinOp::NT) return {M, K, N, K, {M, N, K}};
+    if (op == LinOp::NN) return {M, N, N, K, {M, K, N}};
+    return {M, N, M, K, {N, K, M}};
+}
+size_t lin_split_bytes(LinForm f, const GemmShape &s) {
+    return f == LinForm::F32 ? g32_ws_bytes_for(s.M, s.N, s.K) : g16_ws_bytes_for(s.M, s.N, s.K);
+}
+
+}  // namespace
+
+bool lin_packs(LinOp op, LinForm f, const void *a, const void *b, int M, int N, int K) {
+    const LinDims d = lin_dims(op, M, N, K);
+    return needs_pack(f, a, d.ca) || needs_pack(f, b, d.cb);
+}
+
+size_t lin_ws_bytes(LinOp op, LinForm f, const void *a, const void *b, int M, int N, int K) {
+    const LinDims d = lin_dims(op, M, N, K);
+    return (needs_pack(f, a, d.ca) ? packed_bytes(f, d.ra, d.ca) : 0) +
+           (needs_pack(f, b, d.cb) ? packed_bytes(f, d.rb, d.cb) : 0) + lin_split_bytes(f, d.s);
+}
+
+// Packs the operands whose `rows` are not 0 (dense rows of `run` elements).
+hipError_t lin_pack(LinForm f, const void *a, long ra, long ca, void *da, const void *b, long rb,
+                    long cb, void *db, hipStream_t st) {
+    const long v = chunk_elems(f);
+    auto seg = [&](const void *p, long rows, long run, void *dst) {
+        const unsigned ch = (unsigned)((run + v - 1) / v);
+        return PackSeg{p, dst, (size_t)rows * ch, ch ? ch : 1, (int)run};
+    };
+    const PackSeg s0 = seg(a, ra, ca, da), s1 = seg(b, rb, cb, db);
+    if (f == LinForm::MIXED) return pack_rows<float, bf16>(s0, s1, st);
+    if (f == LinForm::F32) return pack_rows<float, float>(s0, s1, st);
+    return pack_rows<bf16, bf16>(s0, s1, st);
+}
+
+hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out, int M, int N, int K,
+                   const GemmWs &ws, hipStream_t st) {
+    const LinDims d = lin_dims(op, M, N, K);
+    const long v = chunk_elems(f);
+    char *w = (char *)ws.p;
+    long lda = d.ca, ldb = d.cb;
+    const bool pa = needs_pack(f, a, d.ca), pb = needs_pack(f, b, d.cb);
+    if (pa || pb) {
+        void *da = w, *db = w + (pa ? packed_bytes(f, d.ra, d.ca) : 0);
+        const hipError_t e = lin_pack(f, a, pa ? d.ra : 0, d.ca, da, b, pb ? d.rb : 0, d.cb, db, st);
+        if (e != hipSuccess) return e;
+        w = (char *)db + (pb ? packed_bytes(f, d.rb, d.cb) : 0);
+        if (pa) a = da, lda = (d.ca + v - 1) / v * v;
+        if (pb) b = db, ldb = (d.cb + v - 1) / v * v;
+    }
+    const GemmWs rest{w, ws.p ? ws.bytes - (size_t)(w - (char *)ws.p) : 0};
+    // views of 2 GiB and more go through g16_* / g32_* (row chunks or the generic kernel)
+    const int es = f == LinForm::F32 ? 4 : 2;
+    const size_t ba = ((size_t)(d.ra - 1) * lda + (lda > d.ca ? lda : d.ca)) * es,
+                 bb = ((size_t)(d.rb - 1) * ldb + (ldb > d.cb ? ldb : d.cb)) * es;
+    if (ba < (1ull << 31) && bb < (1ull << 31)) {
+        // both aligned now; the zeros past a packed row's run are part of its chunks
+        const Op16 oa{(const bf16 *)a, lda, (unsigned)ba}, ob{(const bf16 *)b, ldb, (unsigned)bb};
+        const EpiStore ep{out, d.s.N, nullptr, 0, 1.f, 0.f};
+        if (f == LinForm::F32) {
+            if (op == LinOp::NT) return run32<Lay::K, Lay::K>(oa, ob, d.s, ep, rest, st);
+            if (op == LinOp::NN) return run32<Lay::K, Lay::MN>(oa, ob, d.s, ep, rest, st);
+            return run32<Lay::MN, Lay::MN>(oa, ob, d.s, ep, rest, st);
+        }
+        if (op == LinOp::NT) return run16<Lay::K, Lay::K>(oa, ob, d.s, ep, rest, st);
+        if (op == LinOp::NN) return run16<Lay::K, Lay::MN>(oa, ob, d.s, ep, rest, st);
+        return run16<Lay::MN, Lay::MN>(oa, ob, d.s, ep, rest, st);
+    }
+    if (f == LinForm::F32) {
+        const float *x = (const float *)a, *y = (const float *)b;
+        if (op == LinOp::NT) return g32_nt(x, lda, y, ldb, out, N, M, N, K, nullptr, 0, 1.f, 0.f, rest, st);
+        if (op == LinOp::NN) return g32_nn(x, lda, y, ldb, out, K, M, N, K, 1.f, 0.f, rest, st);
+        return g32_tn(x, lda, y, ldb, out, K, M, N, K, 1.f, 0.f, rest, st);
+    }
+    const bf16 *x = (const bf16 *)a, *y = (const bf16 *)b;
+    if (op == LinOp::NT) return g16_nt(x, lda, y, ldb, out, N, M, N, K, nullptr, 0, 1.f, 0.f, rest, st);
+    if (op == LinOp::NN) return g16_nn(x, lda, y, ldb, out, K, M, N, K, 1.f, 0.f, rest, st);
+    return g16_tn(x, lda, y, ldb, out, K, M, N, K, 1.f, 0.f, rest, st);
+}
+
 size_t g32_ws_bytes_for(int M, int N, int K) {
     const GemmShape s{M, N, K};
     return ws_for(plan32(s, ~size_t(0)), s);

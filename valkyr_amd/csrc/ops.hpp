@@ -69,6 +69,26 @@ hipError_t g32_nn(const float *dy, long lddy, const float *w, long ldw, float *d
 hipError_t g32_tn(const float *dy, long lddy, const float *x, long ldx, float *dw, long lddw, int M,
                   int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st);
 size_t g32_ws_bytes_for(int M, int N, int K);
+// The three contractions of a linear layer on dense row-major operands of any
+// width and alignment: NT y = x W^T (a = x, b = W), NN dx = dy W, TN dW = dy^T x,
+// output overwritten.  F32: fp32 products; MIXED: fp32 operands rounded to bf16
+// on the way in; BF16: bf16 operands.  An operand the DMA-staged kernels cannot
+// take as it is (MIXED; rows that are not whole aligned 16-byte chunks) is first
+// copied into `ws` (lin_ws_bytes(...) bytes) with its rows padded by zeros.
+enum class LinOp { NT, NN, TN };
+enum class LinForm { F32, MIXED, BF16 };
+size_t lin_ws_bytes(LinOp op, LinForm f, const void *a, const void *b, int M, int N, int K);
+bool lin_packs(LinOp op, LinForm f, const void *a, const void *b, int M, int N, int K);
+// The packed copies themselves, one launch for two operands of `r` dense rows of
+// `c` elements each (r = 0: none); a packed row is lin_packed_ld elements.
+hipError_t lin_pack(LinForm f, const void *a, long ra, long ca, void *da, const void *b, long rb,
+                    long cb, void *db, hipStream_t st);
+inline long lin_packed_ld(LinForm f, long run) {
+    const long v = f == LinForm::F32 ? 4 : 8;
+    return (run + v - 1) / v * v;
+}
+hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out, int M, int N, int K,
+                   const GemmWs &ws, hipStream_t st);
 
 // ── LoRA rank-r products (k_lora.hip) ───────────────────────────────────
 // One adapter of a launch: its columns [col, col + ncols) of the shared X
