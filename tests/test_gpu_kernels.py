@@ -307,6 +307,39 @@ def test_linear_gemms_bf16_operands(shape):
         assert e < 1e-5, name
 
 
+@pytest.mark.parametrize("form", ["fp32", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 64, 64), (16, 1024, 3072), (33, 72, 4096), (96, 264, 8200),
+                                   (128, 6144, 1024), (250, 1032, 2048), (768, 1024, 1032)])
+def test_linear_products_of_few_tiles(form, shape):
+    """Products of few output tiles (32 / 64 / 128-row tiles, split over K or in two
+    wave groups) at tile edges, one row, and ragged K: against float64 on the same
+    operands, with the bound of test_linear_products_of_any_width_and_alignment; and
+    the same call twice gives the same bits."""
+    from valkyr_amd import kernels as K
+
+    M, N, Kd = shape
+    note(f"few tiles {form} M={M} N={N} K={Kd}")
+    rng = np.random.default_rng(M + N + Kd)
+    x, w, dy = (rng.standard_normal(s, dtype=np.float32) for s in ((M, Kd), (N, Kd), (M, N)))
+    if form == "bf16":
+        (bx, x), (bw, w), (bdy, dy) = (bf16_dev(t) for t in (x, w, dy))
+        x, w, dy = x.reshape(M, Kd), w.reshape(N, Kd), dy.reshape(M, N)
+    else:
+        bx, bw, bdy = dev(x), dev(w), dev(dy)
+    x, w, dy = (t.astype(np.float64) for t in (x, w, dy))
+    for n, ref, call in ((Kd, x @ w.T, "nt"), (N, dy @ w, "nn"), (M, dy.T @ x, "tn")):
+        a, b = {"nt": (bx, bw), "nn": (bdy, bw), "tn": (bdy, bx)}[call]
+        f = {"nt": (K.matmul_nt, K.matmul_nt_bf16), "nn": (K.linear_backward_dx, K.linear_backward_dx_bf16),
+             "tn": (K.linear_backward_dw, K.linear_backward_dw_bf16)}[call]
+        got = []
+        for _ in range(2):
+            out = zeros(ref.size)
+            f[form == "bf16"](a, b, out, M, N, Kd)
+            got.append(host(out))
+        assert rel_l2(ref, got[0]) < 1e-6 + 4 * math.sqrt(n) * 2.0 ** -24
+        assert np.array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("form", ["fp32", "mixed", "bf16"])
 @pytest.mark.parametrize("shape,skew", [((1, 9, 17), 0), ((65, 129, 63), 0), ((130, 257, 1001), 0),
                                         ((128, 64, 72), 1), ((2048, 264, 520), 1)])

@@ -642,7 +642,7 @@ vkh_status vkh_cce_backward(const vkh_cce_params *p, const float *h, const float
     note_allocation();
     VKH_HIP(hipMallocAsync(&dz, zb, st));
     hipError_t e = cce_backward(PR(p->precision), s, h, w, targets, lse, dz, dh, dw,
-                                accumulate_dw ? 1.f : 0.f, st);
+                                accumulate_dw ? 1.f : 0.f, GemmWs{nullptr, 0}, st);
     (void)hipFreeAsync(dz, st);
     if (e != hipSuccess) return hip_fail(e, "cce_backward");
     return VKH_OK;

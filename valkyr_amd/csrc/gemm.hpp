@@ -307,6 +307,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmOperand a, GemmOperand
 
 // C = alpha * acc (+ beta * C_old) (+ R), fp32 row-major.
 struct EpiStore {
+    static constexpr bool kSplits = true;  // runs fragment by fragment after a split-K sum
     float *C;
     long ldc;
     const float *R;  // optional residual, same shape as C
@@ -337,6 +338,7 @@ struct EpiStore {
 
 // C_bf16 = bf16(alpha * acc)
 struct EpiStoreBf16 {
+    static constexpr bool kSplits = true;
     bf16 *C;
     long ldc;
     float alpha;

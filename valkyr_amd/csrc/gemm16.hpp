@@ -499,7 +499,10 @@ __global__ __launch_bounds__(Cfg::NT, 1) void gemm16_swiglu_kernel(Op16 a, Op16 
         }
 }
 
-// One block per output tile: sum the split partials in order, then the epilogue.
+// One block per 16 x 16 accumulator fragment (i, j) of every wave of an output
+// tile: sum the split partials in order, then the epilogue on that fragment.
+// (Bound by reading the partials; a block per whole tile left a 16-token
+// product's 16 tiles x 32 splits to 16 CUs.)
 template <class Cfg, class Epi>
 __global__ __launch_bounds__(Cfg::NT) void gemm16_reduce_kernel(GemmShape s, Epi epi, SplitK sk,
                                                                 int tgrp) {
@@ -510,23 +513,15 @@ __global__ __launch_bounds__(Cfg::NT) void gemm16_reduce_kernel(GemmShape s, Epi
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int wm = wave / Cfg::WGN, wn = wave % Cfg::WGN;
     const int nbm = (s.M + BM - 1) / BM, nbn = (s.N + BN - 1) / BN;
-    const int tile = blockIdx.x;
+    const int tile = blockIdx.x / (TM * TN), frag = blockIdx.x % (TM * TN);
     int bm, bn;
     tile_rc(tile, nbm, nbn, tgrp, bm, bn);
-    const int m0 = bm * BM, n0 = bn * BN;
-    const f32x4 *parts = sk.ws + (size_t)tile * sk.splits * TILE4;
-    f32x4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int e = (i * TN + j) * NT + tid;
-            f32x4 sum = parts[e];
-            for (int q = 1; q < sk.splits; ++q) sum += parts[(size_t)q * TILE4 + e];
-            acc[i][j] = sum;
-        }
-    FragPos fp{m0 + wm * WM, n0 + wn * WN, lane};
-    epi.template apply<TM, TN>(acc, fp, s);
+    const f32x4 *parts = sk.ws + (size_t)tile * sk.splits * TILE4 + frag * NT + tid;
+    f32x4 acc[1][1] = {{parts[0]}};
+#pragma unroll 4
+    for (int q = 1; q < sk.splits; ++q) acc[0][0] += parts[(size_t)q * TILE4];
+    FragPos fp{bm * BM + wm * WM + 16 * (frag / TN), bn * BN + wn * WN + 16 * (frag % TN), lane};
+    epi.template apply<1, 1>(acc, fp, s);
 }
 
 template <class Cfg>
@@ -539,13 +534,16 @@ template <class Cfg, Lay LA, Lay LB, class Epi, bool F32 = false>
 hipError_t launch_gemm16(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &epi,
                          const SplitK &sk, int tgrp, hipStream_t st) {
     if (s.M <= 0 || s.N <= 0) return hipSuccess;
-    if (sk.splits < 1 || (sk.splits > 1 && !sk.ws)) return hipErrorInvalidValue;
+    if (sk.splits < 1 || (sk.splits > 1 && (!sk.ws || !Epi::kSplits))) return hipErrorInvalidValue;
     const unsigned tiles = ceil_div(s.M, Cfg::BM) * ceil_div(s.N, Cfg::BN);
     hipLaunchKernelGGL((gemm16_kernel<Cfg, LA, LB, Epi, F32>), dim3(tiles * sk.splits), dim3(Cfg::NT),
                        0, st, a, b, s, epi, sk, tgrp);
-    if (sk.splits > 1)
-        hipLaunchKernelGGL((gemm16_reduce_kernel<Cfg, Epi>), dim3(tiles), dim3(Cfg::NT), 0, st, s,
-                           epi, sk, tgrp);
+    if constexpr (Epi::kSplits) {
+        constexpr int frags = Cfg::BM / Cfg::WGM / 16 * (Cfg::BN / Cfg::WGN / 16);
+        if (sk.splits > 1)
+            hipLaunchKernelGGL((gemm16_reduce_kernel<Cfg, Epi>), dim3(tiles * frags), dim3(Cfg::NT), 0,
+                               st, s, epi, sk, tgrp);
+    }
     return hipGetLastError();
 }
 

@@ -44,6 +44,7 @@ inline CceWork carve(float *work, const CceShape &s) {
 }
 
 struct EpiCceStats {
+    static constexpr bool kSplits = false;
     CceWork w;
     const uint32_t *tgt;
     int V;
@@ -120,6 +121,7 @@ VKH_DEV float dz_elem(float z, const DzRow &r, float off, float tsc, bool is_t) 
 
 template <typename TZ>
 struct EpiCceDz {
+    static constexpr bool kSplits = false;
     TZ *dz;
     const uint32_t *tgt;
     const float *lse;
@@ -288,7 +290,7 @@ hipError_t cce_forward(Precision pr, const CceShape &s, const float *h, const fl
 
 hipError_t cce_backward(Precision pr, const CceShape &s, const float *h, const float *w,
                         const uint32_t *tgt, const float *lse, void *dz, float *dh, float *dw,
-                        float dw_beta, hipStream_t st, const float *z) {
+                        float dw_beta, const GemmWs &ws, hipStream_t st, const float *z) {
     if (s.N <= 0) return hipSuccess;
     const float inv_n = 1.0f / (float)s.N;
     const float t_scale = 1.0f - s.label_smoothing;
@@ -317,12 +319,11 @@ hipError_t cce_backward(Precision pr, const CceShape &s, const float *h, const f
     if (err != hipSuccess) return err;
     const Mat mz{dz, s.V, zdt};
     if (zdt == DType::F32) {  // fp32: the DMA-staged fp32 kernels (generic where they do not apply)
-        const GemmWs none{nullptr, 0};
         if (dw) {
-            err = g32_tn((const float *)dz, s.V, h, s.D, dw, s.D, s.N, s.V, s.D, 1.f, dw_beta, none, st);
+            err = g32_tn((const float *)dz, s.V, h, s.D, dw, s.D, s.N, s.V, s.D, 1.f, dw_beta, ws, st);
             if (err != hipSuccess) return err;
         }
-        if (dh) err = g32_nn((const float *)dz, s.V, w, s.D, dh, s.D, s.N, s.V, s.D, 1.f, 0.f, none, st);
+        if (dh) err = g32_nn((const float *)dz, s.V, w, s.D, dh, s.D, s.N, s.V, s.D, 1.f, 0.f, ws, st);
         return err;
     }
     if (dw) {

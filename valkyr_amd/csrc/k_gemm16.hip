@@ -9,10 +9,13 @@
 //   * K >= 16384 and >= 256 tiles of 128 x 128 -> 256 x 256 split-K 3 ways
 //   * K >= 4096 and >= 256 tiles of 128 x 128  -> 128 x 128, 8 waves
 //   * K >= 16384 and < 256 such tiles -> 256 x 256 split-K 8 ways (head dh)
+//   * <= 96 tiles of 128 x 64, or < 256 with K <= 1024 -> plan_few
 //   * < 384 tiles of 128 x 64, K >= 2048 -> 128 x 64 split-K 2 ways
 //   * otherwise                       -> 128 x 64
 // Operands that break the kernel's layout rules (16-byte alignment, ld and
 // the contiguous extent multiples of 8, < 2 GiB) take the generic MFMA GEMM.
+#include <math.h>
+
 #include <algorithm>
 
 #include "gemm16.hpp"
@@ -34,6 +37,9 @@ using T128w8 = Tile16<128, 128, 2, 4>;  // 8 waves of 64 x 32
 // us; the bf16 step 19.33-19.34 -> 19.31-19.32 ms.  (In fp32 mode, whose slabs
 // are half as deep, it made the fp32 step slower: 77.3 against 76.65 ms.)
 using T128x64s3 = Tile16<128, 64, 2, 2, 3>;
+// Few-tile products (plan_few): smaller tiles, split over K.
+using T64 = Tile16<64, 64, 2, 2>;
+using T32x64 = Tile16<32, 64, 1, 4>;  // K-major A only (a bf16 MN tile is 64 rows or 128 n)
 // (Three slab buffers were measured slower for these tiles: the larger LDS
 // footprint drops a block per CU.  Staging the slabs through VGPRs two slabs
 // ahead, which doubles the time a load has to arrive without more LDS, was
@@ -42,7 +48,7 @@ using T128x64s3 = Tile16<128, 64, 2, 2, 3>;
 
 constexpr bool kUseKs2 = true;
 
-enum class Pick { Big, T128, T128x64, T128w8, T128x64ks2 };
+enum class Pick { Big, T128, T128x64, T128w8, T128x64ks2, T64, T32x64, T64ks2, T32x64ks2 };
 struct Plan {
     Pick tile;
     int splits;
@@ -55,15 +61,76 @@ size_t ws_for(const Plan &p, const GemmShape &s) {
     case Pick::Big: return gemm16_ws_bytes<TBig>(s, p.splits);
     case Pick::T128: return gemm16_ws_bytes<T128>(s, p.splits);
     case Pick::T128w8: return gemm16_ws_bytes<T128w8>(s, p.splits);
+    case Pick::T64: return gemm16_ws_bytes<T64>(s, p.splits);
+    case Pick::T32x64: return gemm16_ws_bytes<T32x64>(s, p.splits);
     default: return gemm16_ws_bytes<T128x64>(s, p.splits);
     }
 }
 
-Plan plan(const GemmShape &s, size_t ws_bytes) {
+// Products of few tiles (short sequences, small models): most CUs would idle on
+// 128-row tiles, and a block's K loop is a serial chain of slabs (0.29 us each in
+// bf16, 0.36 in fp32, where the matrix cores are the slower part).  The tile and
+// the split over K come from a model of the launch: its fixed cost, the slower of
+// the slab chain, the CU's matrix time when blocks share it, operand traffic and
+// output traffic, and the reduce launch of a split.  Fitted (least squares on the
+// logarithm, 11-15 % rms) to 2800 timings of 16-512 rows over widths 256-32000 in
+// the three layouts; the pick is 4-6 % above the best of the table on average, and
+// against the 128 x 64 tiles before it: fp32 16 x 1024 x 3072 107 -> 9.7 us,
+// 128 x 512 x 512 22 -> 7.3, 512 x 1024 x 1024 39 -> 16; bf16 16 x 1024 x 3072
+// 18.8 -> 7.3 us, 128 x 1024 x 1024 10.6 -> 6.5, 512 x 768 x 32000 95 -> 55.
+// fp32 also has the in-block split (two wave groups on the halves of K, no reduce
+// launch), and with two_halves nothing else (a 2-layer 256-wide step of 128 tokens
+// 980 -> 620 us with the same bits).
+Plan plan_few(const GemmShape &s, size_t ws_bytes, bool f32, bool mn_a, bool two_halves = false) {
+    struct Fit { double launch, slab0, slab1, mfma, l2, red, part, hbm; };
+    constexpr Fit kB{3.8, 0.088, 0.199, 0.225, 21.2, 2.5, 6.6, 5.2},
+        kF{4.5, 0.314, 0.047, 0.574, 10.7, 2.0, 6.5, 4.4};
+    const Fit &f = f32 ? kF : kB;
+    const double es = f32 ? 4 : 2;
+    const double hbm = (es * s.K * ((double)s.M + s.N) + 4.0 * s.M * s.N) / (f.hbm * 1e6);
+    const int nk = (s.K + (f32 ? 31 : 63)) / (f32 ? 32 : 64);
+    const int min_slabs = f32 ? 1 : 8;  // of a split: 512 of K in bf16, as in plan()
+    Plan best{Pick::T128x64, 1};
+    double tb = 1e30;
+    auto tile = [&](Pick pick, Pick ks2, int bm, int bn) {
+        const double tiles = (double)ceil_div(s.M, bm) * ceil_div(s.N, bn);
+        if (f32) {  // both groups of a block share its CU's matrix cores
+            const double slabs = (nk + 1) / 2, share = ceil(tiles / 256) * 2 * f.mfma * bm * bn / 4096;
+            const double t = std::max(slabs * std::max(f.slab0 + f.slab1 * (bm + bn) / 128, share),
+                                      tiles * nk * (bm + bn) * 128 / (f.l2 * 1e6));
+            if (f.launch + 0.7 + std::max(t, hbm) < tb) {
+                tb = f.launch + 0.7 + std::max(t, hbm);
+                best = Plan{ks2, 1};
+            }
+            if (two_halves) return;
+        }
+        for (int sp = 1; sp <= 32; sp *= 2) {
+            const Plan p{pick, sp};
+            if (sp > 1 && (nk / sp < min_slabs || ws_for(p, s) > ws_bytes)) break;
+            const double slabs = (nk + sp - 1) / sp, blocks = tiles * sp;
+            const double share = ceil(blocks / 256) * f.mfma * bm * bn / 4096;
+            double t = std::max(slabs * std::max(f.slab0 + f.slab1 * (bm + bn) / 128, share),
+                                blocks * slabs * (bm + bn) * 128 / (f.l2 * 1e6));
+            t = f.launch + std::max(t, hbm);
+            if (sp > 1) t += f.red + blocks * bm * bn * 8 / (f.part * 1e6);
+            if (t < tb) tb = t, best = p;
+        }
+    };
+    tile(Pick::T128x64, Pick::T128x64ks2, 128, 64);
+    tile(Pick::T64, Pick::T64ks2, 64, 64);
+    if (f32 || !mn_a) tile(Pick::T32x64, Pick::T32x64ks2, 32, 64);
+    return best;
+}
+
+// mn_a: the A operand is MN-major (the weight gradients).
+Plan plan(const GemmShape &s, size_t ws_bytes, bool mn_a = false) {
     auto tiles = [&](int bm, int bn) { return (long)ceil_div(s.M, bm) * (long)ceil_div(s.N, bn); };
     if (tiles(256, 256) >= 512) return {Pick::Big, 1};
     const long t128 = tiles(128, 128), t64 = tiles(128, 64);
     if (t128 >= 512) return {Pick::T128w8, 1};
+    // few tiles: up to 96 of 128 x 64, and up to 255 where K is short (beyond, the
+    // two-group 128 x 64 blocks are as fast: 256 x 4096 x 4096 26.5 against 32.5 us)
+    if (t64 <= 96 || (t64 < 256 && s.K <= 1024)) return plan_few(s, ws_bytes, false, mn_a);
     const int nk = (s.K + 63) / 64;
     Plan p{Pick::T128x64, 1};
     if (s.K >= 16384 && t128 >= 256)
@@ -107,7 +174,7 @@ bool fused_tile_ok(const GemmShape &s, bool paired) {
 template <Lay LA, Lay LB, class Epi>
 hipError_t run16(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e, const GemmWs &ws,
                  hipStream_t st) {
-    const Plan p = plan(s, ws.p ? ws.bytes : 0);
+    const Plan p = plan(GemmShape{ws.plan_rows ? ws.plan_rows : s.M, s.N, s.K}, ws.p ? ws.bytes : 0, LA == Lay::MN);
     const SplitK sk{p.splits, (f32x4 *)ws.p};
     const int g = p.column_order ? 0 : tile_group_rows<LA, LB>();
     switch (p.tile) {
@@ -115,6 +182,10 @@ hipError_t run16(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e,
     case Pick::T128: return launch_gemm16<T128, LA, LB>(a, b, s, e, sk, g, st);
     case Pick::T128w8: return launch_gemm16<T128w8, LA, LB>(a, b, s, e, sk, g, st);
     case Pick::T128x64ks2: return launch_gemm16_ks2<T128x64s3, LA, LB>(a, b, s, e, g, st);
+    case Pick::T64: return launch_gemm16<T64, LA, LB>(a, b, s, e, sk, g, st);
+    case Pick::T32x64:
+        if constexpr (LA == Lay::K) return launch_gemm16<T32x64, LA, LB>(a, b, s, e, sk, g, st);
+        else return hipErrorInvalidValue;
     default: return launch_gemm16<T128x64, LA, LB>(a, b, s, e, sk, g, st);
     }
 }
@@ -137,22 +208,24 @@ hipError_t run16(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e,
 //     but in the two-stream step the in-block form is (76.3-77.0 against
 //     76.5-77.1 ms in four alternating pairs; plain 128 x 64: 77.3-77.4): the
 //     reduce launches' 4.2 ms of partial traffic per step is gone.
-Plan plan32(const GemmShape &s, size_t ws_bytes) {
+// Fewer than 256 tiles of 128 x 64, or fewer than 512 with a K of at most 1024:
+// plan_few (there the in-block split leaves CUs idle or its second group without
+// work: 2560-wide products of 512 rows 95 -> 64 us, 3072 x 1024 dW of 16 rows 15 -> 8).
+Plan plan32(const GemmShape &s, size_t ws_bytes, bool mn_a = false, bool two_halves = false) {
     auto tiles = [&](int bm, int bn) { return (long)ceil_div(s.M, bm) * (long)ceil_div(s.N, bn); };
     auto fill = [](long t) { return (double)t / (256.0 * (double)((t + 255) / 256)); };
     const long t128 = tiles(128, 128), t64 = tiles(128, 64);
-    const int nk = (s.K + 31) / 32;
     Plan p{Pick::T128x64, 1};
     if (t128 >= 256 && fill(t128) >= fill(t64)) p = Plan{Pick::T128w8, 1};
+    else if (t64 < 256 || (t64 < 512 && s.K <= 1024)) p = plan_few(s, ws_bytes, true, mn_a, two_halves);
     else if (t64 < 512) p = Plan{Pick::T128x64ks2, 1};
-    while (p.splits > 1 && (nk / p.splits < 8 || ws_for(p, s) > ws_bytes)) --p.splits;
     return p;
 }
 
 template <Lay LA, Lay LB, class Epi>
 hipError_t run32(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e, const GemmWs &ws,
                  hipStream_t st) {
-    const Plan p = plan32(s, ws.p ? ws.bytes : 0);
+    const Plan p = plan32(s, ws.p ? ws.bytes : 0, LA == Lay::MN, ws.two_halves);
     const SplitK sk{p.splits, (f32x4 *)ws.p};
     const int g = p.column_order ? 0 : tile_group_rows<LA, LB>();
     switch (p.tile) {
@@ -160,6 +233,10 @@ hipError_t run32(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e,
     case Pick::T128: return launch_gemm16<T128, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
     case Pick::T128w8: return launch_gemm16<T128w8, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
     case Pick::T128x64ks2: return launch_gemm16_ks2<T128x64, LA, LB, Epi, true>(a, b, s, e, g, st);
+    case Pick::T64: return launch_gemm16<T64, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
+    case Pick::T32x64: return launch_gemm16<T32x64, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
+    case Pick::T64ks2: return launch_gemm16_ks2<T64, LA, LB, Epi, true>(a, b, s, e, g, st);
+    case Pick::T32x64ks2: return launch_gemm16_ks2<T32x64, LA, LB, Epi, true>(a, b, s, e, g, st);
     default: return launch_gemm16<T128x64, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
     }
 }
@@ -211,6 +288,7 @@ int rows_per_2g_chunk(long rows, long ld, long run) {
 // reads them.  Base's own alpha must be 1 (the linear layers' products).
 template <class Base>
 struct EpiLora {
+    static constexpr bool kSplits = Base::kSplits;
     Base base;
     LoraSegs sg;
     int r;
@@ -734,12 +812,12 @@ hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out
 
 size_t g32_ws_bytes_for(int M, int N, int K) {
     const GemmShape s{M, N, K};
-    return ws_for(plan32(s, ~size_t(0)), s);
+    return std::max(ws_for(plan32(s, ~size_t(0)), s), ws_for(plan32(s, ~size_t(0), true), s));
 }
 
 size_t g16_ws_bytes_for(int M, int N, int K) {
     const GemmShape s{M, N, K};
-    return ws_for(plan(s, ~size_t(0)), s);
+    return std::max(ws_for(plan(s, ~size_t(0)), s), ws_for(plan(s, ~size_t(0), true), s));
 }
 
 }  // namespace vkh

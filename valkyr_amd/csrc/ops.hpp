@@ -37,6 +37,14 @@ hipError_t gemm_tn(Precision pr, Mat dy, Mat x, float *dw, long lddw, int M, int
 struct GemmWs {
     void *p;
     size_t bytes;
+    // rows to plan for instead of M (0: M): a product run as parts of one with more
+    // rows (the forward's half batches) takes the whole product's split over K, so
+    // its sums have the same bits either way
+    int plan_rows = 0;
+    // fp32 products keep the summation order of two halves of K whatever their tile:
+    // the training step's gradients, and with them its Adam trajectory, stay the same
+    // bits on every tile plan
+    bool two_halves = false;
 };
 hipError_t g16_nt(const bf16 *x, long ldx, const bf16 *w, long ldw, float *y, long ldy, int M,
                   int N, int K, const float *R, long ldr, float alpha, float beta,
@@ -416,6 +424,6 @@ hipError_t cce_backward16(const CceShape &s, const bf16 *h, const bf16 *w, const
 // recomputing them; nullptr recomputes.
 hipError_t cce_backward(Precision pr, const CceShape &s, const float *h, const float *w,
                         const uint32_t *tgt, const float *lse, void *dz, float *dh, float *dw,
-                        float dw_beta, hipStream_t st, const float *z = nullptr);
+                        float dw_beta, const GemmWs &ws, hipStream_t st, const float *z = nullptr);
 
 }  // namespace vkh

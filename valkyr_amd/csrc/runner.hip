@@ -511,32 +511,28 @@ struct vkh_runner {
                 VKH_TRY(alloc(attn_split, fa_bw_v4_split_ws_floats(attn_shape())));
             if (attn_fused && fa_bw_ws_bytes(attn_shape(), attn_v4))
                 VKH_TRY(alloc(attn_ds, fa_bw_ws_bytes(attn_shape(), attn_v4) / sizeof(bf16)));
-            // split-K workspace: the largest the planner asks for over the step's GEMMs
-            size_t wsb = 0;
-            auto need = [&](int m, int n, int k) { wsb = std::max(wsb, g16_ws_bytes_for(m, n, k)); };
-            need(T, qkvd, D); need(T, D, qd); need(T, 2 * F, D); need(T, D, F);
-            need(T, F, D); need(T, D, 2 * F); need(T, qd, D); need(T, D, qkvd);
-            need(D, F, T); need(2 * F, D, T); need(D, qd, T); need(qkvd, D, T);
-            need(T, D, V); need(V, D, T);
-            if (wsb) {
-                char *w = nullptr;
-                VKH_TRY(alloc(w, wsb));
-                gws = GemmWs{w, wsb};
-            }
         } else {
             VKH_TRY(alloc(fn_out, (size_t)T * D));
-            // split-K workspace of the fp32 GEMMs (g32_*), if their plan asks for one
-            size_t wsb = 0;
-            auto need = [&](int m, int n, int k) { wsb = std::max(wsb, g32_ws_bytes_for(m, n, k)); };
-            need(T, qkvd, D); need(T, D, qd); need(T, 2 * F, D); need(T, D, F);
-            need(T, F, D); need(T, D, 2 * F); need(T, qd, D); need(T, D, qkvd);
-            need(D, F, T); need(2 * F, D, T); need(D, qd, T); need(qkvd, D, T);
-            if (wsb) {
-                char *w = nullptr;
-                VKH_TRY(alloc(w, wsb));
-                gws = GemmWs{w, wsb};
-            }
         }
+        // split-K workspace, one per stream: the largest the planner asks for over the
+        // bf16 step's GEMMs (the forward also runs them as two half batches); the fp32
+        // step keeps its sums in two halves of K, in one block each, and needs none
+        size_t wsb = 0;
+        auto need = [&](int m, int n, int k) {
+            if (b16()) wsb = std::max(wsb, g16_ws_bytes_for(m, n, k));
+        };
+        for (const int t : {T, T / 2}) {
+            need(t, qkvd, D); need(t, D, qd); need(t, 2 * F, D); need(t, D, F); need(t, V, D);
+        }
+        need(T, F, D); need(T, D, 2 * F); need(T, qd, D); need(T, D, qkvd);
+        need(D, F, T); need(2 * F, D, T); need(D, qd, T); need(qkvd, D, T);
+        need(T, D, V); need(V, D, T);
+        if (wsb) {
+            char *w = nullptr;
+            VKH_TRY(alloc(w, wsb));
+            gws = GemmWs{w, wsb};
+        }
+        gws.two_halves = gws2.two_halves = !b16();
         if (concurrent) {
             // the side stream (weight gradients, Adam) and each layer's gradient
             // operands for it, in the step's precision
@@ -593,16 +589,11 @@ struct vkh_runner {
                 VKH_TRY(alloc(lg[l].pn2, rmsnorm_partial_floats(T, D)));
                 if (cfg.qk_norm) VKH_TRY(alloc(lg[l].pqk, qk_partial_floats()));
             }
-            // the side stream's own split-K workspace
-            size_t wsb2 = 0;
-            auto need2 = [&](int m, int n, int k) {
-                wsb2 = std::max(wsb2, b16() ? g16_ws_bytes_for(m, n, k) : g32_ws_bytes_for(m, n, k));
-            };
-            need2(D, F, T); need2(2 * F, D, T); need2(D, qd, T); need2(qkvd, D, T); need2(V, D, T);
-            if (wsb2) {
+            if (wsb) {  // the side stream's own
                 char *w = nullptr;
-                VKH_TRY(alloc(w, wsb2));
-                gws2 = GemmWs{w, wsb2};
+                VKH_TRY(alloc(w, wsb));
+                gws2 = GemmWs{w, wsb};
+                gws2.two_halves = !b16();
             }
         }
         VKH_TRY(alloc(ce_lse, T));
@@ -1118,6 +1109,7 @@ struct vkh_runner {
             for (int h = 0; h < 2 && st == VKH_OK; ++h) {
                 cur = h ? side : c0;
                 gws = h ? gws2 : w0;
+                gws.plan_rows = T0;
                 x_emb = x0 + h * th * D;
                 std::swap(acts, acts_h[h]);
                 st = layer_forward(l);
@@ -1416,7 +1408,7 @@ struct vkh_runner {
             // measured 0.05-0.09 ms slower this way and keeps dh first)
             const bool dw_early = concurrent && dw_lm;
             VKH_HIP(cce_backward(pr, cs, fn_out, W(lm_head), tgt_d, ce_lse, dz, dw_early ? nullptr : d_fn,
-                                 concurrent ? nullptr : dw_lm, 0.f, cur, (const float *)dz));
+                                 concurrent ? nullptr : dw_lm, 0.f, gws, cur, (const float *)dz));
             if (concurrent && dw_lm) {  // as above, on the fp32 logits gradient
                 if (split) {
                     if (++mark_stamp == 0) {
@@ -1430,8 +1422,7 @@ struct vkh_runner {
                 VKH_HIP(g32_tn((const float *)dz, V, fn_out, D, dw_lm, D, T, V, D, 1.f, 0.f, gws2, side));
                 // dh = dz W_lm (cce_backward's own call); the table's Adam on the
                 // side stream rewrites W_lm, so it waits for dh
-                VKH_HIP(g32_nn((const float *)dz, V, W(lm_head), D, d_fn, D, T, V, D, 1.f, 0.f,
-                               GemmWs{nullptr, 0}, cur));
+                VKH_HIP(g32_nn((const float *)dz, V, W(lm_head), D, d_fn, D, T, V, D, 1.f, 0.f, gws, cur));
                 VKH_HIP(hipEventRecord(ev_dh, cur));
                 VKH_HIP(hipStreamWaitEvent(side, ev_dh, 0));
                 if (split) VKH_TRY(embed_adam_early());
