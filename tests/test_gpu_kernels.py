@@ -662,6 +662,36 @@ def test_cce_forward_backward(prec, n, V, D, zl, ls):
     assert rel_l2(dW_ref, host(bdW)) < tol
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n,V,D,skew", [(1, 65, 64, 0), (33, 1003, 61, 0), (129, 8191, 72, 0),
+                                        (64, 257, 66, 1), (300, 20001, 136, 0)])
+def test_cce_odd_vocabulary_width_and_alignment(prec, n, V, D, skew):
+    """The head on operands that are packed into padded rows (odd widths, addresses
+    off by one float, fp32 operands in bf16 products) and an odd vocabulary (padded
+    dz rows), accumulating into dW: against the oracle on the rounded operands."""
+    from valkyr_amd import kernels as K
+
+    note(f"cce odd prec={prec} n={n} V={V} D={D} skew={skew}")
+    h, w = O.normal(n * D, 91), O.normal(V * D, 92, 0.05)
+    if prec == 1:
+        h, w = O.round_bf16(h), O.round_bf16(w)
+    t, dw0 = O.ids(n, 93, V), O.normal(V * D, 94, 1e-3)
+    _, lse_ref, row_ref = O.cce_forward(h, w, t, n, V, D, 1024, 1e-4, 0.1)
+    dh_ref, dW_ref = O.cce_backward(h, w, t, lse_ref, n, V, D, 1024, 1e-4, 0.1)
+    p = K.cce_params(n, V, D, 1e-4, 0.1, prec)
+    pad = np.zeros(skew, np.float32)
+    bh, bw = dev(np.concatenate([pad, h])), dev(np.concatenate([pad, w]))
+    ph, pw, bt = bh.offset(4 * skew), bw.offset(4 * skew), dev(t)
+    blse, brow, bdh, bdW = zeros(n), zeros(n), zeros(n * D), dev(dw0)
+    K.cce_forward(p, ph, pw, bt, blse, brow)
+    K.cce_backward(p, ph, pw, bt, blse, bdh, bdW, accumulate_dw=True)
+    assert grel(lse_ref, host(blse)) < 1e-5
+    assert grel(row_ref, host(brow)) < 1e-4
+    tol = FP32_TOL if prec == 0 else BF16_TOL
+    assert rel_l2(dh_ref, host(bdh)) < tol
+    assert rel_l2(dW_ref, host(bdW) - dw0) < tol
+
+
 # ── FlashAttention ───────────────────────────────────────────────────────
 
 FA_F32_CASES = [  # smoke/cpu.zig:909-916 shapes (n_q, n_kv, H, Hkv, hd, causal) + batch

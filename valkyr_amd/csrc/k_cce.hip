@@ -21,6 +21,8 @@
 // them in place with one streaming pass (cce_dz_k, the dz epilogue's
 // arithmetic element by element) instead of recomputing the logits GEMM: the
 // same values bit for bit, 2.5 GB of traffic in place of a 0.64 TFLOP product.
+#include <math.h>
+
 #include "gemm16.hpp"
 #include "ops.hpp"
 
@@ -48,7 +50,8 @@ struct EpiCceStats {
     CceWork w;
     const uint32_t *tgt;
     int V;
-    float *zo = nullptr;  // when set: the logits themselves, [N, V] row-major
+    float *zo = nullptr;  // when set: the logits themselves, rows of ldz
+    long ldz = 0;
 
     template <int TM, int TN>
     VKH_DEV void apply(const f32x4 (&acc)[TM][TN], const FragPos &fp, const GemmShape &s) const {
@@ -83,7 +86,7 @@ struct EpiCceStats {
                         mx = fmaxf(mx, z);
                         zs += z;
                         if (tc == 16 * j) w.zt[row] = z;
-                        if (zo && rok) zo[(size_t)row * V + fp.col0 + 16 * j + c16] = z;
+                        if (zo && rok) zo[(size_t)row * ldz + fp.col0 + 16 * j + c16] = z;
                     }
                 }
                 mx = row16_max(mx);
@@ -126,6 +129,7 @@ struct EpiCceDz {
     const uint32_t *tgt;
     const float *lse;
     int V;
+    long ldz;  // zeros go to columns [V, ldz)
     float inv_n, t_scale, eps_over_v, zl2;
 
     template <int TM, int TN>
@@ -148,41 +152,50 @@ struct EpiCceDz {
                 if (row >= s.M) continue;
                 const DzRow dr = dz_row(lse[row], zl2, inv_n);
                 const int tc = (int)tgt[row] - fp.col0 - c16;
-                TZ *out = dz + (size_t)row * V + fp.col0 + c16;
+                TZ *out = dz + (size_t)row * ldz + fp.col0 + c16;
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    if (!FULL && fp.col0 + 16 * j + c16 >= V) continue;
+                    if (!FULL && fp.col0 + 16 * j + c16 >= V) {
+                        if (fp.col0 + 16 * j + c16 < ldz) out[16 * j] = (TZ)0.f;
+                        continue;
+                    }
                     out[16 * j] = (TZ)dz_elem(acc[i][j][r], dr, off, tsc, tc == 16 * j);
                 }
             }
     }
 };
 
-// dz from the stored fp32 logits z [N, V] (z and dz may be the same buffer: each
+// dz from the stored fp32 logits z, rows of ldz (z and dz may be the same buffer: each
 // element is read and then written by one thread).  Block (x, row): 4 columns
-// per thread with 16-byte rows (V % 4 == 0 and 16-byte aligned), else 1.
+// per thread with 16-byte rows (ldz % 4 == 0 and 16-byte aligned), else 1.
 template <typename TZ, int VEC>
 __global__ __launch_bounds__(256) void cce_dz_k(const float *z, TZ *dz, const uint32_t *tgt,
-                                                const float *lse, int V, float inv_n, float t_scale,
-                                                float eps_over_v, float zl2) {
+                                                const float *lse, int V, long ldz, float inv_n,
+                                                float t_scale, float eps_over_v, float zl2) {
     const int row = blockIdx.y;
     const int c0 = (blockIdx.x * 256 + threadIdx.x) * VEC;
-    if (c0 >= V) return;
+    if (c0 >= ldz) return;
     const DzRow dr = dz_row(lse[row], zl2, inv_n);
     const float off = eps_over_v * inv_n, tsc = t_scale * inv_n;
     const int t = (int)tgt[row];
-    const size_t i = (size_t)row * V + c0;
+    const size_t i = (size_t)row * ldz + c0;
     if constexpr (VEC == 4) {
         const float4 zv = *reinterpret_cast<const float4 *>(z + i);
-        const float d0 = dz_elem(zv.x, dr, off, tsc, t == c0), d1 = dz_elem(zv.y, dr, off, tsc, t == c0 + 1),
-                    d2 = dz_elem(zv.z, dr, off, tsc, t == c0 + 2), d3 = dz_elem(zv.w, dr, off, tsc, t == c0 + 3);
+        float d0 = dz_elem(zv.x, dr, off, tsc, t == c0), d1 = dz_elem(zv.y, dr, off, tsc, t == c0 + 1),
+              d2 = dz_elem(zv.z, dr, off, tsc, t == c0 + 2), d3 = dz_elem(zv.w, dr, off, tsc, t == c0 + 3);
+        if (c0 + 4 > V) {  // the zeros of a padded row (its stored logits end at V)
+            if (c0 >= V) d0 = 0.f;
+            if (c0 + 1 >= V) d1 = 0.f;
+            if (c0 + 2 >= V) d2 = 0.f;
+            d3 = 0.f;
+        }
         if constexpr (sizeof(TZ) == 4) {
             *reinterpret_cast<float4 *>(dz + i) = make_float4(d0, d1, d2, d3);
         } else {
             dz[i] = (TZ)d0; dz[i + 1] = (TZ)d1; dz[i + 2] = (TZ)d2; dz[i + 3] = (TZ)d3;
         }
     } else {
-        dz[i] = (TZ)dz_elem(z[i], dr, off, tsc, t == c0);
+        dz[i] = c0 < V ? (TZ)dz_elem(z[i], dr, off, tsc, t == c0) : (TZ)0.f;
     }
 }
 
@@ -225,47 +238,85 @@ __global__ void cce_mean_k(CceShape s, CceWork w, float *loss_mean) {
     if (threadIdx.x == 0) loss_mean[0] = (float)((sh[0] + sh[1] + sh[2] + sh[3]) / (double)s.N);
 }
 
+// The logits GEMM's tile (wave slices of 64 columns in each, as the epilogues need):
+// the one with the least rounds x tile area over its rate relative to 256 x 256.
+// fp32 is bound by the matrix cores, so the small tiles lose little and fill the
+// chip better (127 x 32003 x 768 took 197 us on 126 blocks of 256 x 256; 502 of
+// 64 x 128 share its matrix work over all CUs); bf16 needs the large ones wherever they fill it.
+template <bool F32, class Epi>
+hipError_t logits_tiles(const Op16 &a, const Op16 &b, const GemmShape &sh, const Epi &epi, hipStream_t st) {
+    const SplitK one{1, nullptr};
+    constexpr int g = tile_group_rows<Lay::K, Lay::K>();
+    auto cost = [&](int bm, int bn, double rate) {
+        const double tiles = (double)ceil_div(sh.M, bm) * ceil_div(sh.N, bn);
+        return ceil(tiles / 256) * bm * bn / rate;
+    };
+    const double c0 = cost(256, 256, 1.0), c1 = cost(128, 256, F32 ? 0.98 : 0.8),
+                 c2 = cost(128, 128, F32 ? 0.96 : 0.65), c3 = cost(64, 128, F32 ? 0.9 : 0.45);
+    if (c0 <= c1 && c0 <= c2 && c0 <= c3)
+        return launch_gemm16<Tile16<256, 256, 2, 4>, Lay::K, Lay::K, Epi, F32>(a, b, sh, epi, one, g, st);
+    if (c1 <= c2 && c1 <= c3)
+        return launch_gemm16<Tile16<128, 256, 2, 4>, Lay::K, Lay::K, Epi, F32>(a, b, sh, epi, one, g, st);
+    if (c2 <= c3)
+        return launch_gemm16<Tile16<128, 128, 2, 2>, Lay::K, Lay::K, Epi, F32>(a, b, sh, epi, one, g, st);
+    return launch_gemm16<Tile16<64, 128, 2, 2>, Lay::K, Lay::K, Epi, F32>(a, b, sh, epi, one, g, st);
+}
+
+// fp32 operands; the generic MFMA GEMM where they do not fit the DMA-staged rules.
 template <class Epi>
-hipError_t logits_gemm(Precision pr, const CceShape &s, const float *h, const float *w,
-                       const Epi &epi, hipStream_t st) {
-    GemmOperand a{h, s.D, vec_ok(h, s.D, 4, Lay::K)};
-    GemmOperand b{w, s.D, vec_ok(w, s.D, 4, Lay::K)};
+hipError_t logits32(const CceShape &s, const float *h, const float *w, const Epi &epi, hipStream_t st) {
+    const long ld = s.hs();
     GemmShape sh{s.N, s.V, s.D};
-    if (pr == Precision::BF16)
-        return launch_gemm<TileCfg<128, 128, 64>, true, float, Lay::K, float, Lay::K>(a, b, sh, epi, st);
-    // fp32: the DMA-staged 256 x 256 tile on the fp32 matrix cores (64-column
-    // wave slices, as the epilogues need) where the operands fit its rules
-    const size_t hb = ((size_t)(s.N - 1) * s.D + s.D) * 4, wb = ((size_t)(s.V - 1) * s.D + s.D) * 4;
-    if (s.D % 4 == 0 && ((uintptr_t)h & 15u) == 0 && ((uintptr_t)w & 15u) == 0 &&
-        hb < (1ull << 31) && wb < (1ull << 31)) {
-        const Op16 a16{(const bf16 *)h, s.D, (unsigned)hb}, b16{(const bf16 *)w, s.D, (unsigned)wb};
-        const SplitK one{1, nullptr};
-        return launch_gemm16<Tile16<256, 256, 2, 4>, Lay::K, Lay::K, Epi, true>(
-            a16, b16, sh, epi, one, tile_group_rows<Lay::K, Lay::K>(), st);
-    }
+    const size_t hb = (size_t)s.N * ld * 4, wb = (size_t)s.V * ld * 4;
+    if (ld % 4 == 0 && ((uintptr_t)h & 15u) == 0 && ((uintptr_t)w & 15u) == 0 && hb < (1ull << 31) &&
+        wb < (1ull << 31))
+        return logits_tiles<true>(Op16{(const bf16 *)h, ld, (unsigned)hb},
+                                  Op16{(const bf16 *)w, ld, (unsigned)wb}, sh, epi, st);
+    GemmOperand a{h, ld, vec_ok(h, ld, 4, Lay::K)};
+    GemmOperand b{w, ld, vec_ok(w, ld, 4, Lay::K)};
     return launch_gemm<TileCfg<128, 128, 32>, false, float, Lay::K, float, Lay::K>(a, b, sh, epi, st);
 }
 
-// bf16 operands: the gemm16 kernel with 64-column wave slices (8 waves in a
-// 2 x 4 grid), falling back to the generic MFMA GEMM for unaligned shapes.
+// bf16 operands, the same way.
 template <class Epi>
 hipError_t logits16(const CceShape &s, const bf16 *h, const bf16 *w, const Epi &epi,
                     hipStream_t st) {
+    const long ld = s.hs();
     GemmShape sh{s.N, s.V, s.D};
-    const size_t hb = ((size_t)(s.N - 1) * s.D + s.D) * 2, wb = ((size_t)(s.V - 1) * s.D + s.D) * 2;
-    const bool ok = s.D % 8 == 0 && ((uintptr_t)h & 15u) == 0 && ((uintptr_t)w & 15u) == 0 &&
-                    hb < (1ull << 31) && wb < (1ull << 31);
-    if (!ok) {
-        GemmOperand a{h, s.D, vec_ok(h, s.D, 2, Lay::K)};
-        GemmOperand b{w, s.D, vec_ok(w, s.D, 2, Lay::K)};
-        return launch_gemm<TileCfg<128, 128, 64>, true, bf16, Lay::K, bf16, Lay::K>(a, b, sh, epi, st);
-    }
-    const Op16 a{h, s.D, (unsigned)hb}, b{w, s.D, (unsigned)wb};
-    const SplitK one{1, nullptr};
-    constexpr int g = tile_group_rows<Lay::K, Lay::K>();
-    if ((long)ceil_div(s.N, 256) * ceil_div(s.V, 256) >= 256)
-        return launch_gemm16<Tile16<256, 256, 2, 4>, Lay::K, Lay::K>(a, b, sh, epi, one, g, st);
-    return launch_gemm16<Tile16<128, 256, 2, 4>, Lay::K, Lay::K>(a, b, sh, epi, one, g, st);
+    const size_t hb = (size_t)s.N * ld * 2, wb = (size_t)s.V * ld * 2;
+    if (ld % 8 == 0 && ((uintptr_t)h & 15u) == 0 && ((uintptr_t)w & 15u) == 0 && hb < (1ull << 31) &&
+        wb < (1ull << 31))
+        return logits_tiles<false>(Op16{h, ld, (unsigned)hb}, Op16{w, ld, (unsigned)wb}, sh, epi, st);
+    GemmOperand a{h, ld, vec_ok(h, ld, 2, Lay::K)};
+    GemmOperand b{w, ld, vec_ok(w, ld, 2, Lay::K)};
+    return launch_gemm<TileCfg<128, 128, 64>, true, bf16, Lay::K, bf16, Lay::K>(a, b, sh, epi, st);
+}
+
+template <typename TZ>
+hipError_t dz_from_logits(const CceShape &s, const float *z, const EpiCceDz<TZ> &e, hipStream_t st) {
+    const long ld = s.zs();
+    const bool v4 = ld % 4 == 0 && ((uintptr_t)z & 15u) == 0 && ((uintptr_t)e.dz & 15u) == 0;
+    const dim3 grid((unsigned)ceil_div(ld, 256 * (v4 ? 4 : 1)), (unsigned)s.N);
+    if (v4)
+        hipLaunchKernelGGL((cce_dz_k<TZ, 4>), grid, dim3(256), 0, st, z, e.dz, e.tgt, e.lse, s.V, ld,
+                           e.inv_n, e.t_scale, e.eps_over_v, e.zl2);
+    else
+        hipLaunchKernelGGL((cce_dz_k<TZ, 1>), grid, dim3(256), 0, st, z, e.dz, e.tgt, e.lse, s.V, ld,
+                           e.inv_n, e.t_scale, e.eps_over_v, e.zl2);
+    return hipGetLastError();
+}
+
+template <typename TZ>
+EpiCceDz<TZ> dz_epi(const CceShape &s, TZ *dz, const uint32_t *tgt, const float *lse) {
+    return EpiCceDz<TZ>{dz, tgt, lse, s.V, s.zs(), 1.0f / (float)s.N, 1.0f - s.label_smoothing,
+                        s.label_smoothing / (float)s.V, 2.0f * s.z_loss_scale};
+}
+
+hipError_t merge(const CceShape &s, const CceWork &cw, float *lse, float *loss_row, float *loss_mean,
+                 hipStream_t st) {
+    hipLaunchKernelGGL(cce_merge_k, dim3(ceil_div(s.N, 4)), dim3(256), 0, st, s, cw, lse, loss_row);
+    if (loss_mean) hipLaunchKernelGGL(cce_mean_k, dim3(1), dim3(256), 0, st, s, cw, loss_mean);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -275,105 +326,54 @@ size_t cce_work_floats(const CceShape &s) {
     return 3 * (size_t)s.N * np + s.N;
 }
 
-hipError_t cce_forward(Precision pr, const CceShape &s, const float *h, const float *w,
-                       const uint32_t *tgt, float *lse, float *loss_row, float *loss_mean,
-                       float *work, hipStream_t st, float *z_out) {
+hipError_t cce_forward(const CceShape &s, const float *h, const float *w, const uint32_t *tgt,
+                       float *lse, float *loss_row, float *loss_mean, float *work, hipStream_t st,
+                       float *z_out) {
     if (s.N <= 0) return hipSuccess;
-    CceWork cw = carve(work, s);
-    EpiCceStats e{cw, tgt, s.V, z_out};
-    hipError_t err = logits_gemm(pr, s, h, w, e, st);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(cce_merge_k, dim3(ceil_div(s.N, 4)), dim3(256), 0, st, s, cw, lse, loss_row);
-    if (loss_mean) hipLaunchKernelGGL(cce_mean_k, dim3(1), dim3(256), 0, st, s, cw, loss_mean);
-    return hipGetLastError();
+    const CceWork cw = carve(work, s);
+    const hipError_t err = logits32(s, h, w, EpiCceStats{cw, tgt, s.V, z_out, s.zs()}, st);
+    return err != hipSuccess ? err : merge(s, cw, lse, loss_row, loss_mean, st);
 }
 
-hipError_t cce_backward(Precision pr, const CceShape &s, const float *h, const float *w,
-                        const uint32_t *tgt, const float *lse, void *dz, float *dh, float *dw,
-                        float dw_beta, const GemmWs &ws, hipStream_t st, const float *z) {
+hipError_t cce_backward(const CceShape &s, const float *h, const float *w, const uint32_t *tgt,
+                        const float *lse, float *dz, float *dh, float *dw, float dw_beta,
+                        const GemmWs &ws, hipStream_t st, const float *z) {
     if (s.N <= 0) return hipSuccess;
-    const float inv_n = 1.0f / (float)s.N;
-    const float t_scale = 1.0f - s.label_smoothing;
-    const float eps_over_v = s.label_smoothing / (float)s.V;
-    const float zl2 = 2.0f * s.z_loss_scale;
-    hipError_t err;
-    const DType zdt = pr == Precision::BF16 ? DType::BF16 : DType::F32;
-    if (z) {  // the logits the forward stored: dz in one streaming pass
-        const bool v4 = s.V % 4 == 0 && ((uintptr_t)z & 15u) == 0 && ((uintptr_t)dz & 15u) == 0;
-        const dim3 grid((unsigned)ceil_div(s.V, 256 * (v4 ? 4 : 1)), (unsigned)s.N);
-        if (zdt == DType::BF16) {
-            if (v4) hipLaunchKernelGGL((cce_dz_k<bf16, 4>), grid, dim3(256), 0, st, z, (bf16 *)dz, tgt, lse, s.V, inv_n, t_scale, eps_over_v, zl2);
-            else hipLaunchKernelGGL((cce_dz_k<bf16, 1>), grid, dim3(256), 0, st, z, (bf16 *)dz, tgt, lse, s.V, inv_n, t_scale, eps_over_v, zl2);
-        } else {
-            if (v4) hipLaunchKernelGGL((cce_dz_k<float, 4>), grid, dim3(256), 0, st, z, (float *)dz, tgt, lse, s.V, inv_n, t_scale, eps_over_v, zl2);
-            else hipLaunchKernelGGL((cce_dz_k<float, 1>), grid, dim3(256), 0, st, z, (float *)dz, tgt, lse, s.V, inv_n, t_scale, eps_over_v, zl2);
-        }
-        err = hipGetLastError();
-    } else if (zdt == DType::BF16) {
-        EpiCceDz<bf16> e{(bf16 *)dz, tgt, lse, s.V, inv_n, t_scale, eps_over_v, zl2};
-        err = logits_gemm(pr, s, h, w, e, st);
-    } else {
-        EpiCceDz<float> e{(float *)dz, tgt, lse, s.V, inv_n, t_scale, eps_over_v, zl2};
-        err = logits_gemm(pr, s, h, w, e, st);
-    }
+    const EpiCceDz<float> e = dz_epi(s, dz, tgt, lse);
+    hipError_t err = z ? dz_from_logits(s, z, e, st) : logits32(s, h, w, e, st);
     if (err != hipSuccess) return err;
-    const Mat mz{dz, s.V, zdt};
-    if (zdt == DType::F32) {  // fp32: the DMA-staged fp32 kernels (generic where they do not apply)
-        if (dw) {
-            err = g32_tn((const float *)dz, s.V, h, s.D, dw, s.D, s.N, s.V, s.D, 1.f, dw_beta, ws, st);
-            if (err != hipSuccess) return err;
-        }
-        if (dh) err = g32_nn((const float *)dz, s.V, w, s.D, dh, s.D, s.N, s.V, s.D, 1.f, 0.f, ws, st);
-        return err;
-    }
+    // dW[V, D] = dz^T h ;  dh[N, D] = dz W
+    const bool pad = s.ldh || s.ldz;
     if (dw) {
-        err = gemm_tn(pr, mz, matf(h, s.D), dw, s.D, s.N, s.V, s.D, 1.f, dw_beta, st);
+        err = g32_tn(dz, s.zs(), h, s.hs(), dw, s.D, s.N, s.V, s.D, 1.f, dw_beta, ws, st, pad);
         if (err != hipSuccess) return err;
     }
-    if (dh) err = gemm_nn(pr, mz, matf(w, s.D), dh, s.D, s.N, s.V, s.D, 1.f, 0.f, st);
+    if (dh) err = g32_nn(dz, s.zs(), w, s.hs(), dh, s.D, s.N, s.V, s.D, 1.f, 0.f, ws, st, pad);
     return err;
 }
-
-}  // namespace vkh
-
-namespace vkh {
 
 hipError_t cce_forward16(const CceShape &s, const bf16 *h, const bf16 *w, const uint32_t *tgt,
                          float *lse, float *loss_row, float *loss_mean, float *work,
                          hipStream_t st, float *z_out) {
     if (s.N <= 0) return hipSuccess;
-    CceWork cw = carve(work, s);
-    EpiCceStats e{cw, tgt, s.V, z_out};
-    hipError_t err = logits16(s, h, w, e, st);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(cce_merge_k, dim3(ceil_div(s.N, 4)), dim3(256), 0, st, s, cw, lse, loss_row);
-    if (loss_mean) hipLaunchKernelGGL(cce_mean_k, dim3(1), dim3(256), 0, st, s, cw, loss_mean);
-    return hipGetLastError();
+    const CceWork cw = carve(work, s);
+    const hipError_t err = logits16(s, h, w, EpiCceStats{cw, tgt, s.V, z_out, s.zs()}, st);
+    return err != hipSuccess ? err : merge(s, cw, lse, loss_row, loss_mean, st);
 }
 
 hipError_t cce_backward16(const CceShape &s, const bf16 *h, const bf16 *w, const uint32_t *tgt,
                           const float *lse, bf16 *dz, float *dh, float *dw, float dw_beta,
                           const GemmWs &ws, hipStream_t st, const float *z) {
     if (s.N <= 0) return hipSuccess;
-    EpiCceDz<bf16> e{dz, tgt, lse, s.V, 1.0f / (float)s.N, 1.0f - s.label_smoothing,
-                     s.label_smoothing / (float)s.V, 2.0f * s.z_loss_scale};
-    hipError_t err;
-    if (z) {
-        const bool v4 = s.V % 4 == 0 && ((uintptr_t)z & 15u) == 0;
-        const dim3 grid((unsigned)ceil_div(s.V, 256 * (v4 ? 4 : 1)), (unsigned)s.N);
-        if (v4) hipLaunchKernelGGL((cce_dz_k<bf16, 4>), grid, dim3(256), 0, st, z, dz, tgt, lse, s.V, e.inv_n, e.t_scale, e.eps_over_v, e.zl2);
-        else hipLaunchKernelGGL((cce_dz_k<bf16, 1>), grid, dim3(256), 0, st, z, dz, tgt, lse, s.V, e.inv_n, e.t_scale, e.eps_over_v, e.zl2);
-        err = hipGetLastError();
-    } else {
-        err = logits16(s, h, w, e, st);
-    }
+    const EpiCceDz<bf16> e = dz_epi(s, dz, tgt, lse);
+    hipError_t err = z ? dz_from_logits(s, z, e, st) : logits16(s, h, w, e, st);
     if (err != hipSuccess) return err;
-    // dW[V, D] = dz^T h ;  dh[N, D] = dz W
+    const bool pad = s.ldh || s.ldz;
     if (dw) {
-        err = g16_tn(dz, s.V, h, s.D, dw, s.D, s.N, s.V, s.D, 1.f, dw_beta, ws, st);
+        err = g16_tn(dz, s.zs(), h, s.hs(), dw, s.D, s.N, s.V, s.D, 1.f, dw_beta, ws, st, pad);
         if (err != hipSuccess) return err;
     }
-    if (dh) err = g16_nn(dz, s.V, w, s.D, dh, s.D, s.N, s.V, s.D, 1.f, 0.f, ws, st);
+    if (dh) err = g16_nn(dz, s.zs(), w, s.hs(), dh, s.D, s.N, s.V, s.D, 1.f, 0.f, ws, st, pad);
     return err;
 }
 

@@ -243,7 +243,8 @@ hipError_t run32(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e,
 
 // fp32 operand view: 16-byte aligned, ld and the contiguous run multiples of 4
 // floats (whole 16-byte chunks), under 2 GiB (32-bit buffer offsets).
-bool make_op32(const float *p, long ld, long rows, long run, Op16 &o) {
+bool make_op32(const float *p, long ld, long rows, long run, Op16 &o, bool padded = false) {
+    if (padded) run = std::min(ld, (run + 3) / 4 * 4);
     if (((uintptr_t)p & 15u) || ld % 4 || run % 4 || rows <= 0) return false;
     const size_t bytes = ((size_t)(rows - 1) * ld + run) * 4;
     if (bytes >= (1ull << 31)) return false;
@@ -254,7 +255,8 @@ bool make_op32(const float *p, long ld, long rows, long run, Op16 &o) {
 Mat matf32(const float *p, long ld) { return Mat{p, ld, DType::F32}; }
 
 // Operand of `rows` storage rows whose contiguous run is `run` elements.
-bool make_op(const bf16 *p, long ld, long rows, long run, Op16 &o) {
+bool make_op(const bf16 *p, long ld, long rows, long run, Op16 &o, bool padded = false) {
+    if (padded) run = std::min(ld, (run + 7) / 8 * 8);
     if (((uintptr_t)p & 15u) || ld % 8 || run % 8 || rows <= 0) return false;
     const size_t bytes = ((size_t)(rows - 1) * ld + run) * 2;
     if (bytes >= (1ull << 31)) return false;
@@ -584,19 +586,19 @@ hipError_t g32_gate_up_swiglu(const float *x, long ldx, const float *w, long ldw
 }
 
 hipError_t g16_nn(const bf16 *dy, long lddy, const bf16 *w, long ldw, float *dx, long lddx, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st) {
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st, bool padded) {
     // an over-2 GiB dy (the head's dz at 8192 tokens): independent row chunks
     if (const int mc = M > 64 ? rows_per_2g_chunk(M, lddy, N) : 0) {
         for (int m0 = 0; m0 < M; m0 += mc) {
             const hipError_t e = g16_nn(dy + (long)m0 * lddy, lddy, w, ldw, dx + (long)m0 * lddx,
-                                        lddx, std::min(mc, M - m0), N, K, alpha, beta, ws, st);
+                                        lddx, std::min(mc, M - m0), N, K, alpha, beta, ws, st, padded);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     }
     // C[m, k'] = sum_n dy[m, n] W[n, k']: A = dy (K-major over n), B(k', n) = W[n][k'] (MN)
     Op16 a, b;
-    if (!make_op(dy, lddy, M, N, a) || !make_op(w, ldw, N, K, b))
+    if (!make_op(dy, lddy, M, N, a, padded) || !make_op(w, ldw, N, K, b, padded))
         return gemm_nn(Precision::BF16, matb(dy, lddy), matb(w, ldw), dx, lddx, M, N, K, alpha,
                        beta, st);
     EpiStore e{dx, lddx, nullptr, 0, alpha, beta};
@@ -612,21 +614,22 @@ hipError_t g16_nn_bf16(const bf16 *dy, long lddy, const bf16 *w, long ldw, bf16 
 }
 
 hipError_t g16_tn(const bf16 *dy, long lddy, const bf16 *x, long ldx, float *dw, long lddw, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st) {
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st, bool padded) {
     // an over-2 GiB dy (the head's dz at 8192 tokens): the contraction over m in
     // row chunks, each chunk after the first accumulating (beta = 1)
     const int ca = M > 64 ? rows_per_2g_chunk(M, lddy, N) : 0, cb = M > 64 ? rows_per_2g_chunk(M, ldx, K) : 0;
     if (const int mc = (ca && cb) ? std::min(ca, cb) : std::max(ca, cb)) {
         for (int m0 = 0; m0 < M; m0 += mc) {
             const hipError_t e = g16_tn(dy + (long)m0 * lddy, lddy, x + (long)m0 * ldx, ldx, dw, lddw,
-                                        std::min(mc, M - m0), N, K, alpha, m0 ? 1.f : beta, ws, st);
+                                        std::min(mc, M - m0), N, K, alpha, m0 ? 1.f : beta, ws, st,
+                                        padded);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     }
     // C[n, k'] = sum_m dy[m, n] x[m, k']: both operands MN-major over m
     Op16 a, b;
-    if (!make_op(dy, lddy, M, N, a) || !make_op(x, ldx, M, K, b))
+    if (!make_op(dy, lddy, M, N, a, padded) || !make_op(x, ldx, M, K, b, padded))
         return gemm_tn(Precision::BF16, matb(dy, lddy), matb(x, ldx), dw, lddw, M, N, K, alpha,
                        beta, st);
     EpiStore e{dw, lddw, nullptr, 0, alpha, beta};
@@ -645,9 +648,9 @@ hipError_t g32_nt(const float *x, long ldx, const float *w, long ldw, float *y, 
 }
 
 hipError_t g32_nn(const float *dy, long lddy, const float *w, long ldw, float *dx, long lddx, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st) {
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st, bool padded) {
     Op16 a, b;
-    if (!make_op32(dy, lddy, M, N, a) || !make_op32(w, ldw, N, K, b))
+    if (!make_op32(dy, lddy, M, N, a, padded) || !make_op32(w, ldw, N, K, b, padded))
         return gemm_nn(Precision::FP32, matf32(dy, lddy), matf32(w, ldw), dx, lddx, M, N, K, alpha,
                        beta, st);
     EpiStore e{dx, lddx, nullptr, 0, alpha, beta};
@@ -655,9 +658,9 @@ hipError_t g32_nn(const float *dy, long lddy, const float *w, long ldw, float *d
 }
 
 hipError_t g32_tn(const float *dy, long lddy, const float *x, long ldx, float *dw, long lddw, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st) {
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st, bool padded) {
     Op16 a, b;
-    if (!make_op32(dy, lddy, M, N, a) || !make_op32(x, ldx, M, K, b))
+    if (!make_op32(dy, lddy, M, N, a, padded) || !make_op32(x, ldx, M, K, b, padded))
         return gemm_tn(Precision::FP32, matf32(dy, lddy), matf32(x, ldx), dw, lddw, M, N, K, alpha,
                        beta, st);
     EpiStore e{dw, lddw, nullptr, 0, alpha, beta};

@@ -58,13 +58,17 @@ hipError_t g16_nt(const bf16 *x, long ldx, const bf16 *w, long ldw, float *y, lo
 hipError_t g16_gate_up_swiglu(const bf16 *x, long ldx, const bf16 *w, long ldw, float *gu,
                               long ldgu, bf16 *gated, long ldg, int M, int F, int K, hipStream_t st,
                               bool paired = false);
+// padded (here and below): the rows of both operands run on with zeros to whole 16-byte
+// chunks, so their widths need not be multiples of one.
 hipError_t g16_nn(const bf16 *dy, long lddy, const bf16 *w, long ldw, float *dx, long lddx, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st);
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st,
+                  bool padded = false);
 // dx as bf16 (the operand precision of the next kernel), no split-K / fp32 copy.
 hipError_t g16_nn_bf16(const bf16 *dy, long lddy, const bf16 *w, long ldw, bf16 *dx, long lddx,
                        int M, int N, int K, const GemmWs &ws, hipStream_t st);
 hipError_t g16_tn(const bf16 *dy, long lddy, const bf16 *x, long ldx, float *dw, long lddw, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st);
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st,
+                  bool padded = false);
 size_t g16_ws_bytes_for(int M, int N, int K);
 // fp32 operands on the same DMA-staged kernels (fp32 matrix cores); operands
 // the DMA path cannot take (alignment, ld or extent not a multiple of 4, over
@@ -73,9 +77,11 @@ hipError_t g32_nt(const float *x, long ldx, const float *w, long ldw, float *y, 
                   int N, int K, const float *R, long ldr, float alpha, float beta,
                   const GemmWs &ws, hipStream_t st);
 hipError_t g32_nn(const float *dy, long lddy, const float *w, long ldw, float *dx, long lddx, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st);
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st,
+                  bool padded = false);
 hipError_t g32_tn(const float *dy, long lddy, const float *x, long ldx, float *dw, long lddw, int M,
-                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st);
+                  int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st,
+                  bool padded = false);
 size_t g32_ws_bytes_for(int M, int N, int K);
 // The three contractions of a linear layer on dense row-major operands of any
 // width and alignment: NT y = x W^T (a = x, b = W), NN dx = dy W, TN dW = dy^T x,
@@ -404,11 +410,17 @@ hipError_t fa_bw_fused(const AttnShape &s, const AttnPtrs &p, bf16 *ds_ws, bool 
 struct CceShape {
     int N, V, D;
     float z_loss_scale, label_smoothing;
+    // row strides: of h and W (0: D) and of dz and the stored logits (0: V).  Where a
+    // stride is more, h and W hold zeros from D on, and dz gets zeros from V on, so that
+    // every row is whole 16-byte chunks for the DMA-staged products.
+    long ldh = 0, ldz = 0;
+    long hs() const { return ldh ? ldh : D; }
+    long zs() const { return ldz ? ldz : V; }
 };
 size_t cce_work_floats(const CceShape &s);
-// z_out (optional): the fp32 logits [N, V] are stored there too, for
+// z_out (optional): the fp32 logits (rows of zs()) are stored there too, for
 // cce_backward's z.
-hipError_t cce_forward(Precision pr, const CceShape &s, const float *h, const float *w,
+hipError_t cce_forward(const CceShape &s, const float *h, const float *w,
                        const uint32_t *tgt, float *lse, float *loss_row, float *loss_mean,
                        float *work, hipStream_t st, float *z_out = nullptr);
 // bf16-operand forms (h, W bf16; dz bf16), on the gemm16 kernel.
@@ -418,12 +430,12 @@ hipError_t cce_forward16(const CceShape &s, const bf16 *h, const bf16 *w, const 
 hipError_t cce_backward16(const CceShape &s, const bf16 *h, const bf16 *w, const uint32_t *tgt,
                           const float *lse, bf16 *dz, float *dh, float *dw, float dw_beta,
                           const GemmWs &ws, hipStream_t st, const float *z = nullptr);
-// dz (bf16 for Precision::BF16 else fp32) [N, V] is materialised in `dz`;
+// fp32 operands: dz [N, zs()] is materialised in `dz`;
 // dh overwritten (if non-null); dW = beta*dW + dz^T h (if non-null).  z: the
 // logits cce_forward stored with z_out (may be dz itself), read instead of
 // recomputing them; nullptr recomputes.
-hipError_t cce_backward(Precision pr, const CceShape &s, const float *h, const float *w,
-                        const uint32_t *tgt, const float *lse, void *dz, float *dh, float *dw,
+hipError_t cce_backward(const CceShape &s, const float *h, const float *w,
+                        const uint32_t *tgt, const float *lse, float *dz, float *dh, float *dw,
                         float dw_beta, const GemmWs &ws, hipStream_t st, const float *z = nullptr);
 
 }  // namespace vkh

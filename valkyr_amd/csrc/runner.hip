@@ -613,13 +613,13 @@ struct vkh_runner {
         size_t pf = rmsnorm_partial_floats(T, D);
         if (qk_partial_floats() > pf) pf = qk_partial_floats();
         VKH_TRY(alloc(partial, pf));
-        CceShape cs{T, V, D, 0.f, 0.f};
+        const CceShape cs = cce_shape();
         VKH_TRY(alloc(cce_work, cce_work_floats(cs)));
         char *z = nullptr;
-        VKH_TRY(alloc(z, (size_t)T * V * (b16() ? 2 : 4)));
+        VKH_TRY(alloc(z, (size_t)T * cs.zs() * (b16() ? 2 : 4)));
         // 18.41-18.47 -> 18.27-18.29 ms at config 3 (1.24 GB), same losses; config 5
         // (8192 tokens, 4.98 GB): 587.4 -> 581.4-581.7 ms in 157.1 GiB
-        if (b16() && (size_t)T * V * 4 <= kLogitsCap) VKH_TRY(alloc(zf, (size_t)T * V));
+        if (b16() && (size_t)T * V * 4 <= kLogitsCap) VKH_TRY(alloc(zf, (size_t)T * cs.zs()));
         dz = z;
         char *ew = nullptr;
         VKH_TRY(alloc(ew, embed_bw_work_bytes(T)));
@@ -1368,11 +1368,20 @@ struct vkh_runner {
         return VKH_OK;
     }
 
+    // The head's shape.  bf16: rows of dz and of the kept logits are whole 16-byte chunks
+    // also for an odd vocabulary, so that its dh and dW take the DMA-staged GEMMs; fp32
+    // keeps dense rows and, there, the generic GEMM's summation order.
+    CceShape cce_shape() const {
+        CceShape cs{T, V, D, 0.f, 0.f};
+        if (b16() && V % 8) cs.ldz = lin_packed_ld(LinForm::BF16, V);
+        return cs;
+    }
+
     // with_adam: the concurrent mode applies Adam inside the backward (per layer
     // on the side stream); otherwise the caller enqueues adam_enqueue() after.
     vkh_status forward_backward_enqueue(bool with_adam) {
         VKH_TRY(forward_all());
-        const CceShape cs{T, V, D, 0.f, 0.f};
+        const CceShape cs = cce_shape();
         // head backward: dh and dW_lm (tied: the embed grad slot)
         float *dw_lm = lora ? nullptr : Gd(lm_head);
         const bool split = with_adam && embed_split_ok();
@@ -1393,21 +1402,22 @@ struct vkh_runner {
                 // below adds into the same gradient and waits for it
                 VKH_HIP(hipEventRecord(ev_head, cur));
                 VKH_HIP(hipStreamWaitEvent(side, ev_head, 0));
-                VKH_HIP(g16_tn((const bf16 *)dz, V, fn_outb, D, dw_lm, D, T, V, D, 1.f, 0.f, gws2, side));
+                VKH_HIP(g16_tn((const bf16 *)dz, cs.zs(), fn_outb, D, dw_lm, D, T, V, D, 1.f, 0.f, gws2, side,
+                               cs.ldz != 0));
                 if (split) VKH_TRY(embed_adam_early());
                 VKH_HIP(hipEventRecord(ev_lm, side));
             }
         } else {
             // the fp32 logits kept in the dz buffer, which the backward turns
             // into dz in place (no second logits GEMM)
-            VKH_HIP(cce_forward(pr, cs, fn_out, W(lm_head), tgt_d, ce_lse, loss_row, loss_mean,
+            VKH_HIP(cce_forward(cs, fn_out, W(lm_head), tgt_d, ce_lse, loss_row, loss_mean,
                                 cce_work, cur, (float *)dz));
             // two streams: dW_lm on the side stream starts as soon as dz is
             // written, beside dh on the main stream (fp32: 75.97-75.99 -> 75.30 ms,
             // same losses; the bf16 step, whose dh is the short split-K form,
             // measured 0.05-0.09 ms slower this way and keeps dh first)
             const bool dw_early = concurrent && dw_lm;
-            VKH_HIP(cce_backward(pr, cs, fn_out, W(lm_head), tgt_d, ce_lse, dz, dw_early ? nullptr : d_fn,
+            VKH_HIP(cce_backward(cs, fn_out, W(lm_head), tgt_d, ce_lse, (float *)dz, dw_early ? nullptr : d_fn,
                                  concurrent ? nullptr : dw_lm, 0.f, gws, cur, (const float *)dz));
             if (concurrent && dw_lm) {  // as above, on the fp32 logits gradient
                 if (split) {
@@ -1647,12 +1657,12 @@ struct vkh_runner {
     // target, so a new batch whose loss is above the target resumes training).
     vkh_status loss_eval_enqueue() {
         VKH_TRY(forward_all());
-        const CceShape cs{T, V, D, 0.f, 0.f};
+        const CceShape cs = cce_shape();
         if (b16())
             VKH_HIP(cce_forward16(cs, fn_outb, Wb(lm_head), tgt_d, ce_lse, loss_row, loss_mean,
                                   cce_work, cur));
         else
-            VKH_HIP(cce_forward(pr, cs, fn_out, W(lm_head), tgt_d, ce_lse, loss_row, loss_mean,
+            VKH_HIP(cce_forward(cs, fn_out, W(lm_head), tgt_d, ce_lse, loss_row, loss_mean,
                                 cce_work, cur));
         return record_tick_loss();
     }
