@@ -765,6 +765,45 @@ FA_BF16_CASES = [  # (n, H, Hkv, hd, causal, B)
 ]
 
 
+@pytest.mark.parametrize("case", [  # (n_q, n_kv, H, Hkv, hd, causal, B)
+    (1, 1, 4, 2, 64, True, 2), (100, 100, 16, 8, 128, True, 1), (65, 65, 8, 2, 64, True, 2),
+    (33, 97, 4, 2, 128, True, 1), (64, 129, 4, 4, 128, True, 2), (31, 200, 4, 4, 64, False, 2),
+    (200, 31, 4, 2, 128, False, 1), (257, 257, 4, 1, 128, True, 1)])
+def test_flash_attention_fp32_ragged_lengths(case):
+    """The fp32 matrix-core kernels on lengths that are not whole tiles (one row, a row
+    past a tile, causal with more keys than queries, either side longer without a mask),
+    held to test_flash_attention_fp32's bounds."""
+    test_flash_attention_fp32(case)
+
+
+def test_flash_attention_fp32_ragged_masked_rows():
+    """A query whose scores are all -inf (keys of -inf against a positive query, as an
+    additive mask leaves them) gets O = 0, LSE = -inf, and no gradient flows from it."""
+    from valkyr_amd import kernels as K
+
+    n, H, hd = 37, 2, 64
+    q, k = O.normal(n * H * hd, 11), np.zeros((n, H, hd), np.float32)
+    q = q.reshape(n, H, hd)
+    q[:, :, 0] = 1.0
+    k[:5, :, 0] = -np.inf
+    v, do = O.normal(n * H * hd, 12), O.normal(n * H * hd, 13)
+    p = K.attn_params(n, n, H, H, hd, True, 1, K.F32)
+    bq, bk, bv, bdo = dev(q), dev(k), dev(v), dev(do)
+    bo, blse, bd = zeros(n * H * hd), zeros(n * H), zeros(n * H)
+    bdk, bdv = zeros(n * H * hd), zeros(n * H * hd)
+    K.fa_forward(p, bq, bk, bv, bo, blse)
+    K.fa_bw_d(p, bo, bdo, bd)
+    K.fa_bw_dkv(p, bq, bk, bv, bdo, blse, bd, bdk, bdv)
+    o, lse = host(bo).reshape(n, H, hd), host(blse).reshape(n, H)
+    assert np.all(o[:5] == 0) and np.all(lse[:5] == -np.inf)
+    # keys of one finite score: O is the mean of the visible values, LSE = log(count)
+    cnt = np.arange(1, n - 4)
+    ref = np.cumsum(v.reshape(n, H, hd)[5:].astype(np.float64), 0) / cnt[:, None, None]
+    assert rel_l2(ref, o[5:]) < 1e-6 and np.allclose(lse[5:], np.log(cnt)[:, None], atol=1e-6)
+    dv = host(bdv).reshape(n, H, hd)
+    assert np.all(np.isfinite(dv)) and np.all(dv[:5] == 0)
+
+
 @pytest.mark.parametrize("hd,rows", [(128, 4 * 2048 * 16), (64, 3 * 100 * 4)])
 def test_fa_bw_d_bf16_inputs(hd, rows):
     """D = rowsum(O dO) from bf16 O and dO (fa_bw_d.comp with bf16 storage) vs

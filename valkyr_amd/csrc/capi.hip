@@ -140,6 +140,7 @@ static AttnShape attn_shape(const vkh_attn_params *p) {
     s.n_batch = p->n_batch ? (int)p->n_batch : 1;
     s.n_q = p->n_q; s.n_kv = p->n_kv; s.n_heads = p->n_heads; s.n_kv_heads = p->n_kv_heads;
     s.head_dim = p->head_dim; s.causal = p->causal ? 1 : 0; s.inv_sqrt_dim = p->inv_sqrt_dim;
+    s.ragged = 1;
     return s;
 }
 

@@ -66,6 +66,14 @@ struct Tile {
             v[i] = f4(base + (long)r * ld + 4 * c);
         }
     }
+    // rows from `rows` on are zero
+    VKH_DEV void load(const float *base, long ld, int tid, int rows) {
+#pragma unroll
+        for (int i = 0; i < N4; ++i) {
+            const int x = tid + NT * i, r = x / (HD / 4), c = x % (HD / 4);
+            v[i] = r < rows ? f4(base + (long)r * ld + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
     VKH_DEV void store(float *lds, int tid) const {
 #pragma unroll
         for (int i = 0; i < N4; ++i) {
@@ -75,8 +83,15 @@ struct Tile {
     }
 };
 
+// RAG (all three kernels): any n_q and n_kv, a causal mask also with n_q < n_kv
+// (query q sees keys up to q + n_kv - n_q).  Rows past the end load as zero and are
+// not stored, their scores are masked to exact zeros, and a row whose scores are all
+// -inf gets O = 0 and LSE = -inf (backward: no gradient), as the per-row kernels do.
+// Bound by the matrix cores of the few CUs a short sequence reaches; against the
+// per-row kernels (one wave a row, a dot product at a time).
+
 // ── forward: block = 64 queries of one (sequence, head) ─────────────────
-template <int HD>
+template <int HD, bool RAG = false>
 __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float *q, long ldq,
                                                        const float *k, long ldk, const float *v,
                                                        long ldv, float *o, long ldo, float *lse,
@@ -84,7 +99,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
     constexpr int P = HD + 4, NU = HD / 16;
     __shared__ __attribute__((aligned(16))) float Ks[2][FT * P], Vs[2][FT * P];
     const int h = blockIdx.x % s.n_heads, b = blockIdx.x / s.n_heads;
-    const int nqb = s.n_q / 64;
+    const int nqb = (s.n_q + 63) / 64;
     const int y = (int)blockIdx.y, qb = s.causal ? nqb - 1 - (zz ? zigzag(y, nqb) : y) : y;
     const int tid = threadIdx.x, lane = tid % 64, g = lane / 16, c = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -93,16 +108,27 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
     const float c2 = s.inv_sqrt_dim * F_LOG2E;
     float4 qf[NU];  // B of S^T = K Q^T: Q[qi][16 u + 4 g + e], pre-scaled
     {
-        const float *qr = q + ((long)b * s.n_q + qi) * ldq + h * HD + 4 * g;
+        const int ql = RAG ? min(qi, s.n_q - 1) : qi;  // (rows past the end are not stored)
+        const float *qr = q + ((long)b * s.n_q + ql) * ldq + h * HD + 4 * g;
 #pragma unroll
         for (int u = 0; u < NU; ++u) qf[u] = f4_scale(f4(qr + 16 * u), c2);
     }
-    const int nkt = s.causal ? (q0 + 64) / FT : s.n_kv / FT;
+    const int shift = RAG ? s.n_kv - s.n_q : 0;
+    const int nkt = RAG ? ((s.causal ? min(s.n_kv, q0 + 64 + shift) : s.n_kv) + FT - 1) / FT
+                        : s.causal ? (q0 + 64) / FT : s.n_kv / FT;
     const float *kb = k + (long)b * s.n_kv * ldk + kvh * HD;
     const float *vb = v + (long)b * s.n_kv * ldv + kvh * HD;
     Tile<HD> tk, tv;
-    tk.load(kb, ldk, tid);
-    tv.load(vb, ldv, tid);
+    auto load = [&](int it) {
+        if constexpr (RAG) {
+            tk.load(kb + (long)it * FT * ldk, ldk, tid, s.n_kv - it * FT);
+            tv.load(vb + (long)it * FT * ldv, ldv, tid, s.n_kv - it * FT);
+        } else {
+            tk.load(kb + (long)it * FT * ldk, ldk, tid);
+            tv.load(vb + (long)it * FT * ldv, ldv, tid);
+        }
+    };
+    load(0);
     tk.store(Ks[0], tid);
     tv.store(Vs[0], tid);
     __syncthreads();
@@ -112,10 +138,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
     float m = -INFINITY, l = 0.f;  // running max (log2 units) and this lane's share of the sum
     for (int it = 0; it < nkt; ++it) {
         const int buf = it & 1;
-        if (it + 1 < nkt) {
-            tk.load(kb + (long)(it + 1) * FT * ldk, ldk, tid);
-            tv.load(vb + (long)(it + 1) * FT * ldv, ldv, tid);
-        }
+        if (it + 1 < nkt) load(it + 1);
         const float *Kl = Ks[buf], *Vl = Vs[buf];
         const int kt0 = it * FT;
         f32x4 st[2];  // S^T[kt0 + 16 ks + 4 g + r][qi]
@@ -123,7 +146,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             st[ks] = f32x4{0, 0, 0, 0};
-            live[ks] = !s.causal || kt0 + 16 * ks <= qw + 15;  // wave-uniform
+            live[ks] = !s.causal || kt0 + 16 * ks <= qw + 15 + shift;  // wave-uniform
             if (live[ks]) {
                 const float *kr = Kl + (16 * ks + c) * P + 4 * g;
 #pragma unroll
@@ -135,11 +158,13 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                if (s.causal && kt0 + 16 * ks + 4 * g + r > qi) st[ks][r] = -INFINITY;
+                const int kk = kt0 + 16 * ks + 4 * g + r;
+                if ((s.causal && kk > qi + shift) || (RAG && kk >= s.n_kv)) st[ks][r] = -INFINITY;
                 tmax = fmaxf(tmax, st[ks][r]);
             }
-        const float mn = fmaxf(m, xmax(tmax));  // finite: tile 0 holds key 0 <= qi
-        const float alpha = __builtin_amdgcn_exp2f(m - mn);
+        const float mn = fmaxf(m, xmax(tmax));  // finite for finite scores: tile 0 holds key 0 <= qi
+        const float ms = RAG && mn == -INFINITY ? 0.f : mn;  // every score so far is -inf: P = 0
+        const float alpha = __builtin_amdgcn_exp2f(m - ms);
         l *= alpha;
 #pragma unroll
         for (int j = 0; j < NU; ++j) ot[j] *= alpha;
@@ -147,7 +172,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float pv = __builtin_amdgcn_exp2f(st[ks][r] - mn);
+                const float pv = __builtin_amdgcn_exp2f(st[ks][r] - ms);
                 st[ks][r] = pv;
                 l += pv;
             }
@@ -170,7 +195,8 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
         __syncthreads();
     }
     l = xsum(l);
-    const float inv = 1.0f / l;
+    if (RAG && qi >= s.n_q) return;
+    const float inv = RAG && l == 0.f ? 0.f : 1.0f / l;
     float *orow = o + ((long)b * s.n_q + qi) * ldo + h * HD + 4 * g;
 #pragma unroll
     for (int j = 0; j < NU; ++j)
@@ -196,16 +222,16 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
 // total work, not by this kernel's span.)
 // QKE: dK leaves through RoPE^T and the K-RMSNorm backward (p.qk), each block
 // writing its k-gain partial to p.qk.pk[block].
-template <int HD, bool QKE>
+template <int HD, bool QKE, bool RAG = false>
 __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtrs p, bool zz) {
-    static_assert(!QKE || HD == 128, "the fused q/k epilogue takes 128-wide head rows");
+    static_assert(!QKE || (HD == 128 && !RAG), "the fused q/k epilogue takes 128-wide head rows");
     constexpr int P = HD + 4, NU = HD / 16;
     __shared__ __attribute__((aligned(16))) float Qs[2][FT * P], Os[2][FT * P];
     __shared__ float Ls[2][FT], Dl[2][FT];
     const int kvh = blockIdx.x % s.n_kv_heads, b = blockIdx.x / s.n_kv_heads;
     const int tid = threadIdx.x, lane = tid % 64, g = lane / 16, c = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
-    const int kb = s.causal && zz ? zigzag((int)blockIdx.y, s.n_kv / 64) : (int)blockIdx.y;
+    const int kb = s.causal && zz ? zigzag((int)blockIdx.y, (s.n_kv + 63) / 64) : (int)blockIdx.y;
     const int k0 = kb * 64, kw = k0 + 16 * wave, ki = kw + c;
     const int hpk = s.n_heads / s.n_kv_heads;
     const float c2 = s.inv_sqrt_dim * F_LOG2E;
@@ -213,16 +239,18 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
                 *dO = (const float *)p.dout;
     float4 kf[NU], vf[NU];  // B of S = Q K^T and dP = dO V^T: K / V[ki][16 u + 4 g + e]
     {
-        const float *kr = K + ((long)b * s.n_kv + ki) * p.ldk + kvh * HD + 4 * g;
-        const float *vr = V + ((long)b * s.n_kv + ki) * p.ldv + kvh * HD + 4 * g;
+        const int kl = RAG ? min(ki, s.n_kv - 1) : ki;  // (rows past the end are not stored)
+        const float *kr = K + ((long)b * s.n_kv + kl) * p.ldk + kvh * HD + 4 * g;
+        const float *vr = V + ((long)b * s.n_kv + kl) * p.ldv + kvh * HD + 4 * g;
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
             kf[u] = f4_scale(f4(kr + 16 * u), c2);
             vf[u] = f4(vr + 16 * u);
         }
     }
-    const int qstart = s.causal ? k0 : 0;  // causal needs n_q == n_kv
-    const int nqt = (s.n_q - qstart) / FT;
+    const int shift = RAG ? s.n_kv - s.n_q : 0;
+    const int qstart = s.causal ? max(0, k0 - shift) : 0;  // (without RAG causal needs n_q == n_kv)
+    const int nqt = RAG ? (s.n_q - qstart + FT - 1) / FT : (s.n_q - qstart) / FT;
     const int niter = hpk * nqt;
     auto tile_of = [&](int it, int &h, int &q0) {
         h = kvh * hpk + it / nqt;
@@ -234,9 +262,19 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
         int h, q0;
         tile_of(it, h, q0);
         const long row0 = (long)b * s.n_q + q0;
-        tq.load(Q + row0 * p.ldq + h * HD, p.ldq, tid);
-        tdo.load(dO + row0 * p.lddo + h * HD, p.lddo, tid);
-        if (tid < 2 * FT) stat = (tid < FT ? p.lse : p.d)[(row0 + tid % FT) * s.n_heads + h];
+        if constexpr (RAG) {
+            tq.load(Q + row0 * p.ldq + h * HD, p.ldq, tid, s.n_q - q0);
+            tdo.load(dO + row0 * p.lddo + h * HD, p.lddo, tid, s.n_q - q0);
+            if (tid < 2 * FT) {
+                stat = tid < FT ? INFINITY : 0.f;  // P = 0 past the end, and where LSE is -inf
+                if (tid % FT < s.n_q - q0) stat = (tid < FT ? p.lse : p.d)[(row0 + tid % FT) * s.n_heads + h];
+                if (tid < FT && stat == -INFINITY) stat = INFINITY;
+            }
+        } else {
+            tq.load(Q + row0 * p.ldq + h * HD, p.ldq, tid);
+            tdo.load(dO + row0 * p.lddo + h * HD, p.lddo, tid);
+            if (tid < 2 * FT) stat = (tid < FT ? p.lse : p.d)[(row0 + tid % FT) * s.n_heads + h];
+        }
     };
     auto store = [&](int buf) {
         tq.store(Qs[buf], tid);
@@ -264,7 +302,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
 #pragma unroll
         for (int qs = 0; qs < 2; ++qs) {
             sa[qs] = da[qs] = f32x4{0, 0, 0, 0};
-            live[qs] = !s.causal || kw <= q0 + 16 * qs + 15;  // wave-uniform
+            live[qs] = !s.causal || kw <= q0 + 16 * qs + 15 + shift;  // wave-uniform
             if (live[qs]) {
                 const float *qr = Ql + (16 * qs + c) * P + 4 * g;
                 const float *orr = Ol + (16 * qs + c) * P + 4 * g;
@@ -282,9 +320,10 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
             for (int r = 0; r < 4; ++r) {
                 const int qr = 16 * qs + 4 * g + r;
                 float pv = __builtin_amdgcn_exp2f(sa[qs][r] - Ls[buf][qr]);
-                if (s.causal && ki > q0 + qr) pv = 0.f;
+                const bool past = RAG && q0 + qr >= s.n_q;  // a zero row (against an infinite K or V: NaN)
+                if ((s.causal && ki > q0 + qr + shift) || past) pv = 0.f;
                 sa[qs][r] = pv;
-                da[qs][r] = pv * (da[qs][r] - Dl[buf][qr]);
+                da[qs][r] = past ? 0.f : pv * (da[qs][r] - Dl[buf][qr]);
             }
         // dV^T += dO^T P, dK^T += Q^T dS: step (qs, e) is query q0 + 16 qs + 4 g + e
 #pragma unroll
@@ -303,6 +342,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
         if (it + 1 < niter) store(buf ^ 1);
         __syncthreads();
     }
+    if (RAG && ki >= s.n_kv) return;
     float *dkr = p.dk + ((long)b * s.n_kv + ki) * p.lddk + kvh * HD + 4 * g;
     float *dvr = p.dv + ((long)b * s.n_kv + ki) * p.lddv + kvh * HD + 4 * g;
     const float sc = s.inv_sqrt_dim;
@@ -335,13 +375,13 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
 // ── dQ: block = 64 queries of one (sequence, head) ──────────────────────
 // QKE: dQ leaves through RoPE^T and the Q-RMSNorm backward (p.qk), each block
 // writing its q-gain partial to p.qk.pq[block].
-template <int HD, bool QKE>
+template <int HD, bool QKE, bool RAG = false>
 __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs p, bool zz) {
-    static_assert(!QKE || HD == 128, "the fused q/k epilogue takes 128-wide head rows");
+    static_assert(!QKE || (HD == 128 && !RAG), "the fused q/k epilogue takes 128-wide head rows");
     constexpr int P = HD + 4, NU = HD / 16;
     __shared__ __attribute__((aligned(16))) float Ks[2][FT * P], Vs[2][FT * P];
     const int h = blockIdx.x % s.n_heads, b = blockIdx.x / s.n_heads;
-    const int nqb = s.n_q / 64;
+    const int nqb = (s.n_q + 63) / 64;
     const int y = (int)blockIdx.y, qb = s.causal ? nqb - 1 - (zz ? zigzag(y, nqb) : y) : y;
     const int tid = threadIdx.x, lane = tid % 64, g = lane / 16, c = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -350,24 +390,36 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
     const float c2 = s.inv_sqrt_dim * F_LOG2E;
     const float *Q = (const float *)p.q, *K = (const float *)p.k, *V = (const float *)p.v,
                 *dO = (const float *)p.dout;
+    const int ql = RAG ? min(qi, s.n_q - 1) : qi;  // (rows past the end are not stored)
     float4 qf[NU], of[NU];  // B of S^T = K Q^T and dP^T = V dO^T
     {
-        const float *qr = Q + ((long)b * s.n_q + qi) * p.ldq + h * HD + 4 * g;
-        const float *orr = dO + ((long)b * s.n_q + qi) * p.lddo + h * HD + 4 * g;
+        const float *qr = Q + ((long)b * s.n_q + ql) * p.ldq + h * HD + 4 * g;
+        const float *orr = dO + ((long)b * s.n_q + ql) * p.lddo + h * HD + 4 * g;
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
             qf[u] = f4_scale(f4(qr + 16 * u), c2);
             of[u] = f4(orr + 16 * u);
         }
     }
-    const float l2 = p.lse[((long)b * s.n_q + qi) * s.n_heads + h] * F_LOG2E;
-    const float dd = p.d[((long)b * s.n_q + qi) * s.n_heads + h];
-    const int nkt = s.causal ? (q0 + 64) / FT : s.n_kv / FT;
+    float l2 = p.lse[((long)b * s.n_q + ql) * s.n_heads + h] * F_LOG2E;
+    if (RAG && l2 == -INFINITY) l2 = INFINITY;  // no gradient: P = 0
+    const float dd = p.d[((long)b * s.n_q + ql) * s.n_heads + h];
+    const int shift = RAG ? s.n_kv - s.n_q : 0;
+    const int nkt = RAG ? ((s.causal ? min(s.n_kv, q0 + 64 + shift) : s.n_kv) + FT - 1) / FT
+                        : s.causal ? (q0 + 64) / FT : s.n_kv / FT;
     const float *kb = K + (long)b * s.n_kv * p.ldk + kvh * HD;
     const float *vb = V + (long)b * s.n_kv * p.ldv + kvh * HD;
     Tile<HD> tk, tv;
-    tk.load(kb, p.ldk, tid);
-    tv.load(vb, p.ldv, tid);
+    auto load = [&](int it) {
+        if constexpr (RAG) {
+            tk.load(kb + (long)it * FT * p.ldk, p.ldk, tid, s.n_kv - it * FT);
+            tv.load(vb + (long)it * FT * p.ldv, p.ldv, tid, s.n_kv - it * FT);
+        } else {
+            tk.load(kb + (long)it * FT * p.ldk, p.ldk, tid);
+            tv.load(vb + (long)it * FT * p.ldv, p.ldv, tid);
+        }
+    };
+    load(0);
     tk.store(Ks[0], tid);
     tv.store(Vs[0], tid);
     __syncthreads();
@@ -376,10 +428,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
     for (int j = 0; j < NU; ++j) dqt[j] = f32x4{0, 0, 0, 0};
     for (int it = 0; it < nkt; ++it) {
         const int buf = it & 1;
-        if (it + 1 < nkt) {
-            tk.load(kb + (long)(it + 1) * FT * p.ldk, p.ldk, tid);
-            tv.load(vb + (long)(it + 1) * FT * p.ldv, p.ldv, tid);
-        }
+        if (it + 1 < nkt) load(it + 1);
         const float *Kl = Ks[buf], *Vl = Vs[buf];
         const int kt0 = it * FT;
         f32x4 sa[2], da[2];  // S^T / dP^T[kt0 + 16 ks + 4 g + r][qi]
@@ -387,7 +436,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             sa[ks] = da[ks] = f32x4{0, 0, 0, 0};
-            live[ks] = !s.causal || kt0 + 16 * ks <= qw + 15;  // wave-uniform
+            live[ks] = !s.causal || kt0 + 16 * ks <= qw + 15 + shift;  // wave-uniform
             if (live[ks]) {
                 const float *kr = Kl + (16 * ks + c) * P + 4 * g;
                 const float *vr = Vl + (16 * ks + c) * P + 4 * g;
@@ -403,8 +452,10 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 float pv = __builtin_amdgcn_exp2f(sa[ks][r] - l2);
-                if (s.causal && kt0 + 16 * ks + 4 * g + r > qi) pv = 0.f;
-                da[ks][r] = pv * (da[ks][r] - dd);  // dS^T
+                const int kk = kt0 + 16 * ks + 4 * g + r;
+                const bool past = RAG && kk >= s.n_kv;
+                if (s.causal && kk > qi + shift) pv = 0.f;
+                da[ks][r] = past ? 0.f : pv * (da[ks][r] - dd);  // dS^T
             }
         // dQ^T += K^T dS^T: step (ks, e) is key kt0 + 16 ks + 4 g + e
 #pragma unroll
@@ -422,6 +473,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
         }
         __syncthreads();
     }
+    if (RAG && qi >= s.n_q) return;
     float *dqr = p.dq + ((long)b * s.n_q + qi) * p.lddq + h * HD + 4 * g;
     const float sc = s.inv_sqrt_dim;
     if constexpr (QKE) {
@@ -450,11 +502,16 @@ bool al16(const void *x) { return ((uintptr_t)x & 15) == 0; }
 
 }  // namespace
 
-// Shapes the fp32 tile kernels take: head_dim 64 or 128, whole 64-row tiles,
-// a causal mask only with n_q == n_kv, rows 16-byte aligned.
+// Shapes the fp32 tile kernels take: head_dim 64 or 128, rows 16-byte aligned, whole
+// 64-row tiles and a causal mask only with n_q == n_kv, or any lengths where the
+// caller allows the ragged form (s.ragged: the standalone entry points; a training
+// step of ragged sequences keeps the per-row kernels' summation order).
+static bool whole_tiles(const AttnShape &s) {
+    return s.n_q % 64 == 0 && s.n_kv % 64 == 0 && (!s.causal || s.n_q == s.n_kv);
+}
 bool fa_f32m_ok(const AttnShape &s) {
     return (s.head_dim == 64 || s.head_dim == 128) && s.n_q > 0 && s.n_kv > 0 &&
-           s.n_q % 64 == 0 && s.n_kv % 64 == 0 && (!s.causal || s.n_q == s.n_kv) &&
+           (whole_tiles(s) || (s.ragged && (!s.causal || s.n_q <= s.n_kv))) &&
            s.n_kv_heads > 0 && s.n_heads % s.n_kv_heads == 0;
 }
 
@@ -463,12 +520,13 @@ bool fa_f32m_fwd(const AttnShape &s, const float *q, long ldq, const float *k, l
     if (!fa_f32m_ok(s) || !al16(q) || !al16(k) || !al16(v) || !al16(o) || ldq % 4 || ldk % 4 ||
         ldv % 4 || ldo % 4)
         return false;
-    const dim3 grid(s.n_heads * s.n_batch, s.n_q / 64);
+    const dim3 grid(s.n_heads * s.n_batch, (s.n_q + 63) / 64);
     const bool zz = fits_two_per_cu((long)grid.x * grid.y);
-    if (s.head_dim == 128)
-        hipLaunchKernelGGL(fa_fwd_f32m_k<128>, grid, dim3(FNT), 0, st, s, q, ldq, k, ldk, v, ldv, o, ldo, lse, zz);
-    else
-        hipLaunchKernelGGL(fa_fwd_f32m_k<64>, grid, dim3(FNT), 0, st, s, q, ldq, k, ldk, v, ldv, o, ldo, lse, zz);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(FNT), 0, st, s, q, ldq, k, ldk, v, ldv, o, ldo, lse, zz);
+    };
+    if (whole_tiles(s)) s.head_dim == 128 ? go(fa_fwd_f32m_k<128>) : go(fa_fwd_f32m_k<64>);
+    else s.head_dim == 128 ? go(fa_fwd_f32m_k<128, true>) : go(fa_fwd_f32m_k<64, true>);
     return true;
 }
 
@@ -481,22 +539,24 @@ bool fa_f32m_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     if (!fa_f32m_ok(s) || !ptrs_ok(p) || !al16(p.dk) || !al16(p.dv) || p.lddk % 4 || p.lddv % 4)
         return false;
     if (p.qk_fp32 && !fa_f32m_qk_ok(s, p)) return false;
-    const dim3 grid(s.n_kv_heads * s.n_batch, s.n_kv / 64);
+    const dim3 grid(s.n_kv_heads * s.n_batch, (s.n_kv + 63) / 64);
     const bool zz = fits_two_per_cu((long)grid.x * grid.y);
-    if (p.qk_fp32) hipLaunchKernelGGL((fa_bwd_dkv_f32m_k<128, true>), grid, dim3(FNT), 0, st, s, p, zz);
-    else if (s.head_dim == 128) hipLaunchKernelGGL((fa_bwd_dkv_f32m_k<128, false>), grid, dim3(FNT), 0, st, s, p, zz);
-    else hipLaunchKernelGGL((fa_bwd_dkv_f32m_k<64, false>), grid, dim3(FNT), 0, st, s, p, zz);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(FNT), 0, st, s, p, zz); };
+    if (p.qk_fp32) go(fa_bwd_dkv_f32m_k<128, true>);
+    else if (whole_tiles(s)) s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false>) : go(fa_bwd_dkv_f32m_k<64, false>);
+    else s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false, true>) : go(fa_bwd_dkv_f32m_k<64, false, true>);
     return true;
 }
 
 bool fa_f32m_dq(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     if (!fa_f32m_ok(s) || !ptrs_ok(p) || !al16(p.dq) || p.lddq % 4) return false;
     if (p.qk_fp32 && !fa_f32m_qk_ok(s, p)) return false;
-    const dim3 grid(s.n_heads * s.n_batch, s.n_q / 64);
+    const dim3 grid(s.n_heads * s.n_batch, (s.n_q + 63) / 64);
     const bool zz = fits_two_per_cu((long)grid.x * grid.y);
-    if (p.qk_fp32) hipLaunchKernelGGL((fa_bwd_dq_f32m_k<128, true>), grid, dim3(FNT), 0, st, s, p, zz);
-    else if (s.head_dim == 128) hipLaunchKernelGGL((fa_bwd_dq_f32m_k<128, false>), grid, dim3(FNT), 0, st, s, p, zz);
-    else hipLaunchKernelGGL((fa_bwd_dq_f32m_k<64, false>), grid, dim3(FNT), 0, st, s, p, zz);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(FNT), 0, st, s, p, zz); };
+    if (p.qk_fp32) go(fa_bwd_dq_f32m_k<128, true>);
+    else if (whole_tiles(s)) s.head_dim == 128 ? go(fa_bwd_dq_f32m_k<128, false>) : go(fa_bwd_dq_f32m_k<64, false>);
+    else s.head_dim == 128 ? go(fa_bwd_dq_f32m_k<128, false, true>) : go(fa_bwd_dq_f32m_k<64, false, true>);
     return true;
 }
 
@@ -505,7 +565,7 @@ bool fa_f32m_dq(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
 // and gains, and every output pointer the tile kernels need.
 bool fa_f32m_qk_ok(const AttnShape &s, const AttnPtrs &p) {
     const QkEpi &e = p.qk;
-    return fa_f32m_ok(s) && s.head_dim == 128 && ptrs_ok(p) && al16(p.dq) && al16(p.dk) &&
+    return fa_f32m_ok(s) && whole_tiles(s) && s.head_dim == 128 && ptrs_ok(p) && al16(p.dq) && al16(p.dk) &&
            al16(p.dv) && p.lddq % 4 == 0 && p.lddk % 4 == 0 && p.lddv % 4 == 0 && e.x && al16(e.x) &&
            e.ldx % 4 == 0 && (e.rot == 0 || (e.rot == 128 && e.rope && al16(e.rope))) &&
            (!e.gq || (al16(e.gq) && e.pq)) && (!e.gk || (al16(e.gk) && e.pk));

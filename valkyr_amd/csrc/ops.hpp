@@ -316,6 +316,7 @@ struct AttnShape {
     int n_batch, n_q, n_kv, n_heads, n_kv_heads, head_dim;
     int causal;
     float inv_sqrt_dim;
+    int ragged = 0;  // fp32: the tile kernels also for lengths that are not whole tiles
 };
 // Fused q/k gradient epilogue of the recompute attention backward: dQ, dK
 // and dV leave the kernels as bf16 rows of one [T, (H + 2 Hkv) hd] matrix
