@@ -879,6 +879,16 @@ def test_flash_attention_bf16_mfma(case):
     _check_from_o(p, qb, kb, vb, o, dob16, lse_r, dO.size, ws)
 
 
+@pytest.mark.parametrize("case", [  # (n, H, Hkv, hd, causal, B)
+    (1, 2, 1, 128, True, 2), (33, 3, 1, 128, True, 2), (129, 4, 4, 128, True, 1),
+    (257, 8, 2, 128, True, 1), (130, 4, 4, 128, False, 2), (95, 5, 5, 128, False, 1)])
+def test_flash_attention_bf16_ragged_recompute(case):
+    """The recompute backward's ragged form (a row past a 32- or 128-row tile, one row,
+    odd head groups whose wave groups share the query tiles), held to the bounds of
+    test_flash_attention_bf16_mfma."""
+    test_flash_attention_bf16_mfma(case)
+
+
 # n_q != n_kv in bf16 (the reference's causal limit k <= q + (n_kv - n_q),
 # fa_bw_dq.comp / flash_attn.zig:66-68 causalKeyLimit): more keys than queries
 # under the causal mask, and more queries than keys without it; GQA 2:1 and

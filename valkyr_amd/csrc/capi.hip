@@ -351,6 +351,18 @@ vkh_status vkh_fa_backward_from_o(const vkh_attn_params *p, const void *q, const
         if (e != hipSuccess) return hip_fail(e, "fa_backward_from_o");
         return VKH_OK;
     }
+    if (!fa_bw_fused_ok(s)) {
+        AttnPtrs a = attn_ptrs(p, q, k, v, dout_bf16, lse, d);
+        a.dq = dq;
+        a.dk = dk;
+        a.dv = dv;
+        a.o16 = o_bf16;
+        a.ldo16 = (long)p->n_heads * p->head_dim;
+        if (fa_bw_ragged(s, a, S(stream))) {
+            VKH_HIP(hipGetLastError());
+            return VKH_OK;
+        }
+    }
     VKH_TRY(vkh_fa_bw_d_bf16(p, o_bf16, dout_bf16, d, stream));
     return vkh_fa_backward(p, q, k, v, dout_bf16, lse, d, dq, dk, dv, workspace, stream);
 }

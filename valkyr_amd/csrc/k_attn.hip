@@ -1125,7 +1125,13 @@ static_assert(2 * STREAM + BN * HD * 2 <= LDS, "tile streams and V slices exceed
 // (fp32, dK scaled) into its own slice of p.split_ws; fa_dkv_combine_k adds the
 // two slices in part order and runs the epilogue.  That doubles the grid where
 // the (sequence, KV head, key block) grid alone leaves CUs idle.
-template <int NWV, bool QKE, int NH = 0, int PARTS = 1>
+// RAG: any n_q and n_kv (equal under a causal mask).  Rows past the end arrive as
+// zeros by the buffer range check (K's registers: a clamped row), their P and dS are
+// set to zero, and keys past the end are not stored.  An odd head group (hpk odd: no
+// two equal head groups) has the two wave groups take alternate query tiles of every
+// head instead, the last pair padded by a tile past the end.  Against the per-row-
+// staged general kernel (n = 1001, 32 / 8 heads, 2 sequences): 349 -> 122 us.
+template <int NWV, bool QKE, int NH = 0, int PARTS = 1, bool RAG = false>
 __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPtrs p) {
     using namespace dkv4;
     constexpr int NS = NWV / 2;                 // key slices per head group
@@ -1139,10 +1145,12 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
     __shared__ __attribute__((aligned(16))) float Ls[2][NBUF][64], Dd[2][NBUF][64];
 
     const int kt = (int)blockIdx.y;
+    static_assert(!RAG || (!QKE && PARTS == 1 && NH == 0), "the ragged form has no fused epilogue or split");
     static_assert(PARTS == 1 || !QKE, "a split launch leaves the epilogue to the combine kernel");
     const int kvh = blockIdx.x % s.n_kv_heads, b = blockIdx.x / s.n_kv_heads;
     const int hpk = s.n_heads / s.n_kv_heads;
-    const int nh = (NH ? NH : hpk / 2) / PARTS;  // this block's heads per head group
+    const bool alt = RAG && (hpk & 1);  // wave groups split the query tiles, not the heads
+    const int nh = alt ? hpk : (NH ? NH : hpk / 2) / PARTS;  // this block's heads per head group
     const int zp = PARTS > 1 ? (int)blockIdx.z : 0;  // this block's half of the heads
     const int tid = threadIdx.x, lane = tid % 64, g = lane / 16, c16 = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -1162,7 +1170,14 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int ds = 0; ds < DS; ++ds) kr[ks][ds] = ld_frag(kb + 16L * ks * p.ldk + 32 * ds);
+            for (int ds = 0; ds < DS; ++ds) {
+                if constexpr (RAG) {
+                    const long past = max(0, kw0 + c16 + 16 * ks - (s.n_kv - 1));
+                    kr[ks][ds] = ld_frag(kb + (16L * ks - past) * p.ldk + 32 * ds);
+                } else {
+                    kr[ks][ds] = ld_frag(kb + 16L * ks * p.ldk + 32 * ds);
+                }
+            }
     }
     // V of the slice (64 rows, swizzled like the tiles) by DMA from the group-0 wave
     char *vsl = smem + 2 * STREAM + sl * KW * HD * 2;
@@ -1186,8 +1201,8 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
 
     // causal: n_q == n_kv, so queries below k0 see none of the block's keys
     const int qstart = s.causal ? k0 : 0;
-    const int nqt = (s.n_q - qstart) / BM;
-    const int niter = nh * nqt;
+    const int nqt = RAG ? (s.n_q - qstart + BM - 1) / BM : (s.n_q - qstart) / BM;
+    const int niter = nh * (alt ? (nqt + 1) / 2 : nqt);
     char *strm = smem + hg * STREAM;
 
     // this wave's DMA share: slice 0 moves Q and lse, slice 1 dO and D
@@ -1199,6 +1214,11 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
     const sgpr4 rs = rsrc4((tdo ? p.d : p.lse) + (long)b * s.n_q * s.n_heads,
                            (unsigned)((long)s.n_q * s.n_heads * 4));
     auto tile_of = [&](int it, int &h, int &q0) {
+        if (alt) {
+            h = kvh * hpk + it % nh;
+            q0 = qstart + ((nqt + 1) / 2 * 2 - 1 - 2 * (it / nh) - hg) * BM;
+            return;
+        }
         h = kvh * hpk + hg + 2 * (zp * nh + it % nh);
         q0 = qstart + (nqt - 1 - it / nh) * BM;
     };
@@ -1314,6 +1334,15 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
                     for (int r = 0; r < 4; ++r)
                         if (16 * ks - r > lim[qs]) sc[qs][ks][r] = 0.f;
         }
+        if (RAG && q0 + BM > s.n_q) {  // query rows past the end
+#pragma unroll
+            for (int qs = 0; qs < QS; ++qs)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (q0 + 16 * qs + 4 * g + r >= s.n_q) sc[qs][ks][r] = dp[qs][ks][r] = 0.f;
+        }
         // dV^T += dO^T P, with dS = P (dP - D) of tile (i / 4, i % 4) (dp holds dP - D)
         {
             bf16x8 pb[KS];
@@ -1377,6 +1406,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
     auto keep = [&](const f32x4 (&a)[DSUB][KS], float *base, long ld, float sc_) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
+            if (RAG && kw0 + 16 * ks + c16 >= s.n_kv) continue;
             float *out = base + ((long)b * s.n_kv + kw0 + 16 * ks + c16) * ld + kvh * HD;
 #pragma unroll
             for (int i = 0; i < DSUB; ++i) {
@@ -2160,11 +2190,81 @@ hipError_t fa_bw_d_bf16(const AttnShape &s, const bf16 *o, long ldo, const bf16 
     return hipGetLastError();
 }
 
+// The dK/dV recompute kernel with the head-group size as a constant where it
+// is one of the common ones.
+template <int W, bool QKE>
+void launch_dkv4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
+    const int nh = s.n_heads / s.n_kv_heads / 2;
+    if (p.split_ws && fa_bw_v4_split(s)) {
+        // two blocks per (sequence, KV head, key block), then their sum and the epilogue
+        const dim3 gkv(s.n_kv_heads * s.n_batch, s.n_kv / dkv4::BN, 2);
+        if (nh == 2) hipLaunchKernelGGL((fa_bwd_dkv4_k<W, false, 2, 2>), gkv, dim3(W * 64), 0, st, s, p);
+        else hipLaunchKernelGGL((fa_bwd_dkv4_k<W, false, 0, 2>), gkv, dim3(W * 64), 0, st, s, p);
+        const dim3 gc((unsigned)(((long)s.n_batch * s.n_kv + 63) / 64), s.n_kv_heads);
+        hipLaunchKernelGGL(fa_dkv_combine_k<QKE>, gc, dim3(256), 0, st, s, p);
+        return;
+    }
+    const dim3 gkv(s.n_kv_heads * s.n_batch, s.n_kv / dkv4::BN);
+    if (nh == 1) hipLaunchKernelGGL((fa_bwd_dkv4_k<W, QKE, 1>), gkv, dim3(W * 64), 0, st, s, p);
+    else if (nh == 2) hipLaunchKernelGGL((fa_bwd_dkv4_k<W, QKE, 2>), gkv, dim3(W * 64), 0, st, s, p);
+    else hipLaunchKernelGGL((fa_bwd_dkv4_k<W, QKE, 0>), gkv, dim3(W * 64), 0, st, s, p);
+}
+
+void launch_dkv4_ragged(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
+    const dim3 gkv(s.n_kv_heads * s.n_batch, (s.n_kv + dkv4::BN - 1) / dkv4::BN);
+    hipLaunchKernelGGL((fa_bwd_dkv4_k<8, false, 0, 1, true>), gkv, dim3(512), 0, st, s, p);
+}
+
+// dQ blocks of 256 queries, or of 128 where 256 would leave fewer blocks than
+// CUs: there a causal grid is also short of work at its end, since a block's
+// work grows with its last query (config 3, 4 x 512: 128 blocks of 256 rows,
+// the later block of each sequence twice the earlier); with 256-query blocks
+// filling the chip, 128 loses (config 2: 0.268 against 0.250 ms per call)
+int dq4_bq(const AttnShape &s) {
+    const long b256 = (long)s.n_heads * s.n_batch * ((s.n_q + 255) / 256);
+    return b256 < 256 ? 128 : 256;
+}
+template <bool WITH_D, bool QKE>
+void launch_dq4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
+    constexpr int W = 8;
+    const int bq = dq4_bq(s);
+    const dim3 gq(s.n_heads * s.n_batch, (s.n_q + bq - 1) / bq);
+    if (bq == 128)
+        hipLaunchKernelGGL((fa_bwd_dq4_k<W, WITH_D, QKE, 128>), gq, dim3(W * 64), 0, st, s, p);
+    else
+        hipLaunchKernelGGL((fa_bwd_dq4_k<W, WITH_D, QKE, 256>), gq, dim3(W * 64), 0, st, s, p);
+}
+
+// The recompute kernels on lengths that are not whole tiles, or with an odd head
+// group: head_dim 128, n_q == n_kv under a causal mask, 16-byte aligned rows under
+// 2 GiB a sequence.
+static bool v4_ragged_ok(const AttnShape &s, const AttnPtrs &p) {
+    auto al = [](const void *x, long ld) { return ((uintptr_t)x & 15) == 0 && ld % 8 == 0; };
+    return p.dt == DType::BF16 && s.head_dim == 128 && (!s.causal || s.n_q == s.n_kv) && s.n_kv > 0 &&
+           al(p.q, p.ldq) && al(p.k, p.ldk) && al(p.v, p.ldv) && al(p.dout, p.lddo) &&
+           (!p.o16 || al(p.o16, p.ldo16)) && (long)s.n_q * std::max(p.ldq, p.lddo) * 2 < (1l << 30) &&
+           (long)s.n_kv * std::max(p.ldk, p.ldv) * 2 < (1l << 30);
+}
+static bool al_out(const float *x, long ld) { return ((uintptr_t)x & 15) == 0 && ld % 4 == 0; }
+
+bool fa_bw_ragged(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
+    if (!p.o16 || !v4_ragged_ok(s, p) || !al_out(p.dq, p.lddq) || !al_out(p.dk, p.lddk) ||
+        !al_out(p.dv, p.lddv))
+        return false;
+    launch_dq4<true, false>(s, p, st);  // forms D
+    launch_dkv4_ragged(s, p, st);
+    return true;
+}
+
 hipError_t fa_bw_dq(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     if (s.n_batch <= 0 || s.n_q <= 0) return hipSuccess;
     if (s.n_kv_heads <= 0 || s.n_heads % s.n_kv_heads) return hipErrorInvalidValue;
     if (p.dt == DType::BF16) {
         if (!bf16_ok(s)) return hipErrorInvalidValue;
+        if (v4_ragged_ok(s, p) && al_out(p.dq, p.lddq)) {
+            launch_dq4<false, false>(s, p, st);
+            return hipGetLastError();
+        }
         dim3 grid(s.n_heads * s.n_batch, (s.n_q + 127) / 128);
         if (s.head_dim == 128)
             hipLaunchKernelGGL(fa_bwd_dq_bf16_k<128>, grid, dim3(NT), 0, st, s, p);
@@ -2203,46 +2303,6 @@ bool fa_bw_v4_ok(const AttnShape &s) {
 // 0.327 ms); below that the two-kernel dS path keeps more blocks in flight.
 bool fa_bw_v4_preferred(const AttnShape &s) {
     return fa_bw_v4_ok(s) && (long)s.n_batch * s.n_kv_heads * (s.n_kv / 128) >= 128;
-}
-
-// The dK/dV recompute kernel with the head-group size as a constant where it
-// is one of the common ones.
-template <int W, bool QKE>
-void launch_dkv4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
-    const int nh = s.n_heads / s.n_kv_heads / 2;
-    if (p.split_ws && fa_bw_v4_split(s)) {
-        // two blocks per (sequence, KV head, key block), then their sum and the epilogue
-        const dim3 gkv(s.n_kv_heads * s.n_batch, s.n_kv / dkv4::BN, 2);
-        if (nh == 2) hipLaunchKernelGGL((fa_bwd_dkv4_k<W, false, 2, 2>), gkv, dim3(W * 64), 0, st, s, p);
-        else hipLaunchKernelGGL((fa_bwd_dkv4_k<W, false, 0, 2>), gkv, dim3(W * 64), 0, st, s, p);
-        const dim3 gc((unsigned)(((long)s.n_batch * s.n_kv + 63) / 64), s.n_kv_heads);
-        hipLaunchKernelGGL(fa_dkv_combine_k<QKE>, gc, dim3(256), 0, st, s, p);
-        return;
-    }
-    const dim3 gkv(s.n_kv_heads * s.n_batch, s.n_kv / dkv4::BN);
-    if (nh == 1) hipLaunchKernelGGL((fa_bwd_dkv4_k<W, QKE, 1>), gkv, dim3(W * 64), 0, st, s, p);
-    else if (nh == 2) hipLaunchKernelGGL((fa_bwd_dkv4_k<W, QKE, 2>), gkv, dim3(W * 64), 0, st, s, p);
-    else hipLaunchKernelGGL((fa_bwd_dkv4_k<W, QKE, 0>), gkv, dim3(W * 64), 0, st, s, p);
-}
-
-// dQ blocks of 256 queries, or of 128 where 256 would leave fewer blocks than
-// CUs: there a causal grid is also short of work at its end, since a block's
-// work grows with its last query (config 3, 4 x 512: 128 blocks of 256 rows,
-// the later block of each sequence twice the earlier); with 256-query blocks
-// filling the chip, 128 loses (config 2: 0.268 against 0.250 ms per call)
-int dq4_bq(const AttnShape &s) {
-    const long b256 = (long)s.n_heads * s.n_batch * ((s.n_q + 255) / 256);
-    return b256 < 256 ? 128 : 256;
-}
-template <bool WITH_D, bool QKE>
-void launch_dq4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
-    constexpr int W = 8;
-    const int bq = dq4_bq(s);
-    const dim3 gq(s.n_heads * s.n_batch, (s.n_q + bq - 1) / bq);
-    if (bq == 128)
-        hipLaunchKernelGGL((fa_bwd_dq4_k<W, WITH_D, QKE, 128>), gq, dim3(W * 64), 0, st, s, p);
-    else
-        hipLaunchKernelGGL((fa_bwd_dq4_k<W, WITH_D, QKE, 256>), gq, dim3(W * 64), 0, st, s, p);
 }
 
 // One of the two recompute kernels alone (D already in p.d): which = 0 the
@@ -2353,6 +2413,10 @@ hipError_t fa_bw_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     if (s.n_kv_heads <= 0 || s.n_heads % s.n_kv_heads) return hipErrorInvalidValue;
     if (p.dt == DType::BF16) {
         if (!bf16_ok(s)) return hipErrorInvalidValue;
+        if (v4_ragged_ok(s, p) && al_out(p.dk, p.lddk) && al_out(p.dv, p.lddv)) {
+            launch_dkv4_ragged(s, p, st);
+            return hipGetLastError();
+        }
         dim3 grid(s.n_kv_heads * s.n_batch, (s.n_kv + 127) / 128);
         if (s.head_dim == 128)
             hipLaunchKernelGGL(fa_bwd_dkv_bf16_k<128>, grid, dim3(NT), 0, st, s, p);

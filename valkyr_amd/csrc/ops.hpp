@@ -383,6 +383,10 @@ hipError_t fa_bw_d_bf16(const AttnShape &s, const bf16 *o, long ldo, const bf16 
                         float *d, hipStream_t st);
 hipError_t fa_bw_dq(const AttnShape &s, const AttnPtrs &p, hipStream_t st);
 hipError_t fa_bw_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st);
+// The whole bf16 backward from bf16 O (p.o16; D is written) on shapes the fused form
+// does not take, with the recompute kernels' ragged form; false, launching nothing,
+// where they do not apply (fa_bw_dkv and fa_bw_dq pick it by the same rule).
+bool fa_bw_ragged(const AttnShape &s, const AttnPtrs &p, hipStream_t st);
 // Fused bf16 backward.  Requires fa_bw_fused_ok(s) (bf16 head_dim 64/128, n_q
 // and n_kv multiples of 64, self-attention when causal).  v4 (requires
 // fa_bw_v4_ok: head_dim 128, even GQA group, n_kv % 128 == 0): dK/dV and dQ
