@@ -768,7 +768,8 @@ FA_BF16_CASES = [  # (n, H, Hkv, hd, causal, B)
 @pytest.mark.parametrize("case", [  # (n_q, n_kv, H, Hkv, hd, causal, B)
     (1, 1, 4, 2, 64, True, 2), (100, 100, 16, 8, 128, True, 1), (65, 65, 8, 2, 64, True, 2),
     (33, 97, 4, 2, 128, True, 1), (64, 129, 4, 4, 128, True, 2), (31, 200, 4, 4, 64, False, 2),
-    (200, 31, 4, 2, 128, False, 1), (257, 257, 4, 1, 128, True, 1)])
+    (200, 31, 4, 2, 128, False, 1), (257, 257, 4, 1, 128, True, 1),
+    (320, 320, 8, 2, 64, True, 1), (100, 300, 4, 2, 64, True, 1)])
 def test_flash_attention_fp32_ragged_lengths(case):
     """The fp32 matrix-core kernels on lengths that are not whole tiles (one row, a row
     past a tile, causal with more keys than queries, either side longer without a mask),
@@ -881,11 +882,13 @@ def test_flash_attention_bf16_mfma(case):
 
 @pytest.mark.parametrize("case", [  # (n, H, Hkv, hd, causal, B)
     (1, 2, 1, 128, True, 2), (33, 3, 1, 128, True, 2), (129, 4, 4, 128, True, 1),
-    (257, 8, 2, 128, True, 1), (130, 4, 4, 128, False, 2), (95, 5, 5, 128, False, 1)])
+    (257, 8, 2, 128, True, 1), (130, 4, 4, 128, False, 2), (95, 5, 5, 128, False, 1),
+    (1, 4, 2, 64, True, 1), (161, 6, 2, 64, True, 2), (256, 4, 1, 64, False, 1),
+    (384, 8, 2, 128, True, 1), (640, 2, 2, 64, True, 1)])
 def test_flash_attention_bf16_ragged_recompute(case):
-    """The recompute backward's ragged form (a row past a 32- or 128-row tile, one row,
-    odd head groups whose wave groups share the query tiles), held to the bounds of
-    test_flash_attention_bf16_mfma."""
+    """The recompute backward's general form (a row past a 32- or 128-row tile, one row,
+    odd head groups whose wave groups share the query tiles, 64-wide heads, key blocks
+    split between blocks), held to the bounds of test_flash_attention_bf16_mfma."""
     test_flash_attention_bf16_mfma(case)
 
 

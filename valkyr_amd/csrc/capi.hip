@@ -71,6 +71,7 @@ static vkh_status rope_table_cached(int seq_len, int rot, float theta, const flo
 // stream created after another was destroyed never inherits its buffer.  A
 // buffer is replaced only after its stream has drained; at most kMaxStreams
 // buffers are kept, and making room for another waits for the whole device.
+constexpr size_t kLeaseMax = 256ull << 20;  // the most that a call keeps here
 class ScratchLease {
   public:
     vkh_status acquire(size_t bytes, hipStream_t st, void **out) {
@@ -280,6 +281,25 @@ vkh_status vkh_fa_bw_dq(const vkh_attn_params *p, const void *q, const void *k, 
     return VKH_OK;
 }
 
+// Scratch of a split dK / dV launch, where the grid asks for one (not under capture).
+static bool capturing(hipStream_t st);
+static vkh_status attn_parts(const AttnShape &s, AttnPtrs &a, ScratchLease &lease, hipStream_t st) {
+    const int parts = fa_bw_parts(s, a.dt);
+    const size_t b = fa_bw_parts_ws_bytes(s, parts);
+    if (!b || b > kLeaseMax || capturing(st)) return VKH_OK;
+    void *w = nullptr;
+    VKH_TRY(lease.acquire(b, st, &w));
+    a.split_ws = (float *)w;
+    a.split_parts = parts;
+    return VKH_OK;
+}
+// bf16 shapes that the recompute kernels' general form takes: all that the fused form's
+// own recompute kernels do not, and those whose dK / dV grid is split.  (4 x 2048
+// tokens, 16 / 8 heads of 64: 289 us on the dS workspace and dQ GEMM, 174 here.)
+static bool attn_general(const AttnShape &s, const AttnPtrs &a) {
+    return a.dt == DType::BF16 && (a.split_ws || !fa_bw_v4_ok(s)) && fa_bw_ragged_ok(s, a);
+}
+
 vkh_status vkh_fa_bw_dkv(const vkh_attn_params *p, const void *q, const void *k, const void *v,
                          const void *dout, const float *lse, const float *d, float *dk,
                          float *dv, vkh_stream stream) {
@@ -288,7 +308,10 @@ vkh_status vkh_fa_bw_dkv(const vkh_attn_params *p, const void *q, const void *k,
     AttnPtrs a = attn_ptrs(p, q, k, v, dout, lse, d);
     a.dk = dk;
     a.dv = dv;
-    VKH_HIP(fa_bw_dkv(attn_shape(p), a, S(stream)));
+    const AttnShape s = attn_shape(p);
+    ScratchLease lease;
+    VKH_TRY(attn_parts(s, a, lease, S(stream)));
+    VKH_HIP(fa_bw_dkv(s, a, S(stream)));
     return VKH_OK;
 }
 
@@ -309,7 +332,9 @@ vkh_status vkh_fa_backward(const vkh_attn_params *p, const void *q, const void *
     a.dv = dv;
     const AttnShape s = attn_shape(p);
     hipStream_t st = S(stream);
-    if (p->dtype != VKH_BF16 || !fa_bw_fused_ok(s)) {
+    ScratchLease lease;
+    VKH_TRY(attn_parts(s, a, lease, st));
+    if (p->dtype != VKH_BF16 || !fa_bw_fused_ok(s) || attn_general(s, a)) {
         VKH_HIP(fa_bw_dkv(s, a, st));
         VKH_HIP(fa_bw_dq(s, a, st));
         return VKH_OK;
@@ -340,28 +365,25 @@ vkh_status vkh_fa_backward_from_o(const vkh_attn_params *p, const void *q, const
     CHECK_ARG(q && k && v && o_bf16 && dout_bf16 && lse && d && dq && dk && dv, "null pointer");
     if (p->dtype != VKH_BF16) return fail(VKH_ERR_INVALID_ARGUMENT, "fa_backward_from_o takes bf16 operands");
     const AttnShape s = attn_shape(p);
-    if (fa_bw_fused_ok(s) && fa_bw_v4_ok(s)) {
-        AttnPtrs a = attn_ptrs(p, q, k, v, dout_bf16, lse, d);
-        a.dq = dq;
-        a.dk = dk;
-        a.dv = dv;
-        a.o16 = o_bf16;
-        a.ldo16 = (long)p->n_heads * p->head_dim;
-        const hipError_t e = fa_bw_fused(s, a, nullptr, true, S(stream));
-        if (e != hipSuccess) return hip_fail(e, "fa_backward_from_o");
-        return VKH_OK;
-    }
-    if (!fa_bw_fused_ok(s)) {
-        AttnPtrs a = attn_ptrs(p, q, k, v, dout_bf16, lse, d);
-        a.dq = dq;
-        a.dk = dk;
-        a.dv = dv;
-        a.o16 = o_bf16;
-        a.ldo16 = (long)p->n_heads * p->head_dim;
-        if (fa_bw_ragged(s, a, S(stream))) {
+    AttnPtrs a = attn_ptrs(p, q, k, v, dout_bf16, lse, d);
+    a.dq = dq;
+    a.dk = dk;
+    a.dv = dv;
+    a.o16 = o_bf16;
+    a.ldo16 = (long)p->n_heads * p->head_dim;
+    {
+        ScratchLease lease;
+        VKH_TRY(attn_parts(s, a, lease, S(stream)));
+        if (attn_general(s, a) && fa_bw_ragged(s, a, S(stream))) {
             VKH_HIP(hipGetLastError());
             return VKH_OK;
         }
+    }
+    a.split_ws = nullptr;
+    if (fa_bw_fused_ok(s) && fa_bw_v4_ok(s)) {
+        const hipError_t e = fa_bw_fused(s, a, nullptr, true, S(stream));
+        if (e != hipSuccess) return hip_fail(e, "fa_backward_from_o");
+        return VKH_OK;
     }
     VKH_TRY(vkh_fa_bw_d_bf16(p, o_bf16, dout_bf16, d, stream));
     return vkh_fa_backward(p, q, k, v, dout_bf16, lse, d, dq, dk, dv, workspace, stream);
@@ -371,7 +393,6 @@ vkh_status vkh_fa_backward_from_o(const vkh_attn_params *p, const void *q, const
 
 // Workspace for one call.  Up to kLeaseMax it is the stream's kept scratch; more
 // is allocated in stream order and freed after the call's work.
-constexpr size_t kLeaseMax = 256ull << 20;
 extern "C++" {
 template <class F>
 static vkh_status with_ws(size_t bytes, hipStream_t st, const char *what, F &&f) {

@@ -1131,12 +1131,21 @@ static_assert(2 * STREAM + BN * HD * 2 <= LDS, "tile streams and V slices exceed
 // two equal head groups) has the two wave groups take alternate query tiles of every
 // head instead, the last pair padded by a tile past the end.  Against the per-row-
 // staged general kernel (n = 1001, 32 / 8 heads, 2 sequences): 349 -> 122 us.
-template <int NWV, bool QKE, int NH = 0, int PARTS = 1, bool RAG = false>
+// RAG with p.split_parts > 1: that many blocks (blockIdx.z) take every split_parts-th
+// (head, query tile) step of a key block and write their raw sums to their slice of
+// p.split_ws ([part][dK, dV][rows][kvd]); fa_dkv_sum_k adds the slices in part order.
+// Short sequences and few KV heads leave most CUs without a key block: 1 x 1000
+// tokens, 16 / 4 heads are 32 blocks.
+// HDR = 64 (RAG only): 64-wide heads in the same 128-wide LDS rows, whose upper half is
+// never read; half the matrix work a step, the same schedule.
+template <int NWV, bool QKE, int NH = 0, int PARTS = 1, bool RAG = false, int HDR = 128>
 __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPtrs p) {
     using namespace dkv4;
     constexpr int NS = NWV / 2;                 // key slices per head group
     constexpr int KW = BN / NS, KS = KW / 16;   // keys per wave, 16-key sub-tiles
-    constexpr int XSLOT = DSUB * KS * 64 * 16;  // one wave's dK^T or dV^T
+    constexpr int DSR = HDR / 32, DSUBR = HDR / 16, NF = 2 * DSR;  // of the real head
+    static_assert(HDR == HD || (RAG && HDR == 64), "head width");
+    constexpr int XSLOT = DSUBR * KS * 64 * 16;  // one wave's dK^T or dV^T
     static_assert(NWV * XSLOT <= LDS, "exchange exceeds the LDS arena");
     constexpr int RP = BM / (NS / 2);           // Q or dO tile rows each wave moves
     using dkv3::frag_row;
@@ -1164,13 +1173,13 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
 
     // K and V of the slice as B operands: lane (g, c16) holds key 16 ks + c16,
     // d = 32 ds + 8 g .. + 7 (n_kv is a multiple of 128: no edge)
-    bf16x8 kr[KS][DS];
+    bf16x8 kr[KS][DSR];
     {
-        const bf16 *kb = (const bf16 *)p.k + ((long)b * s.n_kv + kw0 + c16) * p.ldk + kvh * HD + 8 * g;
+        const bf16 *kb = (const bf16 *)p.k + ((long)b * s.n_kv + kw0 + c16) * p.ldk + kvh * HDR + 8 * g;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int ds = 0; ds < DS; ++ds) {
+            for (int ds = 0; ds < DSR; ++ds) {
                 if constexpr (RAG) {
                     const long past = max(0, kw0 + c16 + 16 * ks - (s.n_kv - 1));
                     kr[ks][ds] = ld_frag(kb + (16L * ks - past) * p.ldk + 32 * ds);
@@ -1187,22 +1196,25 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
 #pragma unroll
         for (int i = 0; i < KW / 4; ++i) {
             const int r = 4 * i + g;
-            const int col = kvh * HD + 8 * (c16 ^ dkv3::swz(r));
-            dma16_async(rv, vsl + 4 * i * HD * 2, (unsigned)(((kw0 + r) * (int)p.ldv + col) * 2));
+            const int ch = c16 ^ dkv3::swz(r), col = kvh * HDR + 8 * ch;
+            dma16_async(rv, vsl + 4 * i * HD * 2,
+                        HDR == HD || ch < HDR / 8 ? (unsigned)(((kw0 + r) * (int)p.ldv + col) * 2) : kOOB);
         }
     }
     wait_vm0();  // K in registers and V in LDS before any tile DMA is queued
     __syncthreads();
-    f32x4 dvt[DSUB][KS], dkt[DSUB][KS];
+    f32x4 dvt[DSUBR][KS], dkt[DSUBR][KS];
 #pragma unroll
-    for (int i = 0; i < DSUB; ++i)
+    for (int i = 0; i < DSUBR; ++i)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) dvt[i][ks] = dkt[i][ks] = f32x4{0, 0, 0, 0};
 
     // causal: n_q == n_kv, so queries below k0 see none of the block's keys
     const int qstart = s.causal ? k0 : 0;
     const int nqt = RAG ? (s.n_q - qstart + BM - 1) / BM : (s.n_q - qstart) / BM;
-    const int niter = nh * (alt ? (nqt + 1) / 2 : nqt);
+    const int zparts = RAG ? max(1, p.split_parts) : 1, zpart = RAG ? (int)blockIdx.z : 0;
+    const int nsteps = nh * (alt ? (nqt + 1) / 2 : nqt);
+    const int niter = (nsteps - zpart + zparts - 1) / zparts;
     char *strm = smem + hg * STREAM;
 
     // this wave's DMA share: slice 0 moves Q and lse, slice 1 dO and D
@@ -1214,6 +1226,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
     const sgpr4 rs = rsrc4((tdo ? p.d : p.lse) + (long)b * s.n_q * s.n_heads,
                            (unsigned)((long)s.n_q * s.n_heads * 4));
     auto tile_of = [&](int it, int &h, int &q0) {
+        if constexpr (RAG) it = it * zparts + zpart;
         if (alt) {
             h = kvh * hpk + it % nh;
             q0 = qstart + ((nqt + 1) / 2 * 2 - 1 - 2 * (it / nh) - hg) * BM;
@@ -1237,8 +1250,9 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
 #pragma unroll
         for (int i = 0; i < RP / 4; ++i) {
             const int r = part * RP + 4 * i + lg;
-            const int col = h * HD + 8 * (l16 ^ dkv3::swz(r));
-            dma16_async(rt, dst + (part * RP + 4 * i) * HD * 2, (unsigned)(((q0 + r) * ldt + col) * 2));
+            const int ch = l16 ^ dkv3::swz(r), col = h * HDR + 8 * ch;
+            dma16_async(rt, dst + (part * RP + 4 * i) * HD * 2,
+                        HDR == HD || ch < HDR / 8 ? (unsigned)(((q0 + r) * ldt + col) * 2) : kOOB);
         }
         if (part == 0) {  // uniform; each branch names its LDS array (no generic pointer)
             const unsigned so = (unsigned)(((q0 + ln) * s.n_heads + h) * 4);
@@ -1275,7 +1289,11 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
         // where they are used (not held across the tile).  Every query row sees
         // at least one key on this path (causal needs n_q == n_kv, so row q sees
         // keys 0..q), so its LSE is finite and no empty-row case arises here.
-        auto lse2 = [&](int qs, int r) { return Ls[hg][buf][16 * qs + 4 * g + r] * LOG2E; };
+        // (RAG keeps the general kernels' rule for a row whose scores are all -inf: P = 0.)
+        auto lse2 = [&](int qs, int r) {
+            const float l = Ls[hg][buf][16 * qs + 4 * g + r];
+            return RAG && l == -INFINITY ? INFINITY : l * LOG2E;
+        };
         auto dval = [&](int qs, int r) { return Dd[hg][buf][16 * qs + 4 * g + r]; };
         // the dP accumulators start at -D, so they end as dP - D
         f32x4 sc[QS][KS], dp[QS][KS];
@@ -1295,9 +1313,9 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
         fr[0] = frag_row(Qb, c16, 8 * g);
         // S = Q K^T; f = (ds, qs) = (f / 2, f % 2)
 #pragma unroll
-        for (int f = 0; f < 8; ++f) {
+        for (int f = 0; f < NF; ++f) {
             const int ds = f / 2, qs = f % 2, n = f + 1;
-            fr[n & 1] = n < 8 ? frag_row(Qb, 16 * (n % 2) + c16, 32 * (n / 2) + 8 * g)
+            fr[n & 1] = n < NF ? frag_row(Qb, 16 * (n % 2) + c16, 32 * (n / 2) + 8 * g)
                               : frag_row(Ob, c16, 8 * g);
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) sc[qs][ks] = mfma16x16x32(fr[f & 1], kr[ks][ds], sc[qs][ks]);
@@ -1306,18 +1324,18 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
         // query halves), with P = exp2(S c - lse) of tile (f / 4, f % 4)
         bf16x8 vf[KS];
 #pragma unroll
-        for (int f = 0; f < 8; ++f) {
+        for (int f = 0; f < NF; ++f) {
             const int ds = f / 2, qs = f % 2, n = f + 1;
             if (qs == 0)
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) vf[ks] = frag_row(vsl, 16 * ks + c16, 32 * ds + 8 * g);
-            fr[n & 1] = n < 8 ? frag_row(Ob, 16 * (n % 2) + c16, 32 * (n / 2) + 8 * g)
+            fr[n & 1] = n < NF ? frag_row(Ob, 16 * (n % 2) + c16, 32 * (n / 2) + 8 * g)
                               : frag_t(Ob, 0, 0, g, c16);
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) dp[qs][ks] = mfma16x16x32(fr[f & 1], vf[ks], dp[qs][ks]);
             // the QS * KS score tiles spread evenly over the 8 steps
-            constexpr int EVERY = 8 / (QS * KS);
-            static_assert(EVERY >= 1 && EVERY * QS * KS == 8, "exp schedule");
+            constexpr int EVERY = NF / (QS * KS);
+            static_assert(EVERY >= 1 && EVERY * QS * KS == NF, "exp schedule");
             if (f % EVERY == 0) {
                 const int t2 = f / EVERY, qs2 = t2 / KS, ks2 = t2 % KS;
 #pragma unroll
@@ -1349,13 +1367,13 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) pb[ks] = frag_acc(sc[0][ks], sc[1][ks]);
 #pragma unroll
-            for (int i = 0; i < DSUB; ++i) {
+            for (int i = 0; i < DSUBR; ++i) {
                 const int n = i + 1;
-                fr[n & 1] = n < DSUB ? frag_t(Ob, 16 * n, 0, g, c16) : frag_t(Qb, 0, 0, g, c16);
+                fr[n & 1] = n < DSUBR ? frag_t(Ob, 16 * n, 0, g, c16) : frag_t(Qb, 0, 0, g, c16);
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) dvt[i][ks] = mfma16x16x32(fr[i & 1], pb[ks], dvt[i][ks]);
-                constexpr int EVERY = DSUB / (QS * KS);
-                static_assert(EVERY >= 1 && EVERY * QS * KS == DSUB, "dS schedule");
+                constexpr int EVERY = DSUBR / (QS * KS);
+                static_assert(EVERY >= 1 && EVERY * QS * KS == DSUBR, "dS schedule");
                 if (i % EVERY == 0) {
                     const int t2 = i / EVERY, qs2 = t2 / KS, ks2 = t2 % KS;
 #pragma unroll
@@ -1370,8 +1388,8 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) sb[ks] = frag_acc(dp[0][ks], dp[1][ks]);
 #pragma unroll
-            for (int i = 0; i < DSUB; ++i) {
-                if (i + 1 < DSUB) fr[(i + 1) & 1] = frag_t(Qb, 16 * (i + 1), 0, g, c16);
+            for (int i = 0; i < DSUBR; ++i) {
+                if (i + 1 < DSUBR) fr[(i + 1) & 1] = frag_t(Qb, 16 * (i + 1), 0, g, c16);
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) dkt[i][ks] = mfma16x16x32(fr[i & 1], sb[ks], dkt[i][ks]);
             }
@@ -1381,7 +1399,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
         // per SIMD the compiler's own split spills less
         if constexpr (NWV == 4) {
 #pragma unroll
-            for (int i = 0; i < DSUB; ++i)
+            for (int i = 0; i < DSUBR; ++i)
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+a"(dvt[i][ks]), "+a"(dkt[i][ks]));
         }
@@ -1397,19 +1415,19 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
     f32x4 *xs = reinterpret_cast<f32x4 *>(smem + (sl * 2 + hg) * XSLOT);
     const f32x4 *xp = reinterpret_cast<const f32x4 *>(smem + (sl * 2 + (1 - hg)) * XSLOT);
     // group 0 hands over dK^T and keeps dV^T; group 1 the other way round
-    auto give = [&](const f32x4 (&a)[DSUB][KS]) {
+    auto give = [&](const f32x4 (&a)[DSUBR][KS]) {
 #pragma unroll
-        for (int i = 0; i < DSUB; ++i)
+        for (int i = 0; i < DSUBR; ++i)
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) xs[(i * KS + ks) * 64 + lane] = a[i][ks];
     };
-    auto keep = [&](const f32x4 (&a)[DSUB][KS], float *base, long ld, float sc_) {
+    auto keep = [&](const f32x4 (&a)[DSUBR][KS], float *base, long ld, float sc_) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             if (RAG && kw0 + 16 * ks + c16 >= s.n_kv) continue;
-            float *out = base + ((long)b * s.n_kv + kw0 + 16 * ks + c16) * ld + kvh * HD;
+            float *out = base + ((long)b * s.n_kv + kw0 + 16 * ks + c16) * ld + kvh * HDR;
 #pragma unroll
-            for (int i = 0; i < DSUB; ++i) {
+            for (int i = 0; i < DSUBR; ++i) {
                 const f32x4 v = a[i][ks] + xp[(i * KS + ks) * 64 + lane];
                 *reinterpret_cast<float4 *>(out + 16 * i + 4 * g) =
                     make_float4(v[0] * sc_, v[1] * sc_, v[2] * sc_, v[3] * sc_);
@@ -1425,6 +1443,13 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
         if (hg == 0) keep(dvt, wv, kvd, 1.0f);
         else keep(dkt, wk, kvd, s.inv_sqrt_dim);
     } else if constexpr (!QKE) {
+        if (RAG && zparts > 1) {
+            const long n = (long)s.n_batch * s.n_kv * s.n_kv_heads * HDR;
+            float *ws = p.split_ws + 2 * zpart * n;
+            if (hg == 0) keep(dvt, ws + n, (long)s.n_kv_heads * HDR, 1.0f);
+            else keep(dkt, ws, (long)s.n_kv_heads * HDR, s.inv_sqrt_dim);
+            return;
+        }
         if (hg == 0) keep(dvt, p.dv, p.lddv, 1.0f);
         else keep(dkt, p.dk, p.lddk, s.inv_sqrt_dim);
     } else {
@@ -1434,7 +1459,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
         const QkEpi &e = p.qk;
         float dw[8][4] = {};
         const int kcol = s.n_heads * HD + kvh * HD, vcol = kcol + s.n_kv_heads * HD;
-        auto rows = [&](const f32x4(&a)[DSUB][KS], bool is_k) {
+        auto rows = [&](const f32x4(&a)[DSUBR][KS], bool is_k) {
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
                 const int key = kw0 + 16 * ks + c16;
@@ -1442,7 +1467,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
                 const float sc_ = is_k ? s.inv_sqrt_dim : 1.0f;
                 float v[8][4];
 #pragma unroll
-                for (int i = 0; i < DSUB; ++i) {
+                for (int i = 0; i < DSUBR; ++i) {
                     const f32x4 w = a[i][ks] + xp[(i * KS + ks) * 64 + lane];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[i][r] = w[r] * sc_;
@@ -1458,6 +1483,24 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
             qk_dw_block(dw, red, sl, NS, hg == 1, lane, e.pk + (long)blk * 128);
         }
     }
+}
+
+// dK and dV from the parts of a split ragged launch, added in part order.  One float4
+// per thread; bound by reading the parts.
+__global__ __launch_bounds__(256) void fa_dkv_sum_k(AttnPtrs p, size_t rows, int kvd4) {
+    const size_t n = rows * kvd4, i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= 2 * n) return;
+    const bool v = i >= n;
+    const size_t j = v ? i - n : i, row = j / kvd4;
+    const int c = (int)(j - row * kvd4);
+    const float4 *ws = reinterpret_cast<const float4 *>(p.split_ws) + i;
+    float4 a = ws[0];
+    for (int z = 1; z < p.split_parts; ++z) {
+        const float4 t = ws[2 * n * z];
+        a.x += t.x; a.y += t.y; a.z += t.z; a.w += t.w;
+    }
+    float *out = v ? p.dv + row * p.lddv : p.dk + row * p.lddk;
+    *reinterpret_cast<float4 *>(out + 4 * c) = a;
 }
 
 // The two slices of a split dK / dV launch (p.split_ws: [part][dK, dV][rows][kvd]
@@ -1538,12 +1581,15 @@ constexpr int NBUF = 3;
 // WITH_D: D = rowsum(O dO) of the block's rows is formed here from bf16 O (the
 // lane's 32 products in fp64, then the row's four lanes) and stored to p.d
 // for the dK/dV kernel, which then runs after this one; no separate pass.
-template <int NWV, bool WITH_D, bool QKE, int BQ>
+// HDR = 64: as in the dK/dV kernel.
+template <int NWV, bool WITH_D, bool QKE, int BQ, int HDR = 128>
 __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtrs p) {
     using namespace dq4;
     constexpr int QSUB = BQ / 16 / NWV;  // 16-row query sub-tiles per wave
     constexpr int QST = 16 * NWV;        // row stride between a wave's sub-tiles
     constexpr int RPW = BN / NWV;        // K / V tile rows each wave moves by DMA
+    constexpr int DSR = HDR / 32, DSUBR = HDR / 16, NF = 2 * DSR;  // of the real head
+    static_assert(HDR == HD || (!QKE && HDR == 64), "head width");
     using dkv3::frag_row;
     using dkv3::frag_t;
     __shared__ __attribute__((aligned(16))) char Kt[NBUF][TILE];
@@ -1557,17 +1603,17 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
     const int q00 = qblk * BQ + 16 * wave;  // first row of sub-tile j is q00 + QST j
     const float c2 = s.inv_sqrt_dim * LOG2E;
 
-    bf16x8 qr[QSUB][DS], orr[QSUB][DS];
+    bf16x8 qr[QSUB][DSR], orr[QSUB][DSR];
     float lq[QSUB], dd[QSUB];
 #pragma unroll
     for (int j = 0; j < QSUB; ++j) {
         const int q = q00 + QST * j + c16;
         const bool ok = q < s.n_q;
         const long t = (long)b * s.n_q + q;
-        const bf16 *qp = (const bf16 *)p.q + t * p.ldq + h * HD + 8 * g;
-        const bf16 *op = (const bf16 *)p.dout + t * p.lddo + h * HD + 8 * g;
+        const bf16 *qp = (const bf16 *)p.q + t * p.ldq + h * HDR + 8 * g;
+        const bf16 *op = (const bf16 *)p.dout + t * p.lddo + h * HDR + 8 * g;
 #pragma unroll
-        for (int ds = 0; ds < DS; ++ds) {
+        for (int ds = 0; ds < DSR; ++ds) {
             qr[j][ds] = ok ? ld_frag(qp + 32 * ds) : bf16x8{};
             orr[j][ds] = ok ? ld_frag(op + 32 * ds) : bf16x8{};
         }
@@ -1575,10 +1621,10 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
         // rows past n_q and fully masked rows (lse = -inf) get P = 0
         lq[j] = l == -INFINITY ? INFINITY : l * LOG2E;
         if constexpr (WITH_D) {
-            const bf16 *opo = (const bf16 *)p.o16 + t * p.ldo16 + h * HD + 8 * g;
+            const bf16 *opo = (const bf16 *)p.o16 + t * p.ldo16 + h * HDR + 8 * g;
             double acc = 0;
 #pragma unroll
-            for (int ds = 0; ds < DS; ++ds) {
+            for (int ds = 0; ds < DSR; ++ds) {
                 const bf16x8 ov = ok ? ld_frag(opo + 32 * ds) : bf16x8{};
 #pragma unroll
                 for (int e = 0; e < 8; ++e) acc += (double)(float)ov[e] * (double)(float)orr[j][ds][e];
@@ -1592,9 +1638,9 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
         }
     }
     wait_vm0();
-    f32x4 acc[DSUB][QSUB];
+    f32x4 acc[DSUBR][QSUB];
 #pragma unroll
-    for (int i = 0; i < DSUB; ++i)
+    for (int i = 0; i < DSUBR; ++i)
 #pragma unroll
         for (int j = 0; j < QSUB; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
 
@@ -1611,10 +1657,11 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
 #pragma unroll
         for (int i = 0; i < RPW / 4; ++i) {
             const int r = RPW * wave + 4 * i + g;
-            const int col = kvh * HD + 8 * (c16 ^ dkv3::swz(r));
+            const int ch = c16 ^ dkv3::swz(r), col = kvh * HDR + 8 * ch;
+            const bool in = HDR == HD || ch < HDR / 8;
             const int lo = (RPW * wave + 4 * i) * HD * 2;
-            dma16_async(rk, Kt[buf] + lo, (unsigned)(((kk + r) * (int)p.ldk + col) * 2));
-            dma16_async(rv, Vt[buf] + lo, (unsigned)(((kk + r) * (int)p.ldv + col) * 2));
+            dma16_async(rk, Kt[buf] + lo, in ? (unsigned)(((kk + r) * (int)p.ldk + col) * 2) : kOOB);
+            dma16_async(rv, Vt[buf] + lo, in ? (unsigned)(((kk + r) * (int)p.ldv + col) * 2) : kOOB);
         }
     };
     if (ntl > 0) dma(0, 0);
@@ -1651,16 +1698,16 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
         // slots ahead of its MFMAs through a ring of PD + 1 fragments.
         constexpr int PD = 2, RING = PD + 1;
         auto ldslot = [&](int n) -> bf16x8 {
-            if (n < 8) return frag_row(Kb, 16 * (n % 2) + c16, 32 * (n / 2) + 8 * g);
-            if (n < 16) return frag_row(Vb, 16 * ((n - 8) % 2) + c16, 32 * ((n - 8) / 2) + 8 * g);
-            return frag_t(Kb, 16 * (n - 16), 0, g, c16);
+            if (n < NF) return frag_row(Kb, 16 * (n % 2) + c16, 32 * (n / 2) + 8 * g);
+            if (n < 2 * NF) return frag_row(Vb, 16 * ((n - NF) % 2) + c16, 32 * ((n - NF) / 2) + 8 * g);
+            return frag_t(Kb, 16 * (n - 2 * NF), 0, g, c16);
         };
         bf16x8 fr[RING];
 #pragma unroll
         for (int n = 0; n < PD; ++n) fr[n] = ldslot(n);
         // S^T = K Q^T
 #pragma unroll
-        for (int f = 0; f < 8; ++f) {
+        for (int f = 0; f < NF; ++f) {
             const int ds = f / 2, ks = f % 2, n = f;
             fr[(n + PD) % RING] = ldslot(n + PD);
 #pragma unroll
@@ -1668,14 +1715,14 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
         }
         // dP^T = V dO^T, with P^T = exp2(S^T c - lse) of one (ks, j) tile per step
 #pragma unroll
-        for (int f = 0; f < 8; ++f) {
-            const int ds = f / 2, ks = f % 2, n = 8 + f;
+        for (int f = 0; f < NF; ++f) {
+            const int ds = f / 2, ks = f % 2, n = NF + f;
             fr[(n + PD) % RING] = ldslot(n + PD);
 #pragma unroll
             for (int j = 0; j < QSUB; ++j) dpt[ks][j] = mfma16x16x32(fr[n % RING], orr[j][ds], dpt[ks][j]);
             // the KS * QSUB score tiles spread evenly over the 8 steps
-            constexpr int EVERY = 8 / (KS * QSUB);
-            static_assert(EVERY >= 1 && EVERY * KS * QSUB == 8, "exp schedule");
+            constexpr int EVERY = NF / (KS * QSUB);
+            static_assert(EVERY >= 1 && EVERY * KS * QSUB == NF, "exp schedule");
             if (f % EVERY == 0) {
                 const int t2 = f / EVERY, ks2 = t2 / QSUB, j2 = t2 % QSUB;
 #pragma unroll
@@ -1704,9 +1751,9 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
         }
         // dQ^T += K^T dS^T
 #pragma unroll
-        for (int i = 0; i < DSUB; ++i) {
-            const int n = 16 + i;
-            if (n + PD < 24) fr[(n + PD) % RING] = ldslot(n + PD);
+        for (int i = 0; i < DSUBR; ++i) {
+            const int n = 2 * NF + i;
+            if (n + PD < 2 * NF + DSUBR) fr[(n + PD) % RING] = ldslot(n + PD);
 #pragma unroll
             for (int j = 0; j < QSUB; ++j) acc[i][j] = mfma16x16x32(fr[n % RING], sb[j], acc[i][j]);
         }
@@ -1729,7 +1776,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
             const long t = (long)b * s.n_q + (ok ? q : 0);
             float v[8][4];
 #pragma unroll
-            for (int i = 0; i < DSUB; ++i)
+            for (int i = 0; i < DSUBR; ++i)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[i][r] = acc[i][j][r] * s.inv_sqrt_dim;
             qk_row_bwd(v, dw, ok, e, e.x + t * e.ldx + h * HD, e.gq, ok ? q : 0, g);
@@ -1745,10 +1792,10 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
     for (int j = 0; j < QSUB; ++j) {
         const int q = q00 + QST * j + c16;
         if (q >= s.n_q) continue;
-        float *dqr = p.dq + ((long)b * s.n_q + q) * p.lddq + h * HD;
+        float *dqr = p.dq + ((long)b * s.n_q + q) * p.lddq + h * HDR;
         const float sc_ = s.inv_sqrt_dim;
 #pragma unroll
-        for (int i = 0; i < DSUB; ++i) {
+        for (int i = 0; i < DSUBR; ++i) {
             const f32x4 a = acc[i][j];
             *reinterpret_cast<float4 *>(dqr + 16 * i + 4 * g) =
                 make_float4(a[0] * sc_, a[1] * sc_, a[2] * sc_, a[3] * sc_);
@@ -2210,12 +2257,24 @@ void launch_dkv4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     else hipLaunchKernelGGL((fa_bwd_dkv4_k<W, QKE, 0>), gkv, dim3(W * 64), 0, st, s, p);
 }
 
+void dkv_sum(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
+    const size_t rows = (size_t)s.n_batch * s.n_kv;
+    const int kvd4 = s.n_kv_heads * s.head_dim / 4;
+    hipLaunchKernelGGL(fa_dkv_sum_k, dim3(ceil_div(2 * rows * kvd4, 256)), dim3(256), 0, st, p, rows, kvd4);
+}
 void launch_dkv4_ragged(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
-    const dim3 gkv(s.n_kv_heads * s.n_batch, (s.n_kv + dkv4::BN - 1) / dkv4::BN);
-    hipLaunchKernelGGL((fa_bwd_dkv4_k<8, false, 0, 1, true>), gkv, dim3(512), 0, st, s, p);
+    const int parts = p.split_ws ? std::max(1, p.split_parts) : 1;
+    const dim3 gkv(s.n_kv_heads * s.n_batch, (s.n_kv + dkv4::BN - 1) / dkv4::BN, parts);
+    AttnPtrs q = p;
+    q.split_parts = parts;
+    if (s.head_dim == 64)
+        hipLaunchKernelGGL((fa_bwd_dkv4_k<8, false, 0, 1, true, 64>), gkv, dim3(512), 0, st, s, q);
+    else
+        hipLaunchKernelGGL((fa_bwd_dkv4_k<8, false, 0, 1, true>), gkv, dim3(512), 0, st, s, q);
+    if (parts > 1) dkv_sum(s, q, st);
 }
 
-// dQ blocks of 256 queries, or of 128 where 256 would leave fewer blocks than
+// dQ blocks of 256 queries (8 waves), of 128 (8 waves) or of 64 (4 waves): of 128 where 256 would leave fewer blocks than
 // CUs: there a causal grid is also short of work at its end, since a block's
 // work grows with its last query (config 3, 4 x 512: 128 blocks of 256 rows,
 // the later block of each sequence twice the earlier); with 256-query blocks
@@ -2224,11 +2283,26 @@ int dq4_bq(const AttnShape &s) {
     const long b256 = (long)s.n_heads * s.n_batch * ((s.n_q + 255) / 256);
     return b256 < 256 ? 128 : 256;
 }
+// ... and of 64 for a standalone call whose grid of 128 would still leave CUs idle
+// (the training step's plan stays at 128: its fused epilogue counts those blocks).
+bool dq4_small(const AttnShape &s) {
+    return s.ragged && (long)s.n_heads * s.n_batch * ((s.n_q + 127) / 128) < 256;
+}
 template <bool WITH_D, bool QKE>
 void launch_dq4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     constexpr int W = 8;
-    const int bq = dq4_bq(s);
+    const int bq = !QKE && dq4_small(s) ? 64 : dq4_bq(s);
     const dim3 gq(s.n_heads * s.n_batch, (s.n_q + bq - 1) / bq);
+    if constexpr (!QKE) {
+        auto go = [&](auto kernel, int nt) { hipLaunchKernelGGL(kernel, gq, dim3(nt), 0, st, s, p); };
+        if (s.head_dim == 64) {
+            if (bq == 64) go(fa_bwd_dq4_k<4, WITH_D, false, 64, 64>, 256);
+            else if (bq == 128) go(fa_bwd_dq4_k<W, WITH_D, false, 128, 64>, W * 64);
+            else go(fa_bwd_dq4_k<W, WITH_D, false, 256, 64>, W * 64);
+            return;
+        }
+        if (bq == 64) return go(fa_bwd_dq4_k<4, WITH_D, false, 64>, 256);
+    }
     if (bq == 128)
         hipLaunchKernelGGL((fa_bwd_dq4_k<W, WITH_D, QKE, 128>), gq, dim3(W * 64), 0, st, s, p);
     else
@@ -2236,21 +2310,42 @@ void launch_dq4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
 }
 
 // The recompute kernels on lengths that are not whole tiles, or with an odd head
-// group: head_dim 128, n_q == n_kv under a causal mask, 16-byte aligned rows under
+// group: head_dim 64 or 128, n_q == n_kv under a causal mask, 16-byte aligned rows under
 // 2 GiB a sequence.
 static bool v4_ragged_ok(const AttnShape &s, const AttnPtrs &p) {
     auto al = [](const void *x, long ld) { return ((uintptr_t)x & 15) == 0 && ld % 8 == 0; };
-    return p.dt == DType::BF16 && s.head_dim == 128 && (!s.causal || s.n_q == s.n_kv) && s.n_kv > 0 &&
+    return p.dt == DType::BF16 && bf16_ok(s) && (!s.causal || s.n_q == s.n_kv) && s.n_kv > 0 &&
            al(p.q, p.ldq) && al(p.k, p.ldk) && al(p.v, p.ldv) && al(p.dout, p.lddo) &&
            (!p.o16 || al(p.o16, p.ldo16)) && (long)s.n_q * std::max(p.ldq, p.lddo) * 2 < (1l << 30) &&
            (long)s.n_kv * std::max(p.ldk, p.ldv) * 2 < (1l << 30);
 }
 static bool al_out(const float *x, long ld) { return ((uintptr_t)x & 15) == 0 && ld % 4 == 0; }
 
+// Blocks per key block of a split dK / dV launch: towards one block per CU (fp32: two
+// of its smaller ones), while each keeps at least four (head, query tile) steps (fp32:
+// two, its tile steps take longer).  bf16 1 x 1024 tokens, 16 / 4 heads, head_dim 128:
+// the backward 138 -> 60 us; fp32 1 x 1000: dK/dV 774 -> 169 us.
+int fa_bw_parts(const AttnShape &s, DType dt) {
+    if (s.head_dim != 128 && s.head_dim != 64) return 1;
+    const bool f32 = dt == DType::F32;
+    if (!f32 && s.causal && s.n_q != s.n_kv) return 1;
+    const int hpk = s.n_heads / s.n_kv_heads;
+    const long rows = (long)s.n_kv_heads * s.n_batch;
+    const long blocks = rows * ((s.n_kv + (f32 ? 63 : dkv4::BN - 1)) / (f32 ? 64 : dkv4::BN));
+    const long tiles = (long)hpk * ((s.n_q + 31) / 32);
+    if (f32) return (int)std::max(1l, std::min({16l, 512 / blocks, tiles / 2}));
+    return (int)std::max(1l, std::min({8l, 256 / blocks, tiles / 8}));
+}
+size_t fa_bw_parts_ws_bytes(const AttnShape &s, int parts) {
+    return parts > 1 ? (size_t)8 * parts * s.n_batch * s.n_kv * s.n_kv_heads * s.head_dim : 0;
+}
+void fa_dkv_sum(const AttnShape &s, const AttnPtrs &p, hipStream_t st) { dkv_sum(s, p, st); }
+
+bool fa_bw_ragged_ok(const AttnShape &s, const AttnPtrs &p) {
+    return v4_ragged_ok(s, p) && al_out(p.dq, p.lddq) && al_out(p.dk, p.lddk) && al_out(p.dv, p.lddv);
+}
 bool fa_bw_ragged(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
-    if (!p.o16 || !v4_ragged_ok(s, p) || !al_out(p.dq, p.lddq) || !al_out(p.dk, p.lddk) ||
-        !al_out(p.dv, p.lddv))
-        return false;
+    if (!p.o16 || !fa_bw_ragged_ok(s, p)) return false;
     launch_dq4<true, false>(s, p, st);  // forms D
     launch_dkv4_ragged(s, p, st);
     return true;

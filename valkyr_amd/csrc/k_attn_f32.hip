@@ -23,6 +23,8 @@
 // log2(e) / sqrt(hd), lse read in natural units and converted.
 #include <math.h>
 
+#include <algorithm>
+
 #include "ops.hpp"
 #include "qkbwd.hpp"
 
@@ -251,8 +253,12 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
     const int shift = RAG ? s.n_kv - s.n_q : 0;
     const int qstart = s.causal ? max(0, k0 - shift) : 0;  // (without RAG causal needs n_q == n_kv)
     const int nqt = RAG ? (s.n_q - qstart + FT - 1) / FT : (s.n_q - qstart) / FT;
-    const int niter = hpk * nqt;
+    // RAG: blockIdx.z takes every split_parts-th step, its raw sums go to its slice of
+    // p.split_ws (as in the bf16 kernel)
+    const int zparts = RAG ? max(1, p.split_parts) : 1, zpart = RAG ? (int)blockIdx.z : 0;
+    const int niter = (hpk * nqt - zpart + zparts - 1) / zparts;
     auto tile_of = [&](int it, int &h, int &q0) {
+        if constexpr (RAG) it = it * zparts + zpart;
         h = kvh * hpk + it / nqt;
         q0 = qstart + (it % nqt) * FT;
     };
@@ -345,6 +351,11 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
     if (RAG && ki >= s.n_kv) return;
     float *dkr = p.dk + ((long)b * s.n_kv + ki) * p.lddk + kvh * HD + 4 * g;
     float *dvr = p.dv + ((long)b * s.n_kv + ki) * p.lddv + kvh * HD + 4 * g;
+    if (RAG && zparts > 1) {
+        const long kvd = (long)s.n_kv_heads * HD, n = (long)s.n_batch * s.n_kv * kvd;
+        dkr = p.split_ws + 2 * zpart * n + ((long)b * s.n_kv + ki) * kvd + kvh * HD + 4 * g;
+        dvr = dkr + n;
+    }
     const float sc = s.inv_sqrt_dim;
     if constexpr (QKE) {
         __shared__ float red[4 * 128];
@@ -539,12 +550,17 @@ bool fa_f32m_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     if (!fa_f32m_ok(s) || !ptrs_ok(p) || !al16(p.dk) || !al16(p.dv) || p.lddk % 4 || p.lddv % 4)
         return false;
     if (p.qk_fp32 && !fa_f32m_qk_ok(s, p)) return false;
-    const dim3 grid(s.n_kv_heads * s.n_batch, (s.n_kv + 63) / 64);
-    const bool zz = fits_two_per_cu((long)grid.x * grid.y);
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(FNT), 0, st, s, p, zz); };
+    AttnPtrs q = p;
+    q.split_parts = s.ragged && p.split_ws ? std::max(1, p.split_parts) : 1;
+    const dim3 grid(s.n_kv_heads * s.n_batch, (s.n_kv + 63) / 64, q.split_parts);
+    const bool zz = q.split_parts == 1 && fits_two_per_cu((long)grid.x * grid.y);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(FNT), 0, st, s, q, zz); };
     if (p.qk_fp32) go(fa_bwd_dkv_f32m_k<128, true>);
-    else if (whole_tiles(s)) s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false>) : go(fa_bwd_dkv_f32m_k<64, false>);
-    else s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false, true>) : go(fa_bwd_dkv_f32m_k<64, false, true>);
+    else if (whole_tiles(s) && q.split_parts == 1)
+        s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false>) : go(fa_bwd_dkv_f32m_k<64, false>);
+    else
+        s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false, true>) : go(fa_bwd_dkv_f32m_k<64, false, true>);
+    if (q.split_parts > 1) fa_dkv_sum(s, q, st);
     return true;
 }
 

@@ -316,7 +316,7 @@ struct AttnShape {
     int n_batch, n_q, n_kv, n_heads, n_kv_heads, head_dim;
     int causal;
     float inv_sqrt_dim;
-    int ragged = 0;  // fp32: the tile kernels also for lengths that are not whole tiles
+    int ragged = 0;  // a standalone call: fp32 tile kernels for any length, small dQ blocks
 };
 // Fused q/k gradient epilogue of the recompute attention backward: dQ, dK
 // and dV leave the kernels as bf16 rows of one [T, (H + 2 Hkv) hd] matrix
@@ -357,6 +357,8 @@ struct AttnPtrs {
     // recompute path: workspace of fa_bw_v4_split_ws_floats(s) floats; when set
     // on a shape fa_bw_v4_split accepts, the dK / dV launch is split in two
     float *split_ws = nullptr;
+    // ragged form: blocks per key block, with fa_bw_parts_ws_bytes(s, parts) in split_ws
+    int split_parts = 0;
 };
 // fp32 attention on the matrix cores (k_attn_f32.hip) for the shapes
 // fa_f32m_ok accepts; each launcher returns false, launching nothing, for a
@@ -386,6 +388,10 @@ hipError_t fa_bw_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st);
 // The whole bf16 backward from bf16 O (p.o16; D is written) on shapes the fused form
 // does not take, with the recompute kernels' ragged form; false, launching nothing,
 // where they do not apply (fa_bw_dkv and fa_bw_dq pick it by the same rule).
+int fa_bw_parts(const AttnShape &s, DType dt);
+void fa_dkv_sum(const AttnShape &s, const AttnPtrs &p, hipStream_t st);  // adds the parts
+bool fa_bw_ragged_ok(const AttnShape &s, const AttnPtrs &p);
+size_t fa_bw_parts_ws_bytes(const AttnShape &s, int parts);
 bool fa_bw_ragged(const AttnShape &s, const AttnPtrs &p, hipStream_t st);
 // Fused bf16 backward.  Requires fa_bw_fused_ok(s) (bf16 head_dim 64/128, n_q
 // and n_kv multiples of 64, self-attention when causal).  v4 (requires
