@@ -1803,7 +1803,30 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
     }
 }
 
-// ── forward v3 (head_dim 128): DMA-staged K / V tiles ────────────────────
+// Maximum / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 that hold one row of a
+// transposed score tile: the swaps give every lane both halves' values.
+// (The compiler's builtin returned one register for both results here, so the two
+// instructions are written out, with the two wait states they need after a VALU write.)
+template <int L>
+VKH_DEV void lane_halves(float v, float &a, float &b) {
+    a = b = v;
+    if constexpr (L == 32) asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    else asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+VKH_DEV float xrow_max(float v) {
+    float a, b;
+    lane_halves<32>(v, a, b);
+    lane_halves<16>(fmaxf(a, b), a, b);
+    return fmaxf(a, b);
+}
+VKH_DEV float xrow_sum(float v) {
+    float a, b;
+    lane_halves<16>(v, a, b);
+    lane_halves<32>(a + b, a, b);
+    return a + b;
+}
+
+// ── forward v3: DMA-staged K / V tiles ───────────────────────────────────
 // One (q tile of 64 QS rows, head, sequence) per block, 4 waves x 16 QS queries
 // (QS = 1 where 128-query blocks would be at most one per CU: config 3's 256
 // become 512 blocks of 64, two per CU: the step 19.06-19.10 -> 18.86-18.89
@@ -1815,12 +1838,19 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
 // tile through the transposing LDS read (no transposed staging copy).
 // Causal q tiles go heaviest first (a zigzag order, zigzag in common.hpp,
 // measured 77.6 against 78.9 us at config 4's 512-block grid: within noise).
-template <int QS>
+// Bound by the vector ALU's softmax beside the matrix cores (about 1.7 of its cycles to
+// 1 of theirs before): the scale is folded into one fma per score, masked scores need no
+// test of their own (exp2 of -inf is 0), the row sum stays per lane until the end, the
+// row maximum crosses lanes by permlane swaps, and the accumulators are rescaled only in
+// tiles where a row of the wave got a new maximum.  HDR = 64: 64-wide heads in the same
+// 128-wide LDS rows (as in the backward).
+template <int QS, int HDR = 128>
 __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, long ldq,
                                                      const bf16 *k, long ldk, const bf16 *v,
                                                      long ldv, float *o, long ldo, float *lse,
                                                      bf16 *ob, long ldob) {
     using namespace dkv3;
+    constexpr int DSR = HDR / 32, DSUBR = HDR / 16;  // of the real head
     constexpr int FBM = 64 * QS, FBN = 64, KT = FBN * HD * 2;
     __shared__ __attribute__((aligned(16))) char Ks[2][KT];
     __shared__ __attribute__((aligned(16))) char Vs[2][KT];
@@ -1834,26 +1864,31 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int q0 = qt * FBM, qw0 = q0 + wave * 16 * QS;
     const int off = s.n_kv - s.n_q;
-    const bf16 *qb = q + (long)b * s.n_q * ldq + h * HD;
-    const float c2 = s.inv_sqrt_dim * LOG2E;
+    const bf16 *qb = q + (long)b * s.n_q * ldq + h * HDR;
+    // scores are compared unscaled: a negative scale flips Q's signs (exact)
+    const float c2 = fmaxf(fabsf(s.inv_sqrt_dim) * LOG2E, 1e-37f);
+    const bool neg = s.inv_sqrt_dim < 0.f;
 
-    bf16x8 qf[QS][DS];
+    bf16x8 qf[QS][DSR];
 #pragma unroll
     for (int qs = 0; qs < QS; ++qs) {
         const int qr = qw0 + 16 * qs + c16;
 #pragma unroll
-        for (int ds = 0; ds < DS; ++ds)
+        for (int ds = 0; ds < DSR; ++ds)
+        {
             qf[qs][ds] = qr < s.n_q ? ld_frag(qb + (long)qr * ldq + 32 * ds + 8 * g) : bf16x8{};
+            if (neg) qf[qs][ds] = -qf[qs][ds];
+        }
     }
     wait_vm0();  // Q fragments are in registers before any DMA is queued
-    f32x4 oacc[DSUB][QS];
+    f32x4 oacc[DSUBR][QS];
     float m[QS], l[QS];
 #pragma unroll
     for (int qs = 0; qs < QS; ++qs) {
         m[qs] = -INFINITY;
         l[qs] = 0.f;
 #pragma unroll
-        for (int i = 0; i < DSUB; ++i) oacc[i][qs] = f32x4{0, 0, 0, 0};
+        for (int i = 0; i < DSUBR; ++i) oacc[i][qs] = f32x4{0, 0, 0, 0};
     }
 
     int kend = s.n_kv;
@@ -1869,10 +1904,11 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
         for (int i = 0; i < 4; ++i) {
             const int r = 16 * wave + 4 * i + g;
             const int c = c16 ^ swz(r);
+            const bool in = HDR == HD || c < HDR / 8;
             dma16_async(rk, Ks[buf] + (16 * wave + 4 * i) * HD * 2,
-                        (unsigned)(((k0 + r) * (int)ldk + kvh * HD + 8 * c) * 2));
+                        in ? (unsigned)(((k0 + r) * (int)ldk + kvh * HDR + 8 * c) * 2) : kOOB);
             dma16_async(rv, Vs[buf] + (16 * wave + 4 * i) * HD * 2,
-                        (unsigned)(((k0 + r) * (int)ldv + kvh * HD + 8 * c) * 2));
+                        in ? (unsigned)(((k0 + r) * (int)ldv + kvh * HDR + 8 * c) * 2) : kOOB);
         }
     };
     if (nkt > 0) dma(0, 0);
@@ -1892,7 +1928,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
 #pragma unroll
             for (int qs = 0; qs < QS; ++qs) st[ks][qs] = f32x4{0, 0, 0, 0};
 #pragma unroll
-        for (int ds = 0; ds < DS; ++ds)
+        for (int ds = 0; ds < DSR; ++ds)
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 const bf16x8 kf = frag_row(Kb, 16 * ks + c16, 32 * ds + 8 * g);
@@ -1904,46 +1940,46 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
 #pragma unroll
         for (int qs = 0; qs < QS; ++qs) {
             const int qa = qw0 + 16 * qs + c16;
+            if (edge) {
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int ka = k0 + 16 * ks + 4 * g + r;
+                        if (ka >= s.n_kv || (s.causal && ka > qa + off)) st[ks][qs][r] = -INFINITY;
+                    }
+            }
             float mt = -INFINITY;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float x = st[ks][qs][r] * c2;
-                    if (edge) {
-                        const int ka = k0 + 16 * ks + 4 * g + r;
-                        if (ka >= s.n_kv || (s.causal && ka > qa + off)) x = -INFINITY;
-                    }
-                    st[ks][qs][r] = x;
-                    mt = fmaxf(mt, x);
-                }
-            mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-            mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-            const float mn = fmaxf(m[qs], mt);
-            const float so = (m[qs] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[qs] - mn);
+                for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[ks][qs][r]);
+            const float mn = fmaxf(m[qs], xrow_max(mt));
+            const float ms = mn == -INFINITY ? 0.f : mn * c2;  // no visible key yet: P = 0
+            if (__any(mn != m[qs])) {
+                const float so = __builtin_amdgcn_exp2f(fmaf(m[qs], c2, -ms));
+                l[qs] *= so;
+#pragma unroll
+                for (int i = 0; i < DSUBR; ++i) oacc[i][qs] *= so;
+                m[qs] = mn;
+            }
             float lt = 0.f;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float x = st[ks][qs][r];
-                    const float pv = (x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(x - mn);
+                    const float pv = __builtin_amdgcn_exp2f(fmaf(st[ks][qs][r], c2, -ms));
                     st[ks][qs][r] = pv;
                     lt += pv;
                 }
-            lt += __shfl_xor(lt, 16, 64);
-            lt += __shfl_xor(lt, 32, 64);
-            l[qs] = l[qs] * so + lt;
-            m[qs] = mn;
-#pragma unroll
-            for (int i = 0; i < DSUB; ++i) oacc[i][qs] *= so;
+            l[qs] += lt;
             pf[qs][0] = frag_acc(st[0][qs], st[1][qs]);
             pf[qs][1] = frag_acc(st[2][qs], st[3][qs]);
         }
 #pragma unroll
         for (int kst = 0; kst < 2; ++kst)
 #pragma unroll
-            for (int i = 0; i < DSUB; ++i) {
+            for (int i = 0; i < DSUBR; ++i) {
                 const bf16x8 vf = frag_t(Vb, 16 * i, 32 * kst, g, c16);
 #pragma unroll
                 for (int qs = 0; qs < QS; ++qs) oacc[i][qs] = mfma16x16x32(vf, pf[qs][kst], oacc[i][qs]);
@@ -1952,23 +1988,24 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
 #pragma unroll
     for (int qs = 0; qs < QS; ++qs) {
         const int qa = qw0 + 16 * qs + c16;
+        const float lq = xrow_sum(l[qs]);
         if (qa >= s.n_q) continue;
-        const float inv = l[qs] > 0.f ? 1.0f / l[qs] : 0.f;
-        float *orow = o + ((long)b * s.n_q + qa) * ldo + h * HD;
+        const float inv = lq > 0.f ? 1.0f / lq : 0.f;
+        float *orow = o + ((long)b * s.n_q + qa) * ldo + h * HDR;
 #pragma unroll
-        for (int i = 0; i < DSUB; ++i) {
+        for (int i = 0; i < DSUBR; ++i) {
             const f32x4 a = oacc[i][qs];
             const float4 ov = make_float4(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
             if (o) *reinterpret_cast<float4 *>(orow + 16 * i + 4 * g) = ov;
             if (ob) {
                 bf16x4 bv;
                 bv[0] = (bf16)ov.x; bv[1] = (bf16)ov.y; bv[2] = (bf16)ov.z; bv[3] = (bf16)ov.w;
-                *reinterpret_cast<bf16x4 *>(ob + ((long)b * s.n_q + qa) * ldob + h * HD + 16 * i + 4 * g) = bv;
+                *reinterpret_cast<bf16x4 *>(ob + ((long)b * s.n_q + qa) * ldob + h * HDR + 16 * i + 4 * g) = bv;
             }
         }
         if (lse && g == 0)
             lse[((long)b * s.n_q + qa) * s.n_heads + h] =
-                l[qs] > 0.f ? (m[qs] + log2f(l[qs])) * LN2 : -INFINITY;
+                lq > 0.f ? fmaf(m[qs], c2, log2f(lq)) * LN2 : -INFINITY;
     }
 }
 
@@ -2172,19 +2209,15 @@ hipError_t fa_forward(const AttnShape &s, const void *q, long ldq, const void *k
         // grids of 128-query blocks that leave the CUs one block each or fewer
         // (short sequences: config 3's 256) take 64-query blocks, two per CU
         const bool q64 = (long)grid.x * grid.y <= cu_count();
-        if (s.head_dim == 128 && dma_ok && q64)
-            hipLaunchKernelGGL(fa_fwd3_k<1>, dim3(grid.x, (s.n_q + 63) / 64), dim3(NT), 0, st, s,
-                               (const bf16 *)q, ldq, (const bf16 *)k, ldk, (const bf16 *)v, ldv, o,
-                               ldo, lse, ob, ldob);
-        else if (s.head_dim == 128 && dma_ok)
-            hipLaunchKernelGGL(fa_fwd3_k<2>, grid, dim3(NT), 0, st, s, (const bf16 *)q, ldq,
-                               (const bf16 *)k, ldk, (const bf16 *)v, ldv, o, ldo, lse, ob, ldob);
-        else if (s.head_dim == 128)
-            hipLaunchKernelGGL(fa_fwd_bf16_k<128>, grid, dim3(NT), 0, st, s, (const bf16 *)q, ldq,
-                               (const bf16 *)k, ldk, (const bf16 *)v, ldv, o, ldo, lse, ob, ldob);
-        else
-            hipLaunchKernelGGL(fa_fwd_bf16_k<64>, grid, dim3(NT), 0, st, s, (const bf16 *)q, ldq,
-                               (const bf16 *)k, ldk, (const bf16 *)v, ldv, o, ldo, lse, ob, ldob);
+        auto go = [&](auto kernel, dim3 gr) {
+            hipLaunchKernelGGL(kernel, gr, dim3(NT), 0, st, s, (const bf16 *)q, ldq, (const bf16 *)k, ldk,
+                               (const bf16 *)v, ldv, o, ldo, lse, ob, ldob);
+        };
+        const dim3 grid64(grid.x, (s.n_q + 63) / 64);
+        if (dma_ok && s.head_dim == 128) q64 ? go(fa_fwd3_k<1>, grid64) : go(fa_fwd3_k<2>, grid);
+        else if (dma_ok) q64 ? go(fa_fwd3_k<1, 64>, grid64) : go(fa_fwd3_k<2, 64>, grid);
+        else if (s.head_dim == 128) go(fa_fwd_bf16_k<128>, grid);
+        else go(fa_fwd_bf16_k<64>, grid);
     } else {
         if (s.head_dim > 64 * MAXE || ob) return hipErrorInvalidValue;
         if (fa_f32m_fwd(s, (const float *)q, ldq, (const float *)k, ldk, (const float *)v, ldv, o,
