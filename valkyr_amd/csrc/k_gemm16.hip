@@ -40,6 +40,8 @@ using T128x64s3 = Tile16<128, 64, 2, 2, 3>;
 // Few-tile products (plan_few): smaller tiles, split over K.
 using T64 = Tile16<64, 64, 2, 2>;
 using T32x64 = Tile16<32, 64, 1, 4>;  // K-major A only (a bf16 MN tile is 64 rows or 128 n)
+using T32 = Tile16<32, 32, 2, 2, 3>;  // fp32, whose products of few tiles are bound by the
+                                      // matrix cores of the CUs they reach
 // (Three slab buffers were measured slower for these tiles: the larger LDS
 // footprint drops a block per CU.  Staging the slabs through VGPRs two slabs
 // ahead, which doubles the time a load has to arrive without more LDS, was
@@ -48,7 +50,7 @@ using T32x64 = Tile16<32, 64, 1, 4>;  // K-major A only (a bf16 MN tile is 64 ro
 
 constexpr bool kUseKs2 = true;
 
-enum class Pick { Big, T128, T128x64, T128w8, T128x64ks2, T64, T32x64, T64ks2, T32x64ks2 };
+enum class Pick { Big, T128, T128x64, T128w8, T128x64ks2, T64, T32x64, T64ks2, T32x64ks2, T32, T32ks2 };
 struct Plan {
     Pick tile;
     int splits;
@@ -63,6 +65,7 @@ size_t ws_for(const Plan &p, const GemmShape &s) {
     case Pick::T128w8: return gemm16_ws_bytes<T128w8>(s, p.splits);
     case Pick::T64: return gemm16_ws_bytes<T64>(s, p.splits);
     case Pick::T32x64: return gemm16_ws_bytes<T32x64>(s, p.splits);
+    case Pick::T32: return gemm16_ws_bytes<T32>(s, p.splits);
     default: return gemm16_ws_bytes<T128x64>(s, p.splits);
     }
 }
@@ -119,6 +122,7 @@ Plan plan_few(const GemmShape &s, size_t ws_bytes, bool f32, bool mn_a, bool two
     tile(Pick::T128x64, Pick::T128x64ks2, 128, 64);
     tile(Pick::T64, Pick::T64ks2, 64, 64);
     if (f32 || !mn_a) tile(Pick::T32x64, Pick::T32x64ks2, 32, 64);
+    if (f32) tile(Pick::T32, Pick::T32ks2, 32, 32);
     return best;
 }
 
@@ -237,6 +241,8 @@ hipError_t run32(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e,
     case Pick::T32x64: return launch_gemm16<T32x64, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
     case Pick::T64ks2: return launch_gemm16_ks2<T64, LA, LB, Epi, true>(a, b, s, e, g, st);
     case Pick::T32x64ks2: return launch_gemm16_ks2<T32x64, LA, LB, Epi, true>(a, b, s, e, g, st);
+    case Pick::T32: return launch_gemm16<T32, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
+    case Pick::T32ks2: return launch_gemm16_ks2<T32, LA, LB, Epi, true>(a, b, s, e, g, st);
     default: return launch_gemm16<T128x64, LA, LB, Epi, true>(a, b, s, e, sk, g, st);
     }
 }
