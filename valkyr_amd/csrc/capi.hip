@@ -521,24 +521,62 @@ vkh_status vkh_linear_backward_dw_bf16(const void *dy, const void *x, float *dw,
     return linear(LinOp::TN, LinForm::BF16, dy, x, dw, M, N, K, "linear_backward_dw_bf16", S(stream));
 }
 
+// Scratch of a LoRA call: the stream's kept buffer, or stream-ordered memory where it is
+// larger than that keeps or the stream is being captured.
+extern "C++" {
+namespace {
+class LoraScratch {
+  public:
+    vkh_status acquire(size_t bytes, hipStream_t st) {
+        st_ = st;
+        if (bytes <= kLeaseMax && !capturing(st)) return lease_.acquire(bytes, st, (void **)&p);
+        note_allocation();
+        VKH_HIP(hipMallocAsync((void **)&p, bytes, st));
+        own_ = true;
+        return VKH_OK;
+    }
+    ~LoraScratch() {
+        if (own_) (void)hipFreeAsync(p, st_);
+    }
+    char *p = nullptr;
+
+  private:
+    ScratchLease lease_;
+    hipStream_t st_ = nullptr;
+    bool own_ = false;
+};
+}  // namespace
+}
+
+// The rank-r products go through the fp32 GEMMs (their few-tile plans split the long
+// sum; one block per column group walked it alone before, dA and dB 21 us each at 2048
+// tokens and 2560 columns), and the rank-r update rides in the base product's epilogue
+// instead of reading the output back (16 and 14 us): that layer, forward and backward
+// at rank 16, 213 -> 157 us.
 vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, const float *b,
                             float *y, float *inter, uint32_t M, uint32_t N, uint32_t K,
                             uint32_t r, float aor, uint32_t precision, vkh_stream stream) {
     CHECK_ARG(x && w && a && b && y && inter, "null pointer");
     CHECK_ARG(r > 0, "rank 0");
     const Precision pr = PR(precision);
+    const LinForm form = form_of(precision);
     hipStream_t st = S(stream);
-    VKH_TRY(linear(LinOp::NT, form_of(precision), x, w, y, M, N, K, "lora_forward", st));
-    // rank-r kernels (fp32 factors and products) where the shape allows
     LoraSegs sa, sb;
     sa.n = sb.n = 1;
     sa.s[0] = LoraSeg{0, (int)K, a, 1, (long)K, inter, (long)r};
     sb.s[0] = LoraSeg{0, (int)N, b, (long)r, 1, inter, (long)r};
-    if (lora_fast_ok(DType::F32, x, K, (int)r, sa) && lora_update_ok(y, N, (int)r, sb)) {
-        VKH_HIP(lora_rows(DType::F32, x, K, (int)M, (int)r, sa, 1.f, st));
-        VKH_HIP(lora_update(y, N, (int)M, (int)r, sb, aor, st));
+    // fp32 factors and products where the shape allows
+    if (lora_fast_ok(DType::F32, x, K, (int)r, sa) && lora_update_ok(y, N, (int)r, sb) &&
+        lin_lora_ok(LinOp::NT, form, M, N, K, sb, (int)r) && M) {
+        const size_t wsb = std::max(lin_ws_bytes(LinOp::NT, form, x, w, M, N, K), g32_ws_bytes_for(M, r, K));
+        LoraScratch sc;
+        if (wsb) VKH_TRY(sc.acquire(wsb, st));
+        const GemmWs ws{sc.p, wsb};
+        VKH_HIP(g32_nt(x, K, a, K, inter, r, M, r, K, nullptr, 0, 1.f, 0.f, ws, st));
+        VKH_HIP(lin_run(LinOp::NT, form, x, w, y, M, N, K, ws, st, &sb, (int)r, aor));
         return VKH_OK;
     }
+    VKH_TRY(linear(LinOp::NT, form, x, w, y, M, N, K, "lora_forward", st));
     VKH_HIP(gemm_nt(pr, matf(x, K), matf(a, K), inter, r, M, r, K, nullptr, 0, 1.f, 0.f, st));
     VKH_HIP(gemm_nt(pr, matf(inter, r), matf(b, r), y, N, M, N, r, nullptr, 0, aor, 1.f, st));
     return VKH_OK;
@@ -551,32 +589,38 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
     CHECK_ARG(dy && x && w && a && b && inter && dA && dB, "null pointer");
     CHECK_ARG(r > 0, "rank 0");
     const Precision pr = PR(precision);
+    const LinForm form = form_of(precision);
     hipStream_t st = S(stream);
-    float *dyB = nullptr;
-    vkh_status base = VKH_OK;  // of the base product
-    note_allocation();
-    VKH_HIP(hipMallocAsync((void **)&dyB, (size_t)M * r * 4 + 256, st));
     LoraSegs sb, sa, sdA, sdB;
     sb.n = sa.n = sdA.n = sdB.n = 1;
-    sb.s[0] = LoraSeg{0, (int)N, b, (long)r, 1, dyB, (long)r};
-    sa.s[0] = LoraSeg{0, (int)K, a, 1, (long)K, dyB, (long)r};
-    sdA.s[0] = LoraSeg{0, (int)K, nullptr, 1, 1, dyB, (long)r, dA, 1, (long)K};
+    sb.s[0] = LoraSeg{0, (int)N, b, (long)r, 1, (float *)inter, (long)r};
+    sa.s[0] = LoraSeg{0, (int)K, a, 1, (long)K, (float *)inter, (long)r};  // (u: dyB, set below)
+    sdA.s[0] = LoraSeg{0, (int)K, nullptr, 1, 1, (float *)inter, (long)r, dA, 1, (long)K};
     sdB.s[0] = LoraSeg{0, (int)N, nullptr, 1, 1, (float *)inter, (long)r, dB, (long)r, 1};
+    const size_t dyb_bytes = ((size_t)M * r * 4 + 511) / 256 * 256;
     if (lora_fast_ok(DType::F32, dy, N, (int)r, sb) && lora_fast_ok(DType::F32, x, K, (int)r, sdA) &&
-        lora_fast_ok(DType::F32, dy, N, (int)r, sdB) && (!dx || lora_update_ok(dx, K, (int)r, sa))) {
-        // rank-r kernels (fp32 factors and products)
-        hipError_t e = lora_rows(DType::F32, dy, N, (int)M, (int)r, sb, 1.f, st);
-        if (e == hipSuccess && dx) base = linear(LinOp::NN, form_of(precision), dy, w, dx, M, N, K, "lora_backward", st);
-        if (e == hipSuccess && base == VKH_OK && dx) e = lora_update(dx, K, (int)M, (int)r, sa, aor, st);
-        if (e == hipSuccess) e = lora_cols(DType::F32, x, K, (int)M, (int)r, sdA, aor, st);
-        if (e == hipSuccess) e = lora_cols(DType::F32, dy, N, (int)M, (int)r, sdB, aor, st);
-        (void)hipFreeAsync(dyB, st);
-        if (base != VKH_OK) return base;
-        if (e != hipSuccess) return hip_fail(e, "lora_backward");
+        lora_fast_ok(DType::F32, dy, N, (int)r, sdB) && M &&
+        (!dx || (lora_update_ok(dx, K, (int)r, sa) && lin_lora_ok(LinOp::NN, form, M, N, K, sa, (int)r)))) {
+        // fp32 factors and products
+        size_t wsb = std::max({g32_ws_bytes_for(M, r, N), g32_ws_bytes_for(r, K, M), g32_ws_bytes_for(N, r, M)});
+        if (dx) wsb = std::max(wsb, lin_ws_bytes(LinOp::NN, form, dy, w, M, N, K));
+        LoraScratch sc;
+        VKH_TRY(sc.acquire(dyb_bytes + wsb, st));
+        float *dyB = (float *)sc.p;
+        const GemmWs ws{wsb ? sc.p + dyb_bytes : nullptr, wsb};
+        sa.s[0].u = dyB;
+        VKH_HIP(g32_nn(dy, N, b, r, dyB, r, M, N, r, 1.f, 0.f, ws, st));
+        if (dx) VKH_HIP(lin_run(LinOp::NN, form, dy, w, dx, M, N, K, ws, st, &sa, (int)r, aor));
+        VKH_HIP(g32_tn(dyB, r, x, K, dA, K, M, r, K, aor, 0.f, ws, st));
+        VKH_HIP(g32_tn(dy, N, inter, r, dB, r, M, N, r, aor, 0.f, ws, st));
         return VKH_OK;
     }
+    float *dyB = nullptr;
+    note_allocation();
+    VKH_HIP(hipMallocAsync((void **)&dyB, dyb_bytes, st));
+    vkh_status base = VKH_OK;  // of the base product
     hipError_t e = gemm_nn(pr, matf(dy, N), matf(b, r), dyB, r, M, N, r, 1.f, 0.f, st);
-    if (e == hipSuccess && dx) base = linear(LinOp::NN, form_of(precision), dy, w, dx, M, N, K, "lora_backward", st);
+    if (e == hipSuccess && dx) base = linear(LinOp::NN, form, dy, w, dx, M, N, K, "lora_backward", st);
     if (e == hipSuccess && base == VKH_OK && dx) e = gemm_nn(pr, matf(dyB, r), matf(a, K), dx, K, M, r, K, aor, 1.f, st);
     if (e == hipSuccess) e = gemm_tn(pr, matf(dyB, r), matf(x, K), dA, K, M, r, K, aor, 0.f, st);
     if (e == hipSuccess) e = gemm_tn(pr, matf(dy, N), matf(inter, r), dB, r, M, N, r, aor, 0.f, st);

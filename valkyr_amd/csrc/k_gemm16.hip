@@ -774,8 +774,14 @@ hipError_t lin_pack(LinForm f, const void *a, long ra, long ca, void *da, const 
     return pack_rows<bf16, bf16>(s0, s1, st);
 }
 
+bool lin_lora_ok(LinOp op, LinForm f, int M, int N, int K, const LoraSegs &g, int r) {
+    const LinDims d = lin_dims(op, M, N, K);
+    auto fits = [&](long rows, long run) { return packed_bytes(f, rows, run) < (1ull << 31); };
+    return op != LinOp::TN && fits(d.ra, d.ca) && fits(d.rb, d.cb) && lora_epi_ok(g, r, d.s.N);
+}
+
 hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out, int M, int N, int K,
-                   const GemmWs &ws, hipStream_t st) {
+                   const GemmWs &ws, hipStream_t st, const LoraSegs *lora, int r, float alpha) {
     const LinDims d = lin_dims(op, M, N, K);
     const long v = chunk_elems(f);
     char *w = (char *)ws.p;
@@ -798,6 +804,14 @@ hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out
         // both aligned now; the zeros past a packed row's run are part of its chunks
         const Op16 oa{(const bf16 *)a, lda, (unsigned)ba}, ob{(const bf16 *)b, ldb, (unsigned)bb};
         const EpiStore ep{out, d.s.N, nullptr, 0, 1.f, 0.f};
+        if (lora) {
+            const EpiLora<EpiStore> el{ep, *lora, r, alpha};
+            if (f == LinForm::F32)
+                return op == LinOp::NT ? run32<Lay::K, Lay::K>(oa, ob, d.s, el, rest, st)
+                                       : run32<Lay::K, Lay::MN>(oa, ob, d.s, el, rest, st);
+            return op == LinOp::NT ? run16<Lay::K, Lay::K>(oa, ob, d.s, el, rest, st)
+                                   : run16<Lay::K, Lay::MN>(oa, ob, d.s, el, rest, st);
+        }
         if (f == LinForm::F32) {
             if (op == LinOp::NT) return run32<Lay::K, Lay::K>(oa, ob, d.s, ep, rest, st);
             if (op == LinOp::NN) return run32<Lay::K, Lay::MN>(oa, ob, d.s, ep, rest, st);
@@ -807,6 +821,7 @@ hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out
         if (op == LinOp::NN) return run16<Lay::K, Lay::MN>(oa, ob, d.s, ep, rest, st);
         return run16<Lay::MN, Lay::MN>(oa, ob, d.s, ep, rest, st);
     }
+    if (lora) return hipErrorInvalidValue;  // lin_lora_ok does not hold
     if (f == LinForm::F32) {
         const float *x = (const float *)a, *y = (const float *)b;
         if (op == LinOp::NT) return g32_nt(x, lda, y, ldb, out, N, M, N, K, nullptr, 0, 1.f, 0.f, rest, st);

@@ -101,8 +101,13 @@ inline long lin_packed_ld(LinForm f, long run) {
     const long v = f == LinForm::F32 ? 4 : 8;
     return (run + v - 1) / v * v;
 }
+// lora (NT and NN, where lin_lora_ok): alpha U_s F_s^T of its adapters added in the
+// epilogue, as lora_update would.
+struct LoraSegs;
 hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out, int M, int N, int K,
-                   const GemmWs &ws, hipStream_t st);
+                   const GemmWs &ws, hipStream_t st, const LoraSegs *lora = nullptr, int r = 0,
+                   float alpha = 0.f);
+bool lin_lora_ok(LinOp op, LinForm f, int M, int N, int K, const LoraSegs &g, int r);
 
 // ── LoRA rank-r products (k_lora.hip) ───────────────────────────────────
 // One adapter of a launch: its columns [col, col + ncols) of the shared X
