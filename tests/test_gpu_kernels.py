@@ -1108,3 +1108,52 @@ def test_flash_attention_bf16_full_size_invariants():
         for i, j in enumerate(keys):
             assert rel_l2(dv_ref[i], dv5[b, j, kv]) < 1e-2, ("dV", b, kv, j)
             assert rel_l2(dk_ref[i], dk5[b, j, kv]) < 1e-2, ("dK", b, kv, j)
+
+
+@pytest.mark.parametrize("call", ["fp32", "mixed", "bf16", "lora fp32", "lora mixed"])
+def test_linear_products_on_a_captured_stream(call):
+    """A few-tile product and a LoRA layer recorded into a graph on a stream that has run
+    nothing yet: the recording succeeds (no scratch of the stream is taken), and each
+    replay gives the eager call's values up to the order of fp32 sums (2 sqrt(K) 2^-23,
+    both sides in different splits), also after a larger eager call on that stream."""
+    import ctypes
+
+    from valkyr_amd import kernels as K
+    from valkyr_amd import lib
+    from valkyr_amd.device import Stream
+
+    note(f"captured {call}")
+    hip = lib()  # the runtime that the library is linked with
+    M, N, Kd, r = 16, 1024, 3072, 16
+    rng = np.random.default_rng(5)
+    x, w, a, b = (rng.standard_normal(s, dtype=np.float32) for s in ((M, Kd), (N, Kd), (r, Kd), (N, r)))
+    if call == "bf16":
+        (bx, _), (bw, _) = bf16_dev(x), bf16_dev(w)
+    else:
+        bx, bw, ba, bb = dev(x), dev(w), dev(a), dev(b)
+    inter, st = zeros(M * r), Stream()
+
+    def run(y, stream, n=N):
+        if call == "bf16":
+            K.matmul_nt_bf16(bx, bw, y, M, n, Kd, stream=stream)
+        elif call.startswith("lora"):
+            K.lora_forward(bx, bw, ba, bb, y, inter, M, n, Kd, r, 0.5, int(call == "lora mixed"), stream=stream)
+        else:
+            K.matmul_nt(bx, bw, y, M, n, Kd, int(call == "mixed"), stream=stream)
+
+    eager, y, other = zeros(M * N), zeros(M * N), zeros(M * N)
+    run(eager, Stream())
+    ref = host(eager)
+    graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(st.handle, 0) == 0
+    run(y, st)
+    assert hip.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        y.upload(np.zeros(M * N, np.float32))
+        assert hip.hipGraphLaunch(ex, st.handle) == 0
+        st.synchronize()
+        assert rel_l2(ref, host(y)) < 2 * math.sqrt(Kd) * 2.0 ** -23
+        run(other, st, N - 64)
+        st.synchronize()
+    assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0

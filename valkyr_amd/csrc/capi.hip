@@ -424,14 +424,17 @@ static bool capturing(hipStream_t st) {
 // One contraction of a linear layer.  Operands that need a packed copy (fp32
 // operands in the bf16 precision; rows that are not whole 16-byte chunks) go
 // through the workspace to the DMA-staged kernels; while the stream is being
-// captured they take the generic kernel, which needs none.  Against the generic
+// captured they take the generic kernel, and the others a plan without a split:
+// a graph outlives the call, so it holds no pointer into the stream's scratch
+// (which a later call may replace).  Against the generic
 // kernel, forward / dx / dW: 2048 tokens, 2560 x 2560, fp32 operands in bf16
 // products 55 / 55 / 63 us (645 / 443 / 351); bf16 operands of 2000 x 4100 x 4099
 // 156 / 143 / 117 us (455 / 638 / 533); fp32 of 1000 x 1500 x 3001 131 / 130 /
 // 117 us (205 / 156 / 211); 16 tokens, 1024 x 1024 mixed 15 / 15 / 8 us (41 / 29 / 7).
 static vkh_status linear(LinOp op, LinForm f, const void *a, const void *b, float *out, uint32_t M,
                          uint32_t N, uint32_t K, const char *what, hipStream_t st) {
-    if (!M || !N || !K || (lin_packs(op, f, a, b, M, N, K) && capturing(st))) {
+    const bool captured = capturing(st);
+    if (!M || !N || !K || (captured && lin_packs(op, f, a, b, M, N, K))) {
         const Precision pr = f == LinForm::F32 ? Precision::FP32 : Precision::BF16;
         const DType dt = f == LinForm::BF16 ? DType::BF16 : DType::F32;
         const Mat ma{a, (long)(op == LinOp::NT ? K : N), dt}, mb{b, (long)K, dt};
@@ -440,7 +443,7 @@ static vkh_status linear(LinOp op, LinForm f, const void *a, const void *b, floa
         else VKH_HIP(gemm_tn(pr, ma, mb, out, K, M, N, K, 1.f, 0.f, st));
         return VKH_OK;
     }
-    return with_ws(lin_ws_bytes(op, f, a, b, M, N, K), st, what, [&](const GemmWs &ws) {
+    return with_ws(captured ? 0 : lin_ws_bytes(op, f, a, b, M, N, K), st, what, [&](const GemmWs &ws) {
         return lin_run(op, f, a, b, out, M, N, K, ws, st);
     });
 }
@@ -522,14 +525,14 @@ vkh_status vkh_linear_backward_dw_bf16(const void *dy, const void *x, float *dw,
 }
 
 // Scratch of a LoRA call: the stream's kept buffer, or stream-ordered memory where it is
-// larger than that keeps or the stream is being captured.
+// larger than that keeps.
 extern "C++" {
 namespace {
 class LoraScratch {
   public:
     vkh_status acquire(size_t bytes, hipStream_t st) {
         st_ = st;
-        if (bytes <= kLeaseMax && !capturing(st)) return lease_.acquire(bytes, st, (void **)&p);
+        if (bytes <= kLeaseMax) return lease_.acquire(bytes, st, (void **)&p);
         note_allocation();
         VKH_HIP(hipMallocAsync((void **)&p, bytes, st));
         own_ = true;
@@ -552,7 +555,8 @@ class LoraScratch {
 // sum; one block per column group walked it alone before, dA and dB 21 us each at 2048
 // tokens and 2560 columns), and the rank-r update rides in the base product's epilogue
 // instead of reading the output back (16 and 14 us): that layer, forward and backward
-// at rank 16, 213 -> 157 us.
+// at rank 16, 213 -> 157 us.  A captured stream (no scratch) and operands of 2 GiB keep
+// the row and update kernels, with fp32 factors and products as well.
 vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, const float *b,
                             float *y, float *inter, uint32_t M, uint32_t N, uint32_t K,
                             uint32_t r, float aor, uint32_t precision, vkh_stream stream) {
@@ -566,8 +570,13 @@ vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, cons
     sa.s[0] = LoraSeg{0, (int)K, a, 1, (long)K, inter, (long)r};
     sb.s[0] = LoraSeg{0, (int)N, b, (long)r, 1, inter, (long)r};
     // fp32 factors and products where the shape allows
-    if (lora_fast_ok(DType::F32, x, K, (int)r, sa) && lora_update_ok(y, N, (int)r, sb) &&
-        lin_lora_ok(LinOp::NT, form, M, N, K, sb, (int)r) && M) {
+    if (lora_fast_ok(DType::F32, x, K, (int)r, sa) && lora_update_ok(y, N, (int)r, sb) && M) {
+        if (capturing(st) || !lin_lora_ok(LinOp::NT, form, M, N, K, sb, (int)r)) {
+            VKH_TRY(linear(LinOp::NT, form, x, w, y, M, N, K, "lora_forward", st));
+            VKH_HIP(lora_rows(DType::F32, x, K, (int)M, (int)r, sa, 1.f, st));
+            VKH_HIP(lora_update(y, N, (int)M, (int)r, sb, aor, st));
+            return VKH_OK;
+        }
         const size_t wsb = std::max(lin_ws_bytes(LinOp::NT, form, x, w, M, N, K), g32_ws_bytes_for(M, r, K));
         LoraScratch sc;
         if (wsb) VKH_TRY(sc.acquire(wsb, st));
@@ -598,9 +607,10 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
     sdA.s[0] = LoraSeg{0, (int)K, nullptr, 1, 1, (float *)inter, (long)r, dA, 1, (long)K};
     sdB.s[0] = LoraSeg{0, (int)N, nullptr, 1, 1, (float *)inter, (long)r, dB, (long)r, 1};
     const size_t dyb_bytes = ((size_t)M * r * 4 + 511) / 256 * 256;
-    if (lora_fast_ok(DType::F32, dy, N, (int)r, sb) && lora_fast_ok(DType::F32, x, K, (int)r, sdA) &&
-        lora_fast_ok(DType::F32, dy, N, (int)r, sdB) && M &&
-        (!dx || (lora_update_ok(dx, K, (int)r, sa) && lin_lora_ok(LinOp::NN, form, M, N, K, sa, (int)r)))) {
+    const bool fast = lora_fast_ok(DType::F32, dy, N, (int)r, sb) && lora_fast_ok(DType::F32, x, K, (int)r, sdA) &&
+                      lora_fast_ok(DType::F32, dy, N, (int)r, sdB) && M &&
+                      (!dx || lora_update_ok(dx, K, (int)r, sa));
+    if (fast && !capturing(st) && (!dx || lin_lora_ok(LinOp::NN, form, M, N, K, sa, (int)r))) {
         // fp32 factors and products
         size_t wsb = std::max({g32_ws_bytes_for(M, r, N), g32_ws_bytes_for(r, K, M), g32_ws_bytes_for(N, r, M)});
         if (dx) wsb = std::max(wsb, lin_ws_bytes(LinOp::NN, form, dy, w, M, N, K));
@@ -619,11 +629,21 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
     note_allocation();
     VKH_HIP(hipMallocAsync((void **)&dyB, dyb_bytes, st));
     vkh_status base = VKH_OK;  // of the base product
-    hipError_t e = gemm_nn(pr, matf(dy, N), matf(b, r), dyB, r, M, N, r, 1.f, 0.f, st);
-    if (e == hipSuccess && dx) base = linear(LinOp::NN, form, dy, w, dx, M, N, K, "lora_backward", st);
-    if (e == hipSuccess && base == VKH_OK && dx) e = gemm_nn(pr, matf(dyB, r), matf(a, K), dx, K, M, r, K, aor, 1.f, st);
-    if (e == hipSuccess) e = gemm_tn(pr, matf(dyB, r), matf(x, K), dA, K, M, r, K, aor, 0.f, st);
-    if (e == hipSuccess) e = gemm_tn(pr, matf(dy, N), matf(inter, r), dB, r, M, N, r, aor, 0.f, st);
+    hipError_t e;
+    if (fast) {
+        for (LoraSegs *g : {&sb, &sa, &sdA}) g->s[0].u = dyB;
+        e = lora_rows(DType::F32, dy, N, (int)M, (int)r, sb, 1.f, st);
+        if (e == hipSuccess && dx) base = linear(LinOp::NN, form, dy, w, dx, M, N, K, "lora_backward", st);
+        if (e == hipSuccess && base == VKH_OK && dx) e = lora_update(dx, K, (int)M, (int)r, sa, aor, st);
+        if (e == hipSuccess) e = lora_cols(DType::F32, x, K, (int)M, (int)r, sdA, aor, st);
+        if (e == hipSuccess) e = lora_cols(DType::F32, dy, N, (int)M, (int)r, sdB, aor, st);
+    } else {
+        e = gemm_nn(pr, matf(dy, N), matf(b, r), dyB, r, M, N, r, 1.f, 0.f, st);
+        if (e == hipSuccess && dx) base = linear(LinOp::NN, form, dy, w, dx, M, N, K, "lora_backward", st);
+        if (e == hipSuccess && base == VKH_OK && dx) e = gemm_nn(pr, matf(dyB, r), matf(a, K), dx, K, M, r, K, aor, 1.f, st);
+        if (e == hipSuccess) e = gemm_tn(pr, matf(dyB, r), matf(x, K), dA, K, M, r, K, aor, 0.f, st);
+        if (e == hipSuccess) e = gemm_tn(pr, matf(dy, N), matf(inter, r), dB, r, M, N, r, aor, 0.f, st);
+    }
     (void)hipFreeAsync(dyB, st);
     if (base != VKH_OK) return base;
     if (e != hipSuccess) return hip_fail(e, "lora_backward");
