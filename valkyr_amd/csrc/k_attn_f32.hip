@@ -244,7 +244,9 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
 // total work, not by this kernel's span.)
 // QKE: dK leaves through RoPE^T and the K-RMSNorm backward (p.qk), each block
 // writing its k-gain partial to p.qk.pk[block].
-template <int HD, bool QKE, bool RAG = false>
+// ACC: the rounding of the per-row kernels (head_dot); whole tiles that are only split
+// keep the rounding of their unsplit form.
+template <int HD, bool QKE, bool RAG = false, bool ACC = RAG>
 __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtrs p, bool zz) {
     static_assert(!QKE || (HD == 128 && !RAG), "the fused q/k epilogue takes 128-wide head rows");
     constexpr int P = HD + 4, NU = HD / 16;
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
         const float *vr = V + ((long)b * s.n_kv + kl) * p.ldv + kvh * HD + 4 * g;
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            kf[u] = f4_scale(f4(kr + 16 * u), RAG ? 1.f : c2);
+            kf[u] = f4_scale(f4(kr + 16 * u), ACC ? 1.f : c2);
             vf[u] = f4(vr + 16 * u);
         }
     }
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
     auto store = [&](int buf) {
         tq.store(Qs[buf], tid);
         tdo.store(Os[buf], tid);
-        if (tid < FT) Ls[buf][tid] = RAG ? stat : stat * F_LOG2E;
+        if (tid < FT) Ls[buf][tid] = ACC ? stat : stat * F_LOG2E;
         else if (tid < 2 * FT) Dl[buf][tid - FT] = stat;
     };
     f32x4 dvt[NU], dkt[NU];  // dV^T / dK^T[16 j + 4 g + r][ki]
@@ -330,8 +332,8 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
             sa[qs] = da[qs] = f32x4{0, 0, 0, 0};
             live[qs] = !s.causal || kw <= q0 + 16 * qs + 15 + shift;  // wave-uniform
             if (live[qs]) {
-                sa[qs] = head_dot<NU, RAG>(Ql + (16 * qs + c) * P + 4 * g, kf);
-                da[qs] = head_dot<NU, RAG>(Ol + (16 * qs + c) * P + 4 * g, vf);
+                sa[qs] = head_dot<NU, ACC>(Ql + (16 * qs + c) * P + 4 * g, kf);
+                da[qs] = head_dot<NU, ACC>(Ol + (16 * qs + c) * P + 4 * g, vf);
             }
         }
         // P = exp2(S c - lse), dS = P (dP - D); zero above the diagonal
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int qr = 16 * qs + 4 * g + r;
-                float pv = RAG ? expf(fmaf(sa[qs][r], s.inv_sqrt_dim, -Ls[buf][qr]))
+                float pv = ACC ? expf(fmaf(sa[qs][r], s.inv_sqrt_dim, -Ls[buf][qr]))
                                : __builtin_amdgcn_exp2f(sa[qs][r] - Ls[buf][qr]);
                 const bool past = RAG && q0 + qr >= s.n_q;  // a zero row (against an infinite K or V: NaN)
                 if ((s.causal && ki > q0 + qr + shift) || past) pv = 0.f;
@@ -569,6 +571,9 @@ bool fa_f32m_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     if (p.qk_fp32) go(fa_bwd_dkv_f32m_k<128, true>);
     else if (whole_tiles(s) && q.split_parts == 1)
         s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false>) : go(fa_bwd_dkv_f32m_k<64, false>);
+    else if (whole_tiles(s))
+        s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false, true, false>)
+                          : go(fa_bwd_dkv_f32m_k<64, false, true, false>);
     else
         s.head_dim == 128 ? go(fa_bwd_dkv_f32m_k<128, false, true>) : go(fa_bwd_dkv_f32m_k<64, false, true>);
     if (q.split_parts > 1) fa_dkv_sum(s, q, st);
