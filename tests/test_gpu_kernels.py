@@ -880,6 +880,60 @@ def test_flash_attention_bf16_mfma(case):
     _check_from_o(p, qb, kb, vb, o, dob16, lse_r, dO.size, ws)
 
 
+@pytest.mark.parametrize("hd,n", [(128, 512), (64, 512), (128, 1001), (64, 4096)])
+def test_flash_attention_bf16_forward_rows_are_independent(hd, n):
+    """A row's O and LSE have the same bits whatever the other queries of its wave hold:
+    every 16th query is replaced by one with other maxima."""
+    from valkyr_amd import kernels as K
+
+    H = 2
+    note(f"fa bf16 forward row independence hd={hd} n={n}")
+    q = O.normal(n * H * hd, 61).reshape(n, H, hd)
+    other = q.copy()
+    other[15::16] = 3 * O.normal(other[15::16].size, 62).reshape(other[15::16].shape)
+    kb, _ = bf16_dev(O.normal(n * H * hd, 63))
+    vb, _ = bf16_dev(O.normal(n * H * hd, 64))
+    p = K.attn_params(n, n, H, H, hd, True, 1, K.BF16)
+
+    def forward(q):
+        qb, _ = bf16_dev(q.reshape(-1))
+        o, lse = zeros(n * H * hd), zeros(n * H)
+        K.fa_forward(p, qb, kb, vb, o, lse)
+        return host(o).reshape(n, H, hd), host(lse).reshape(n, H)
+
+    kept = np.arange(n) % 16 != 15
+    (o, lse), (o2, lse2) = forward(q), forward(other)
+    assert np.all(np.isfinite(o)) and np.all(np.isfinite(lse))
+    note(f"  rows that differ: LSE {np.flatnonzero((lse != lse2)[kept].any(1))[:9]}, O {np.flatnonzero((o != o2)[kept].any((1, 2)))[:9]}")
+    assert np.array_equal(lse[kept], lse2[kept]) and np.array_equal(o[kept], o2[kept])
+
+
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 1.5])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_flash_attention_bf16_forward_scales(hd, scale):
+    """Any score scale, negative and zero too, against float64 on the bf16 operands.
+    O is off by the rounding of P (2^-9 of each term); LSE by the fp32 scores' own error,
+    at most hd roundings of partial sums below 32: hd 32 2^-25 |scale|."""
+    from valkyr_amd import kernels as K
+
+    n, H = 200, 2
+    note(f"fa bf16 forward scale={scale} hd={hd}")
+    qb, q = bf16_dev(O.normal(n * H * hd, 65))
+    kb, k = bf16_dev(O.normal(n * H * hd, 66))
+    vb, v = bf16_dev(O.normal(n * H * hd, 67))
+    q, k, v = (t.reshape(n, H, hd).astype(np.float64).transpose(1, 0, 2) for t in (q, k, v))
+    s = scale * q @ k.transpose(0, 2, 1)
+    s[:, np.triu(np.ones((n, n), bool), 1)] = -np.inf
+    m = s.max(-1, keepdims=True)
+    e = np.exp(s - m)
+    lse_ref = (m + np.log(e.sum(-1, keepdims=True)))[..., 0].T
+    o_ref = (e / e.sum(-1, keepdims=True) @ v).transpose(1, 0, 2)
+    o, lse = zeros(n * H * hd), zeros(n * H)
+    K.fa_forward(K.attn_params(n, n, H, H, hd, True, 1, K.BF16, scale), qb, kb, vb, o, lse)
+    assert rel_l2(o_ref, host(o)) < 2.0 ** -8
+    assert np.abs(host(lse).reshape(n, H) - lse_ref).max() < 2.0 ** -20 + 16 * abs(scale) * hd * 2.0 ** -24
+
+
 @pytest.mark.parametrize("case", [  # (n, H, Hkv, hd, causal, B)
     (1, 2, 1, 128, True, 2), (33, 3, 1, 128, True, 2), (129, 4, 4, 128, True, 1),
     (257, 8, 2, 128, True, 1), (130, 4, 4, 128, False, 2), (95, 5, 5, 128, False, 1),

@@ -1839,10 +1839,10 @@ VKH_DEV float xrow_sum(float v) {
 // Causal q tiles go heaviest first (a zigzag order, zigzag in common.hpp,
 // measured 77.6 against 78.9 us at config 4's 512-block grid: within noise).
 // Bound by the vector ALU's softmax beside the matrix cores (about 1.7 of its cycles to
-// 1 of theirs before): the scale is folded into one fma per score, masked scores need no
-// test of their own (exp2 of -inf is 0), the row sum stays per lane until the end, the
-// row maximum crosses lanes by permlane swaps, and the accumulators are rescaled only in
-// tiles where a row of the wave got a new maximum.  HDR = 64: 64-wide heads in the same
+// 1 of theirs before): masked scores need no test of their own (exp2 of -inf is 0), row
+// maxima and sums cross lanes by permlane swaps, and the accumulators are rescaled only in
+// tiles where a row of the wave got a new maximum (by exactly 1 in the wave's other rows:
+// a row's bits do not depend on its neighbours).  HDR = 64: 64-wide heads in the same
 // 128-wide LDS rows (as in the backward).
 template <int QS, int HDR = 128>
 __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, long ldq,
@@ -1865,9 +1865,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
     const int q0 = qt * FBM, qw0 = q0 + wave * 16 * QS;
     const int off = s.n_kv - s.n_q;
     const bf16 *qb = q + (long)b * s.n_q * ldq + h * HDR;
-    // scores are compared unscaled: a negative scale flips Q's signs (exact)
-    const float c2 = fmaxf(fabsf(s.inv_sqrt_dim) * LOG2E, 1e-37f);
-    const bool neg = s.inv_sqrt_dim < 0.f;
+    const float c2 = s.inv_sqrt_dim * LOG2E;
 
     bf16x8 qf[QS][DSR];
 #pragma unroll
@@ -1875,10 +1873,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
         const int qr = qw0 + 16 * qs + c16;
 #pragma unroll
         for (int ds = 0; ds < DSR; ++ds)
-        {
             qf[qs][ds] = qr < s.n_q ? ld_frag(qb + (long)qr * ldq + 32 * ds + 8 * g) : bf16x8{};
-            if (neg) qf[qs][ds] = -qf[qs][ds];
-        }
     }
     wait_vm0();  // Q fragments are in registers before any DMA is queued
     f32x4 oacc[DSUBR][QS];
@@ -1940,6 +1935,8 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
 #pragma unroll
         for (int qs = 0; qs < QS; ++qs) {
             const int qa = qw0 + 16 * qs + c16;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) st[ks][qs] *= c2;
             if (edge) {
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks)
@@ -1955,10 +1952,10 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
 #pragma unroll
                 for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[ks][qs][r]);
             const float mn = fmaxf(m[qs], xrow_max(mt));
-            const float ms = mn == -INFINITY ? 0.f : mn * c2;  // no visible key yet: P = 0
+            const float ms = mn == -INFINITY ? 0.f : mn;  // no visible key yet: P = 0
+            float so = 1.f;
             if (__any(mn != m[qs])) {
-                const float so = __builtin_amdgcn_exp2f(fmaf(m[qs], c2, -ms));
-                l[qs] *= so;
+                so = __builtin_amdgcn_exp2f(m[qs] - ms);
 #pragma unroll
                 for (int i = 0; i < DSUBR; ++i) oacc[i][qs] *= so;
                 m[qs] = mn;
@@ -1968,11 +1965,11 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
             for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float pv = __builtin_amdgcn_exp2f(fmaf(st[ks][qs][r], c2, -ms));
+                    const float pv = __builtin_amdgcn_exp2f(st[ks][qs][r] - ms);
                     st[ks][qs][r] = pv;
                     lt += pv;
                 }
-            l[qs] += lt;
+            l[qs] = fmaf(l[qs], so, xrow_sum(lt));
             pf[qs][0] = frag_acc(st[0][qs], st[1][qs]);
             pf[qs][1] = frag_acc(st[2][qs], st[3][qs]);
         }
@@ -1988,9 +1985,8 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
 #pragma unroll
     for (int qs = 0; qs < QS; ++qs) {
         const int qa = qw0 + 16 * qs + c16;
-        const float lq = xrow_sum(l[qs]);
         if (qa >= s.n_q) continue;
-        const float inv = lq > 0.f ? 1.0f / lq : 0.f;
+        const float inv = l[qs] > 0.f ? 1.0f / l[qs] : 0.f;
         float *orow = o + ((long)b * s.n_q + qa) * ldo + h * HDR;
 #pragma unroll
         for (int i = 0; i < DSUBR; ++i) {
@@ -2005,7 +2001,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd3_k(AttnShape s, const bf16 *q, 
         }
         if (lse && g == 0)
             lse[((long)b * s.n_q + qa) * s.n_heads + h] =
-                lq > 0.f ? fmaf(m[qs], c2, log2f(lq)) * LN2 : -INFINITY;
+                l[qs] > 0.f ? (m[qs] + log2f(l[qs])) * LN2 : -INFINITY;
     }
 }
 
