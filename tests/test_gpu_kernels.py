@@ -777,32 +777,64 @@ def test_flash_attention_fp32_ragged_lengths(case):
     test_flash_attention_fp32(case)
 
 
-def test_flash_attention_fp32_ragged_masked_rows():
-    """A query whose scores are all -inf (keys of -inf against a positive query, as an
-    additive mask leaves them) gets O = 0, LSE = -inf, and no gradient flows from it."""
+def _fa_f32_all(p, n, H, q, k, v, do, lse=None, d=None):
+    """O, LSE, D, dQ, dK, dV of the four fp32 calls (LSE and D given: the backward's)."""
     from valkyr_amd import kernels as K
 
-    n, H, hd = 37, 2, 64
-    q, k = O.normal(n * H * hd, 11), np.zeros((n, H, hd), np.float32)
-    q = q.reshape(n, H, hd)
-    q[:, :, 0] = 1.0
-    k[:5, :, 0] = -np.inf
-    v, do = O.normal(n * H * hd, 12), O.normal(n * H * hd, 13)
-    p = K.attn_params(n, n, H, H, hd, True, 1, K.F32)
     bq, bk, bv, bdo = dev(q), dev(k), dev(v), dev(do)
-    bo, blse, bd = zeros(n * H * hd), zeros(n * H), zeros(n * H)
-    bdk, bdv = zeros(n * H * hd), zeros(n * H * hd)
+    bo, blse, bd = zeros(q.size), zeros(n * H), zeros(n * H)
+    bdq, bdk, bdv = zeros(q.size), zeros(k.size), zeros(v.size)
     K.fa_forward(p, bq, bk, bv, bo, blse)
     K.fa_bw_d(p, bo, bdo, bd)
-    K.fa_bw_dkv(p, bq, bk, bv, bdo, blse, bd, bdk, bdv)
-    o, lse = host(bo).reshape(n, H, hd), host(blse).reshape(n, H)
-    assert np.all(o[:5] == 0) and np.all(lse[:5] == -np.inf)
+    out = [host(bo), host(blse), host(bd)]
+    bl, bd = (dev(lse), dev(d)) if lse is not None else (blse, bd)
+    K.fa_bw_dkv(p, bq, bk, bv, bdo, bl, bd, bdk, bdv)
+    K.fa_bw_dq(p, bq, bk, bv, bdo, bl, bd, bdq)
+    out += [host(bdq), host(bdk), host(bdv)]
+    hd = q.shape[-1]
+    return [t.reshape(n, H) if i in (1, 2) else t.reshape(-1, H, hd) for i, t in enumerate(out)]
+
+
+@pytest.mark.parametrize("n,hd", [(37, 64), (100, 128)])
+def test_flash_attention_fp32_ragged_masked_rows(n, hd):
+    """A query whose scores are all -inf (keys of -inf against a positive query, as an
+    additive mask leaves them) gets O = 0, LSE = -inf and dQ = 0, and no gradient flows
+    from it to K and V: their gradients are those of a call whose dO is 0 there."""
+    from valkyr_amd import kernels as K
+
+    H = 2
+    note(f"fa fp32 masked rows n={n} hd={hd}")
+    q, k = O.normal(n * H * hd, 11).reshape(n, H, hd), np.zeros((n, H, hd), np.float32)
+    q[:, :, 0] = 1.0
+    k[:5, :, 0] = -np.inf
+    v, do = (O.normal(n * H * hd, i).reshape(n, H, hd) for i in (12, 13))
+    p = K.attn_params(n, n, H, H, hd, True, 1, K.F32)
+    o, lse, d, dq, dk, dv = _fa_f32_all(p, n, H, q, k, v, do)
+    assert np.all(o[:5] == 0) and np.all(lse[:5] == -np.inf) and np.all(dq[:5] == 0)
     # keys of one finite score: O is the mean of the visible values, LSE = log(count)
     cnt = np.arange(1, n - 4)
-    ref = np.cumsum(v.reshape(n, H, hd)[5:].astype(np.float64), 0) / cnt[:, None, None]
+    ref = np.cumsum(v[5:].astype(np.float64), 0) / cnt[:, None, None]
     assert rel_l2(ref, o[5:]) < 1e-6 and np.allclose(lse[5:], np.log(cnt)[:, None], atol=1e-6)
-    dv = host(bdv).reshape(n, H, hd)
-    assert np.all(np.isfinite(dv)) and np.all(dv[:5] == 0)
+    # P = 1 / count for visible finite keys, dS = P (dO v - D)
+    do64, v64, q64 = (t.astype(np.float64) for t in (do, v, q))
+    pr = np.tril(np.ones((n, n)))
+    pr[:, :5] = 0
+    pr = pr / np.maximum(pr.sum(1, keepdims=True), 1)
+    ds = pr[None] * (np.einsum("qhd,khd->hqk", do64, v64) - (do64 * o).sum(-1).T[:, :, None])
+    assert rel_l2(np.einsum("qk,qhd->khd", pr, do64), dv) < 1e-5 and np.all(dv[:5] == 0)
+    assert rel_l2(np.einsum("hqk,qhd->khd", ds, q64) / math.sqrt(hd), dk) < 1e-5 and np.all(dk[:5] == 0)
+    # the infinity in one query row: the other rows' gradients, finite
+    q[:, :, 0], k = 1.0, O.normal(n * H * hd, 14).reshape(n, H, hd)
+    k[:, :, 0], do0 = 1.0, do.copy()
+    do0[7] = 0
+    want = _fa_f32_all(p, n, H, q, k, v, do0)
+    for bad in (-np.inf, np.nan):
+        q[7, :, 0] = bad
+        o, lse, d, dq, dk, dv = _fa_f32_all(p, n, H, q, k, v, do)
+        rest = np.arange(n) != 7
+        assert np.all(lse[7] == -np.inf) and np.all(dq[7] == 0)
+        assert rel_l2(want[3][rest], dq[rest]) < 1e-6
+        assert rel_l2(want[4], dk) < 1e-6 and rel_l2(want[5], dv) < 1e-6
 
 
 @pytest.mark.parametrize("hd,rows", [(128, 4 * 2048 * 16), (64, 3 * 100 * 4)])

@@ -76,6 +76,15 @@ struct Tile {
             v[i] = r < rows ? f4(base + (long)r * ld + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
+    // a stored tile's rows that `out` names become zero
+    template <class Out>
+    static VKH_DEV void drop(float *lds, int tid, Out out) {
+#pragma unroll
+        for (int i = 0; i < N4; ++i) {
+            const int x = tid + NT * i, r = x / (HD / 4), c = x % (HD / 4);
+            if (out(r)) *reinterpret_cast<float4 *>(lds + r * P + 4 * c) = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
     VKH_DEV void store(float *lds, int tid) const {
 #pragma unroll
         for (int i = 0; i < N4; ++i) {
@@ -88,7 +97,9 @@ struct Tile {
 // RAG (all three kernels): any n_q and n_kv, a causal mask also with n_q < n_kv
 // (query q sees keys up to q + n_kv - n_q).  Rows past the end load as zero and are
 // not stored, their scores are masked to exact zeros, and a row whose scores are all
-// -inf gets O = 0 and LSE = -inf (backward: no gradient), as the per-row kernels do.
+// -inf gets O = 0 and LSE = -inf, as one with a NaN among its scores gets LSE = -inf.
+// The backward leaves rows of LSE = -inf out, as the per-row kernels do: their staged Q
+// and dO become zeros (0 times an infinity is NaN) and their dQ is zero.
 // Bound by the matrix cores of the few CUs a short sequence reaches; against the
 // per-row kernels (one wave a row, a dot product at a time).  They round as those did:
 // the contraction over the head runs in a chain per 16 columns and a tree (one chain of
@@ -218,13 +229,15 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
     }
     l = xsum(l);
     if (RAG && qi >= s.n_q) return;
-    const float inv = RAG && l == 0.f ? 0.f : 1.0f / l;
+    const bool dead = RAG && !(l > 0.f);  // every score -inf, or a NaN among them
+    const float inv = dead ? 0.f : 1.0f / l;
     float *orow = o + ((long)b * s.n_q + qi) * ldo + h * HD + 4 * g;
 #pragma unroll
     for (int j = 0; j < NU; ++j)
         *reinterpret_cast<float4 *>(orow + 16 * j) =
             make_float4(ot[j][0] * inv, ot[j][1] * inv, ot[j][2] * inv, ot[j][3] * inv);
-    if (lse && g == 0) lse[((long)b * s.n_q + qi) * s.n_heads + h] = RAG ? m + logf(l) : (m + log2f(l)) * F_LN2;
+    if (lse && g == 0)
+        lse[((long)b * s.n_q + qi) * s.n_heads + h] = dead ? -INFINITY : RAG ? m + logf(l) : (m + log2f(l)) * F_LN2;
 }
 
 // ── dK / dV: block = 64 keys of one (sequence, KV head) ─────────────────
@@ -252,6 +265,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
     constexpr int P = HD + 4, NU = HD / 16;
     __shared__ __attribute__((aligned(16))) float Qs[2][FT * P], Os[2][FT * P];
     __shared__ float Ls[2][FT], Dl[2][FT];
+    __shared__ int any_out[2];  // RAG: a row of the tile has LSE = -inf
     const int kvh = blockIdx.x % s.n_kv_heads, b = blockIdx.x / s.n_kv_heads;
     const int tid = threadIdx.x, lane = tid % 64, g = lane / 16, c = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -286,17 +300,20 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
     };
     Tile<HD> tq, tdo;
     float stat = 0.f;  // lse (threads 0..31) or D (32..63) of one tile row
+    bool out = false;  // RAG: that row's lse is -inf
     auto load = [&](int it) {
         int h, q0;
         tile_of(it, h, q0);
         const long row0 = (long)b * s.n_q + q0;
         if constexpr (RAG) {
-            tq.load(Q + row0 * p.ldq + h * HD, p.ldq, tid, s.n_q - q0);
-            tdo.load(dO + row0 * p.lddo + h * HD, p.lddo, tid, s.n_q - q0);
-            if (tid < 2 * FT) {
-                stat = tid < FT ? INFINITY : 0.f;  // P = 0 past the end, and where LSE is -inf
-                if (tid % FT < s.n_q - q0) stat = (tid < FT ? p.lse : p.d)[(row0 + tid % FT) * s.n_heads + h];
-                if (tid < FT && stat == -INFINITY) stat = INFINITY;
+            const int rows = s.n_q - q0;
+            tq.load(Q + row0 * p.ldq + h * HD, p.ldq, tid, rows);
+            tdo.load(dO + row0 * p.lddo + h * HD, p.lddo, tid, rows);
+            if (tid < 2 * FT) {  // rows past the end: left out, as rows of LSE = -inf
+                const bool ok = tid % FT < rows;
+                stat = tid < FT ? -INFINITY : 0.f;
+                if (ok) stat = (tid < FT ? p.lse : p.d)[(row0 + tid % FT) * s.n_heads + h];
+                out = ok && tid < FT && stat == -INFINITY;
             }
         } else {
             tq.load(Q + row0 * p.ldq + h * HD, p.ldq, tid);
@@ -305,6 +322,10 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
         }
     };
     auto store = [&](int buf) {
+        if (RAG && wave == 0) {
+            const bool any = __any(out);
+            if (tid == 0) any_out[buf] = any;
+        }
         tq.store(Qs[buf], tid);
         tdo.store(Os[buf], tid);
         if (tid < FT) Ls[buf][tid] = ACC ? stat : stat * F_LOG2E;
@@ -324,6 +345,12 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
         int h, q0;
         tile_of(it, h, q0);
         (void)h;
+        if (RAG && any_out[buf]) {
+            auto none = [&](int r) { return Ls[buf][r] == -INFINITY; };
+            Tile<HD>::drop(Qs[buf], tid, none);
+            Tile<HD>::drop(Os[buf], tid, none);
+            __syncthreads();
+        }
         const float *Ql = Qs[buf], *Ol = Os[buf];
         f32x4 sa[2], da[2];  // S / dP[q0 + 16 qs + 4 g + r][ki]
         bool live[2];
@@ -344,10 +371,10 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
                 const int qr = 16 * qs + 4 * g + r;
                 float pv = ACC ? expf(fmaf(sa[qs][r], s.inv_sqrt_dim, -Ls[buf][qr]))
                                : __builtin_amdgcn_exp2f(sa[qs][r] - Ls[buf][qr]);
-                const bool past = RAG && q0 + qr >= s.n_q;  // a zero row (against an infinite K or V: NaN)
-                if ((s.causal && ki > q0 + qr + shift) || past) pv = 0.f;
+                const bool none = RAG && Ls[buf][qr] == -INFINITY;  // a zero row (against an infinite K or V: NaN)
+                if ((s.causal && ki > q0 + qr + shift) || none) pv = 0.f;
                 sa[qs][r] = pv;
-                da[qs][r] = past ? 0.f : pv * (da[qs][r] - Dl[buf][qr]);
+                da[qs][r] = none ? 0.f : pv * (da[qs][r] - Dl[buf][qr]);
             }
         // dV^T += dO^T P, dK^T += Q^T dS: step (qs, e) is query q0 + 16 qs + 4 g + e
 #pragma unroll
@@ -430,8 +457,8 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
             of[u] = f4(orr + 16 * u);
         }
     }
-    float l2 = p.lse[((long)b * s.n_q + ql) * s.n_heads + h] * (RAG ? 1.f : F_LOG2E);
-    if (RAG && l2 == -INFINITY) l2 = INFINITY;  // no gradient: P = 0
+    const float l2 = p.lse[((long)b * s.n_q + ql) * s.n_heads + h] * (RAG ? 1.f : F_LOG2E);
+    const bool dead = RAG && l2 == -INFINITY;  // no gradient
     const float dd = p.d[((long)b * s.n_q + ql) * s.n_heads + h];
     const int shift = RAG ? s.n_kv - s.n_q : 0;
     const int nkt = RAG ? ((s.causal ? min(s.n_kv, q0 + 64 + shift) : s.n_kv) + FT - 1) / FT
@@ -498,6 +525,10 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
         __syncthreads();
     }
     if (RAG && qi >= s.n_q) return;
+    if (dead) {
+#pragma unroll
+        for (int j = 0; j < NU; ++j) dqt[j] = f32x4{0, 0, 0, 0};
+    }
     float *dqr = p.dq + ((long)b * s.n_q + qi) * p.lddq + h * HD + 4 * g;
     const float sc = s.inv_sqrt_dim;
     if constexpr (QKE) {
