@@ -837,6 +837,54 @@ def test_flash_attention_fp32_ragged_masked_rows(n, hd):
         assert rel_l2(want[4], dk) < 1e-6 and rel_l2(want[5], dv) < 1e-6
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(100, 100, 128), (37, 37, 64), (70, 131, 64)])
+def test_flash_attention_fp32_ragged_infinities_behind_the_mask(nq, nkv, hd):
+    """An infinity or NaN in a row that the causal mask hides from a query (or key) does
+    not reach it: V and K of a later key, Q and dO of an earlier query.  LSE and D are the
+    clean call's, so that only the masked products are in question.  The other rows are
+    the clean call's up to the order of fp32 sums (at most nkv 2^-24 of |terms|)."""
+    from valkyr_amd import kernels as K
+
+    H, shift = 2, nkv - nq
+    note(f"fa fp32 masked infinities nq={nq} nkv={nkv} hd={hd}")
+    q, do = (O.normal(nq * H * hd, i).reshape(nq, H, hd) for i in (21, 22))
+    k, v = (O.normal(nkv * H * hd, i).reshape(nkv, H, hd) for i in (23, 24))
+    p = K.attn_params(nq, nkv, H, H, hd, True, 1, K.F32)
+    o, lse, d, dq, dk, dv = _fa_f32_all(p, nq, H, q, k, v, do)
+
+    def close(a, b):
+        assert np.all(np.isfinite(b)) and rel_l2(a, b) < nkv * 2.0 ** -24 + 2e-6
+
+    for bad in (np.inf, -np.inf, np.nan):
+        for key in (shift + 5, shift + nq // 2, nkv - 1):  # seen from query key - shift on
+            t, r = v.copy(), key - shift
+            t[key, :, 3] = bad
+            got = _fa_f32_all(p, nq, H, q, k, t, do, lse, d)
+            close(o[:r], got[0][:r])
+            close(lse, got[1])
+            close(dq[:r], got[3][:r])
+            close(dk[key + 1:], got[4][key + 1:]) if key + 1 < nkv else None
+            close(dv, got[5])
+            assert not np.any(np.isfinite(got[0][r:, :, 3]))
+            t = k.copy()
+            t[key, :, 3] = bad
+            got = _fa_f32_all(p, nq, H, q, t, v, do, lse, d)
+            close(o[:r], got[0][:r])
+            close(dq[:r], got[3][:r])
+        for row in (0, nq // 2, nq - 2):  # the last key that it sees is row + shift
+            t, r = do.copy(), row + shift + 1
+            t[row, :, 3] = bad
+            got = _fa_f32_all(p, nq, H, q, k, v, t, lse, d)
+            close(dv[r:], got[5][r:])
+            close(dk[r:], got[4][r:])
+            t = q.copy()
+            t[row, :, 3] = bad
+            got = _fa_f32_all(p, nq, H, t, k, v, do, lse, d)
+            close(dv[r:], got[5][r:])
+            close(dk[r:], got[4][r:])
+            assert not np.any(np.isfinite(got[4][:r, :, 3]))
+
+
 @pytest.mark.parametrize("hd,rows", [(128, 4 * 2048 * 16), (64, 3 * 100 * 4)])
 def test_fa_bw_d_bf16_inputs(hd, rows):
     """D = rowsum(O dO) from bf16 O and dO (fa_bw_d.comp with bf16 storage) vs

@@ -76,6 +76,15 @@ struct Tile {
             v[i] = r < rows ? f4(base + (long)r * ld + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
+    VKH_DEV bool finite() const {
+        float z = 0.f;  // 0 times an infinity or a NaN is NaN
+#pragma unroll
+        for (int i = 0; i < N4; ++i) {
+            z = fmaf(v[i].x, 0.f, z); z = fmaf(v[i].y, 0.f, z);
+            z = fmaf(v[i].z, 0.f, z); z = fmaf(v[i].w, 0.f, z);
+        }
+        return z == 0.f;
+    }
     // a stored tile's rows that `out` names become zero
     template <class Out>
     static VKH_DEV void drop(float *lds, int tid, Out out) {
@@ -100,13 +109,16 @@ struct Tile {
 // -inf gets O = 0 and LSE = -inf, as one with a NaN among its scores gets LSE = -inf.
 // The backward leaves rows of LSE = -inf out, as the per-row kernels do: their staged Q
 // and dO become zeros (0 times an infinity is NaN) and their dQ is zero.
+// Nor does an infinity or NaN behind the causal mask reach a row that does not see it:
+// tiles that the mask cuts and that hold one are added pair by pair (acc_seen; the check,
+// in cut tiles only, takes 100 tokens from 71 to 73 us).
 // Bound by the matrix cores of the few CUs a short sequence reaches; against the
 // per-row kernels (one wave a row, a dot product at a time).  They round as those did:
 // the contraction over the head runs in a chain per 16 columns and a tree (one chain of
 // 128 put 2e-7 of error on a score), scores are scaled after it and P is expf of them.
 // 16 heads, 100 tokens, head_dim 128, relative error of O / dQ: 2.6e-7 / 4.2e-7 with one
 // chain and exp2 of pre-scaled scores, 1.4e-7 / 2.6e-7 here, 1.5e-7 / 2.6e-7 on the per-row
-// kernels; forward and backward 64 -> 70 us (229 there).
+// kernels; forward and backward 64 -> 70 us (229 there), 73 with the rules above.
 template <int NU, bool RAG>
 VKH_DEV f32x4 head_dot(const float *row, const float4 (&f)[NU]) {
     f32x4 a[NU] = {};
@@ -124,6 +136,29 @@ VKH_DEV f32x4 head_dot(const float *row, const float4 (&f)[NU]) {
     return a[0];
 }
 
+// acc[j][r] += sum over the tile's rows x of T[x][16 j + 4 g + r] W[x][item], W held as
+// the matrix cores take it, without the rows that the lane's item (its query or key)
+// does not see: for a tile under the causal mask that holds an infinity or a NaN, which
+// the mask's zero weights would carry into every item.
+template <int HD, class See>
+VKH_DEV void acc_seen(f32x4 (&acc)[HD / 16], const float *T, const f32x4 (&w)[2], int lane, See see) {
+    const int g = lane / 16, c = lane % 16;
+#pragma unroll
+    for (int xs = 0; xs < 2; ++xs)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            for (int g2 = 0; g2 < 4; ++g2) {
+                const int x = 16 * xs + 4 * g2 + e;
+                const float wx = __shfl(w[xs][e], 16 * g2 + c);
+                if (!see(x)) continue;
+#pragma unroll
+                for (int j = 0; j < HD / 16; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[j][r] = fmaf(T[x * (HD + 4) + 16 * j + 4 * g + r], wx, acc[j][r]);
+            }
+}
+
 // ── forward: block = 64 queries of one (sequence, head) ─────────────────
 template <int HD, bool RAG = false>
 __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float *q, long ldq,
@@ -132,6 +167,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
                                                        bool zz) {
     constexpr int P = HD + 4, NU = HD / 16;
     __shared__ __attribute__((aligned(16))) float Ks[2][FT * P], Vs[2][FT * P];
+    __shared__ int pairs[2];
     const int h = blockIdx.x % s.n_heads, b = blockIdx.x / s.n_heads;
     const int nqb = (s.n_q + 63) / 64;
     const int y = (int)blockIdx.y, qb = s.causal ? nqb - 1 - (zz ? zigzag(y, nqb) : y) : y;
@@ -162,10 +198,17 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
             tv.load(vb + (long)it * FT * ldv, ldv, tid);
         }
     };
+    // RAG: ends the staging of tile `it`; pairs[it % 2] == it where its V is to be added pair by pair
+    auto staged = [&](int it) {
+        if (RAG && s.causal && it * FT + FT - 1 > q0 + shift && !tv.finite()) pairs[it & 1] = it;
+        __syncthreads();
+    };
+    if (RAG && tid < 2) pairs[tid] = -1;
+    if (RAG) __syncthreads();
     load(0);
     tk.store(Ks[0], tid);
     tv.store(Vs[0], tid);
-    __syncthreads();
+    staged(0);
     f32x4 ot[NU];  // O^T[16 j + 4 g + r][qi]
 #pragma unroll
     for (int j = 0; j < NU; ++j) ot[j] = f32x4{0, 0, 0, 0};
@@ -210,6 +253,10 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
                 l += pv;
             }
         m = mn;
+        if (RAG && pairs[buf] == it) {
+            acc_seen<HD>(ot, Vl, st, lane, [&](int x) { return kt0 + x <= qi + shift; });
+            live[0] = live[1] = false;
+        }
         // O^T += V^T P^T: step (ks, e) is key kt0 + 16 ks + 4 g + e
 #pragma unroll
         for (int j = 0; j < NU; ++j)
@@ -225,7 +272,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_fwd_f32m_k(AttnShape s, const float
             tk.store(Ks[buf ^ 1], tid);
             tv.store(Vs[buf ^ 1], tid);
         }
-        __syncthreads();
+        staged(it + 1);
     }
     l = xsum(l);
     if (RAG && qi >= s.n_q) return;
@@ -266,6 +313,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
     __shared__ __attribute__((aligned(16))) float Qs[2][FT * P], Os[2][FT * P];
     __shared__ float Ls[2][FT], Dl[2][FT];
     __shared__ int any_out[2];  // RAG: a row of the tile has LSE = -inf
+    __shared__ int pairs[2];
     const int kvh = blockIdx.x % s.n_kv_heads, b = blockIdx.x / s.n_kv_heads;
     const int tid = threadIdx.x, lane = tid % 64, g = lane / 16, c = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -334,11 +382,23 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
     f32x4 dvt[NU], dkt[NU];  // dV^T / dK^T[16 j + 4 g + r][ki]
 #pragma unroll
     for (int j = 0; j < NU; ++j) dvt[j] = dkt[j] = f32x4{0, 0, 0, 0};
+    // RAG: ends the staging of tile `it`; pairs[it % 2] == it where its Q and dO are to be added
+    // pair by pair
+    auto staged = [&](int it) {
+        if (RAG && s.causal && it < niter) {
+            int h, q0;
+            tile_of(it, h, q0);
+            if (k0 + 63 > q0 + shift && (!tq.finite() || !tdo.finite())) pairs[it & 1] = it;
+        }
+        __syncthreads();
+    };
+    if (RAG && tid < 2) pairs[tid] = -1;
+    if (RAG) __syncthreads();
     if (niter > 0) {
         load(0);
         store(0);
     }
-    __syncthreads();
+    staged(0);
     for (int it = 0; it < niter; ++it) {
         const int buf = it & 1;
         if (it + 1 < niter) load(it + 1);
@@ -372,10 +432,17 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
                 float pv = ACC ? expf(fmaf(sa[qs][r], s.inv_sqrt_dim, -Ls[buf][qr]))
                                : __builtin_amdgcn_exp2f(sa[qs][r] - Ls[buf][qr]);
                 const bool none = RAG && Ls[buf][qr] == -INFINITY;  // a zero row (against an infinite K or V: NaN)
-                if ((s.causal && ki > q0 + qr + shift) || none) pv = 0.f;
+                const bool masked = s.causal && ki > q0 + qr + shift;
+                if (masked || none) pv = 0.f;
                 sa[qs][r] = pv;
-                da[qs][r] = none ? 0.f : pv * (da[qs][r] - Dl[buf][qr]);
+                da[qs][r] = none || (RAG && masked) ? 0.f : pv * (da[qs][r] - Dl[buf][qr]);
             }
+        if (RAG && pairs[buf] == it) {
+            auto see = [&](int x) { return ki <= q0 + x + shift; };
+            acc_seen<HD>(dvt, Ol, sa, lane, see);
+            acc_seen<HD>(dkt, Ql, da, lane, see);
+            live[0] = live[1] = false;
+        }
         // dV^T += dO^T P, dK^T += Q^T dS: step (qs, e) is query q0 + 16 qs + 4 g + e
 #pragma unroll
         for (int j = 0; j < NU; ++j)
@@ -391,7 +458,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dkv_f32m_k(AttnShape s, AttnPtr
                 }
             }
         if (it + 1 < niter) store(buf ^ 1);
-        __syncthreads();
+        staged(it + 1);
     }
     if (RAG && ki >= s.n_kv) return;
     float *dkr = p.dk + ((long)b * s.n_kv + ki) * p.lddk + kvh * HD + 4 * g;
@@ -436,6 +503,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
     static_assert(!QKE || (HD == 128 && !RAG), "the fused q/k epilogue takes 128-wide head rows");
     constexpr int P = HD + 4, NU = HD / 16;
     __shared__ __attribute__((aligned(16))) float Ks[2][FT * P], Vs[2][FT * P];
+    __shared__ int pairs[2];
     const int h = blockIdx.x % s.n_heads, b = blockIdx.x / s.n_heads;
     const int nqb = (s.n_q + 63) / 64;
     const int y = (int)blockIdx.y, qb = s.causal ? nqb - 1 - (zz ? zigzag(y, nqb) : y) : y;
@@ -475,10 +543,17 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
             tv.load(vb + (long)it * FT * p.ldv, p.ldv, tid);
         }
     };
+    // RAG: ends the staging of tile `it`; pairs[it % 2] == it where its K is to be added pair by pair
+    auto staged = [&](int it) {
+        if (RAG && s.causal && it * FT + FT - 1 > q0 + shift && !tk.finite()) pairs[it & 1] = it;
+        __syncthreads();
+    };
+    if (RAG && tid < 2) pairs[tid] = -1;
+    if (RAG) __syncthreads();
     load(0);
     tk.store(Ks[0], tid);
     tv.store(Vs[0], tid);
-    __syncthreads();
+    staged(0);
     f32x4 dqt[NU];  // dQ^T[16 j + 4 g + r][qi]
 #pragma unroll
     for (int j = 0; j < NU; ++j) dqt[j] = f32x4{0, 0, 0, 0};
@@ -504,10 +579,14 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
             for (int r = 0; r < 4; ++r) {
                 float pv = RAG ? expf(fmaf(sa[ks][r], s.inv_sqrt_dim, -l2)) : __builtin_amdgcn_exp2f(sa[ks][r] - l2);
                 const int kk = kt0 + 16 * ks + 4 * g + r;
-                const bool past = RAG && kk >= s.n_kv;
-                if (s.causal && kk > qi + shift) pv = 0.f;
-                da[ks][r] = past ? 0.f : pv * (da[ks][r] - dd);  // dS^T
+                const bool masked = s.causal && kk > qi + shift;
+                if (masked) pv = 0.f;
+                da[ks][r] = RAG && (masked || kk >= s.n_kv) ? 0.f : pv * (da[ks][r] - dd);  // dS^T
             }
+        if (RAG && pairs[buf] == it) {
+            acc_seen<HD>(dqt, Kl, da, lane, [&](int x) { return kt0 + x <= qi + shift; });
+            live[0] = live[1] = false;
+        }
         // dQ^T += K^T dS^T: step (ks, e) is key kt0 + 16 ks + 4 g + e
 #pragma unroll
         for (int j = 0; j < NU; ++j)
@@ -522,7 +601,7 @@ __global__ __launch_bounds__(FNT, 2) void fa_bwd_dq_f32m_k(AttnShape s, AttnPtrs
             tk.store(Ks[buf ^ 1], tid);
             tv.store(Vs[buf ^ 1], tid);
         }
-        __syncthreads();
+        staged(it + 1);
     }
     if (RAG && qi >= s.n_q) return;
     if (dead) {
