@@ -1026,6 +1026,43 @@ def test_flash_attention_bf16_ragged_recompute(case):
     test_flash_attention_bf16_mfma(case)
 
 
+@pytest.mark.parametrize("n,H,Hkv,hd", [(100, 4, 2, 128), (37, 3, 1, 64), (256, 2, 2, 64)])
+def test_flash_attention_bf16_rows_without_gradient(n, H, Hkv, hd):
+    """Rows of LSE = -inf in the bf16 backward: P = 0 there also where a score is a NaN, so
+    dV is that of a call whose dO is 0 in the row, its dQ is zero and the others' stand."""
+    from valkyr_amd import kernels as K
+
+    note(f"fa bf16 rows without gradient n={n} {H}/{Hkv} hd={hd}")
+    q, do = (O.normal(n * H * hd, i).reshape(n, H, hd) for i in (31, 32))
+    kb, _ = bf16_dev(O.normal(n * Hkv * hd, 33))
+    vb, _ = bf16_dev(O.normal(n * Hkv * hd, 34))
+    p = K.attn_params(n, n, H, Hkv, hd, True, 1, K.BF16)
+
+    def run(q, do, lse=None, d=None):
+        (qb, _), (db, _) = bf16_dev(q.reshape(-1)), bf16_dev(do.reshape(-1))
+        o, bl, bd, cp = zeros(q.size), zeros(n * H), zeros(n * H), zeros(q.size // 2 + 8)
+        K.fa_forward(p, qb, kb, vb, o, bl)
+        K.fa_bw_d(p, o, dev(do), bd, cp)
+        fl = host(bl)
+        if lse is not None:
+            bl, bd = dev(lse), dev(d)
+        dq, dk, dv = zeros(q.size), zeros(n * Hkv * hd), zeros(n * Hkv * hd)
+        K.fa_bw_dkv(p, qb, kb, vb, db, bl, bd, dk, dv)
+        K.fa_bw_dq(p, qb, kb, vb, db, bl, bd, dq)
+        return fl.reshape(n, H), host(bd).reshape(n, H), host(dq).reshape(n, H, hd), host(dk), host(dv)
+
+    do0 = do.copy()
+    do0[7] = 0
+    lse, d, dq, dk, dv = run(q, do0)
+    q[7, :, 0] = np.nan
+    fl = run(q, do)[0]
+    assert np.all(fl[7] == -np.inf) and np.array_equal(np.delete(fl, 7, 0), np.delete(lse, 7, 0))
+    lse[7], d[7] = -np.inf, 0
+    _, _, dq2, _, dv2 = run(q, do, lse, d)
+    assert np.all(dq2[7] == 0) and np.array_equal(np.delete(dq2, 7, 0), np.delete(dq, 7, 0))
+    assert rel_l2(dv, dv2) < 1e-6
+
+
 # n_q != n_kv in bf16 (the reference's causal limit k <= q + (n_kv - n_q),
 # fa_bw_dq.comp / flash_attn.zig:66-68 causalKeyLimit): more keys than queries
 # under the causal mask, and more queries than keys without it; GQA 2:1 and

@@ -1289,10 +1289,12 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
         // where they are used (not held across the tile).  Every query row sees
         // at least one key on this path (causal needs n_q == n_kv, so row q sees
         // keys 0..q), so its LSE is finite and no empty-row case arises here.
-        // (RAG keeps the general kernels' rule for a row whose scores are all -inf: P = 0.)
-        auto lse2 = [&](int qs, int r) {
+        // (RAG keeps the general kernels' rule for a row of LSE = -inf, whose scores are
+        // all -inf or hold a NaN: P = 0, selected, since exp2 of a NaN would stay one.)
+        auto prob = [&](float x, int qs, int r) {
             const float l = Ls[hg][buf][16 * qs + 4 * g + r];
-            return RAG && l == -INFINITY ? INFINITY : l * LOG2E;
+            const float e = __builtin_amdgcn_exp2f(x * c2 - l * LOG2E);
+            return RAG && l == -INFINITY ? 0.f : e;
         };
         auto dval = [&](int qs, int r) { return Dd[hg][buf][16 * qs + 4 * g + r]; };
         // the dP accumulators start at -D, so they end as dP - D
@@ -1340,7 +1342,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
                 const int t2 = f / EVERY, qs2 = t2 / KS, ks2 = t2 % KS;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    sc[qs2][ks2][r] = __builtin_amdgcn_exp2f(sc[qs2][ks2][r] * c2 - lse2(qs2, r));
+                    sc[qs2][ks2][r] = prob(sc[qs2][ks2][r], qs2, r);
             }
         }
         if (diag) {  // keys above a query of the tile (uniform; no MFMA inside)
@@ -1635,6 +1637,11 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dq4_k(AttnShape s, AttnPtr
             if (ok && g == 0) p.d[t * s.n_heads + h] = dd[j];
         } else {
             dd[j] = ok ? p.d[t * s.n_heads + h] : 0.f;
+        }
+        if (l == -INFINITY) {  // zero scores too: one that is a NaN would keep P from 0
+            dd[j] = 0.f;
+#pragma unroll
+            for (int ds = 0; ds < DSR; ++ds) qr[j][ds] = orr[j][ds] = bf16x8{};
         }
     }
     wait_vm0();
