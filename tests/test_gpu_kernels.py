@@ -340,6 +340,60 @@ def test_linear_products_of_few_tiles(form, shape):
         assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("form,op,rows,cols,k", [
+    ("fp32", "nt", 537, 3648, 576), ("fp32", "nn", 512, 2560, 960), ("fp32", "tn", 640, 1956, 2072),
+    ("fp32", "nt", 1000, 960, 520), ("fp32", "nt", 16, 1024, 3072), ("fp32", "tn", 3072, 1024, 64),
+    ("fp32", "nn", 188, 2368, 2944), ("mixed", "nt", 494, 1312, 3200), ("bf16", "nt", 494, 1312, 3200),
+    ("bf16", "nn", 101, 5344, 3728), ("bf16", "tn", 940, 664, 2608), ("bf16", "nt", 128, 256, 20480)])
+def test_linear_products_keep_their_partial_sums(form, op, rows, cols, k):
+    """A product of few tiles sums K in at least the two chains (bf16 from K = 2048) of the
+    large tiles.  One term of a row is so large that the chain which holds it loses all its
+    other terms (ones), so at least k / 2 ones must be left, less one slab of 64 and the
+    spacing of the sum."""
+    from valkyr_amd import kernels as K
+
+    note(f"partial sums {form} {op} {rows} x {cols} over {k}")
+    big = 2.0 ** (27 if form == "fp32" else 30)
+    spacing = big * 2.0 ** -23
+    a = np.ones((k, rows) if op == "tn" else (rows, k), np.float32)
+    a[(0,) if op == "tn" else (slice(None), 0)] = big
+    b = np.ones(cols * k, np.float32)
+    up = (lambda t: bf16_dev(t)[0]) if form == "bf16" else dev
+    ba, bb, out = up(a.reshape(-1)), up(b), zeros(rows * cols)
+    f = {"nt": ("matmul_nt", (rows, cols, k)), "nn": ("linear_backward_dx", (rows, k, cols)),
+         "tn": ("linear_backward_dw", (k, rows, cols))}[op]
+    if form == "bf16":
+        getattr(K, f[0] + "_bf16")(ba, bb, out, *f[1])
+    else:
+        getattr(K, f[0])(ba, bb, out, *f[1], int(form == "mixed"))
+    got = host(out).astype(np.float64) - big
+    assert got.min() >= k / 2 - 64 - spacing and got.max() <= k + spacing, (got.min(), got.max())
+
+
+@pytest.mark.parametrize("M,n,r", [(8192, 4096, 16), (300, 2048, 64), (40000, 512, 4)])
+def test_lora_rank_products_keep_their_partial_sums(M, n, r):
+    """x A^T and dy B sum in at least eight chains (as above: of the ones at most an eighth
+    and one slab of 32 are lost)."""
+    from valkyr_amd import kernels as K
+
+    note(f"lora partial sums M={M} n={n} r={r}")
+    big = 2.0 ** 27
+    x = np.ones((M, n), np.float32)
+    x[:, 0] = big
+    bx, one, o64 = dev(x), dev(np.ones(n * max(r, 64), np.float32)), dev(np.ones(M * 64, np.float32))
+    inter, y, dA, dB = zeros(M * r), zeros(M * 64), zeros(n * r), zeros(n * r)
+    K.lora_forward(bx, one, one, one, y, inter, M, 64, n, r, 0.0, 0)
+    got = host(inter).astype(np.float64) - big
+    assert got.min() >= n * 7 / 8 - 32 - 16, got.min()
+    # dx = dy W + 1 (dy B) A with W = 0 and A picking rank 0: its first column is dy B
+    w, a = zeros(n * 64), np.zeros((r, 64), np.float32)
+    a[0, 0] = 1
+    dx = zeros(M * 64)
+    K.lora_backward(bx, o64, w, dev(a), one, inter, dx, dA, dB, M, n, 64, r, 1.0, 0)
+    got = host(dx).reshape(M, 64)[:, 0].astype(np.float64) - big
+    assert got.min() >= n * 7 / 8 - 32 - 16, got.min()
+
+
 @pytest.mark.parametrize("form", ["fp32", "mixed", "bf16"])
 @pytest.mark.parametrize("shape,skew", [((1, 9, 17), 0), ((65, 129, 63), 0), ((130, 257, 1001), 0),
                                         ((128, 64, 72), 1), ((2048, 264, 520), 1)])

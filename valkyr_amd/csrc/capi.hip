@@ -556,7 +556,9 @@ class LoraScratch {
 // tokens and 2560 columns), and the rank-r update rides in the base product's epilogue
 // instead of reading the output back (16 and 14 us): that layer, forward and backward
 // at rank 16, 213 -> 157 us.  A captured stream (no scratch) and operands of 2 GiB keep
-// the row and update kernels, with fp32 factors and products as well.
+// the row and update kernels, with fp32 factors and products as well.  x A^T and dy B
+// sum in at least the row kernel's eight partial sums.
+constexpr int kLoraChains = 8;
 vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, const float *b,
                             float *y, float *inter, uint32_t M, uint32_t N, uint32_t K,
                             uint32_t r, float aor, uint32_t precision, vkh_stream stream) {
@@ -577,11 +579,11 @@ vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, cons
             VKH_HIP(lora_update(y, N, (int)M, (int)r, sb, aor, st));
             return VKH_OK;
         }
-        const size_t wsb = std::max(lin_ws_bytes(LinOp::NT, form, x, w, M, N, K), g32_ws_bytes_for(M, r, K));
+        const size_t wsb = std::max(lin_ws_bytes(LinOp::NT, form, x, w, M, N, K), g32_ws_bytes_for(M, r, K, kLoraChains));
         LoraScratch sc;
         if (wsb) VKH_TRY(sc.acquire(wsb, st));
-        const GemmWs ws{sc.p, wsb};
-        VKH_HIP(g32_nt(x, K, a, K, inter, r, M, r, K, nullptr, 0, 1.f, 0.f, ws, st));
+        const GemmWs ws{sc.p, wsb}, rows{sc.p, wsb, false, kLoraChains};
+        VKH_HIP(g32_nt(x, K, a, K, inter, r, M, r, K, nullptr, 0, 1.f, 0.f, rows, st));
         VKH_HIP(lin_run(LinOp::NT, form, x, w, y, M, N, K, ws, st, &sb, (int)r, aor));
         return VKH_OK;
     }
@@ -612,14 +614,14 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
                       (!dx || lora_update_ok(dx, K, (int)r, sa));
     if (fast && !capturing(st) && (!dx || lin_lora_ok(LinOp::NN, form, M, N, K, sa, (int)r))) {
         // fp32 factors and products
-        size_t wsb = std::max({g32_ws_bytes_for(M, r, N), g32_ws_bytes_for(r, K, M), g32_ws_bytes_for(N, r, M)});
+        size_t wsb = std::max({g32_ws_bytes_for(M, r, N, kLoraChains), g32_ws_bytes_for(r, K, M), g32_ws_bytes_for(N, r, M)});
         if (dx) wsb = std::max(wsb, lin_ws_bytes(LinOp::NN, form, dy, w, M, N, K));
         LoraScratch sc;
         VKH_TRY(sc.acquire(dyb_bytes + wsb, st));
         float *dyB = (float *)sc.p;
-        const GemmWs ws{wsb ? sc.p + dyb_bytes : nullptr, wsb};
+        const GemmWs ws{wsb ? sc.p + dyb_bytes : nullptr, wsb}, rows{ws.p, wsb, false, kLoraChains};
         sa.s[0].u = dyB;
-        VKH_HIP(g32_nn(dy, N, b, r, dyB, r, M, N, r, 1.f, 0.f, ws, st));
+        VKH_HIP(g32_nn(dy, N, b, r, dyB, r, M, N, r, 1.f, 0.f, rows, st));
         if (dx) VKH_HIP(lin_run(LinOp::NN, form, dy, w, dx, M, N, K, ws, st, &sa, (int)r, aor));
         VKH_HIP(g32_tn(dyB, r, x, K, dA, K, M, r, K, aor, 0.f, ws, st));
         VKH_HIP(g32_tn(dy, N, inter, r, dB, r, M, N, r, aor, 0.f, ws, st));

@@ -82,9 +82,12 @@ size_t ws_for(const Plan &p, const GemmShape &s) {
 // 128 x 512 x 512 22 -> 7.3, 512 x 1024 x 1024 39 -> 16; bf16 16 x 1024 x 3072
 // 18.8 -> 7.3 us, 128 x 1024 x 1024 10.6 -> 6.5, 512 x 768 x 32000 95 -> 55.
 // fp32 also has the in-block split (two wave groups on the halves of K, no reduce
-// launch), and with two_halves nothing else (a 2-layer 256-wide step of 128 tokens
-// 980 -> 620 us with the same bits).
-Plan plan_few(const GemmShape &s, size_t ws_bytes, bool f32, bool mn_a, bool two_halves = false) {
+// launch).  `base` is the plan of the large tiles, whose number of partial sums over K
+// is the least that the pick may have: fewer, longer chains would round worse (one
+// chain where base had two was 1.4 times as far from 64 bits at K = 1957).  With
+// ws.keep_sums the pick has base's very sums (a 2-layer 256-wide fp32 step of 128
+// tokens 980 -> 620 us with the same bits), with ws.min_chains at least that many.
+Plan plan_few(const GemmShape &s, const GemmWs &ws, bool f32, bool mn_a, const Plan &base) {
     struct Fit { double launch, slab0, slab1, mfma, l2, red, part, hbm; };
     constexpr Fit kB{3.8, 0.088, 0.199, 0.225, 21.2, 2.5, 6.6, 5.2},
         kF{4.5, 0.314, 0.047, 0.574, 10.7, 2.0, 6.5, 4.4};
@@ -93,11 +96,16 @@ Plan plan_few(const GemmShape &s, size_t ws_bytes, bool f32, bool mn_a, bool two
     const double hbm = (es * s.K * ((double)s.M + s.N) + 4.0 * s.M * s.N) / (f.hbm * 1e6);
     const int nk = (s.K + (f32 ? 31 : 63)) / (f32 ? 32 : 64);
     const int min_slabs = f32 ? 1 : 8;  // of a split: 512 of K in bf16, as in plan()
-    Plan best{Pick::T128x64, 1};
+    const bool halves = base.tile == Pick::T128x64ks2;
+    const int chains = std::max(1, std::min(nk, std::max(halves ? 2 : base.splits, ws.min_chains)));
+    const size_t ws_bytes = ws.p ? ws.bytes : 0;
+    // the halves in bf16 and products without scratch: in one block
+    if (!f32 && halves && ws.keep_sums) return base;
+    Plan best{chains > 1 ? Pick::T128x64ks2 : Pick::T128x64, 1};
     double tb = 1e30;
     auto tile = [&](Pick pick, Pick ks2, int bm, int bn) {
         const double tiles = (double)ceil_div(s.M, bm) * ceil_div(s.N, bn);
-        if (f32) {  // both groups of a block share its CU's matrix cores
+        if (f32 && (chains <= 2 || !ws_bytes)) {  // both groups of a block share its CU's matrix cores
             const double slabs = (nk + 1) / 2, share = ceil(tiles / 256) * 2 * f.mfma * bm * bn / 4096;
             const double t = std::max(slabs * std::max(f.slab0 + f.slab1 * (bm + bn) / 128, share),
                                       tiles * nk * (bm + bn) * 128 / (f.l2 * 1e6));
@@ -105,11 +113,12 @@ Plan plan_few(const GemmShape &s, size_t ws_bytes, bool f32, bool mn_a, bool two
                 tb = f.launch + 0.7 + std::max(t, hbm);
                 best = Plan{ks2, 1};
             }
-            if (two_halves) return;
+            if (ws.keep_sums && halves) return;
         }
-        for (int sp = 1; sp <= 32; sp *= 2) {
+        for (int sp = chains; sp <= 32; sp *= 2) {
             const Plan p{pick, sp};
-            if (sp > 1 && (nk / sp < min_slabs || ws_for(p, s) > ws_bytes)) break;
+            if (sp > chains && (ws.keep_sums || nk / sp < min_slabs)) break;
+            if (ws_for(p, s) > ws_bytes) break;
             const double slabs = (nk + sp - 1) / sp, blocks = tiles * sp;
             const double share = ceil(blocks / 256) * f.mfma * bm * bn / 4096;
             double t = std::max(slabs * std::max(f.slab0 + f.slab1 * (bm + bn) / 128, share),
@@ -126,15 +135,12 @@ Plan plan_few(const GemmShape &s, size_t ws_bytes, bool f32, bool mn_a, bool two
     return best;
 }
 
-// mn_a: the A operand is MN-major (the weight gradients).
-Plan plan(const GemmShape &s, size_t ws_bytes, bool mn_a = false) {
+// The plan of the large tiles.
+Plan plan_large(const GemmShape &s, size_t ws_bytes) {
     auto tiles = [&](int bm, int bn) { return (long)ceil_div(s.M, bm) * (long)ceil_div(s.N, bn); };
     if (tiles(256, 256) >= 512) return {Pick::Big, 1};
     const long t128 = tiles(128, 128), t64 = tiles(128, 64);
     if (t128 >= 512) return {Pick::T128w8, 1};
-    // few tiles: up to 96 of 128 x 64, and up to 255 where K is short (beyond, the
-    // two-group 128 x 64 blocks are as fast: 256 x 4096 x 4096 26.5 against 32.5 us)
-    if (t64 <= 96 || (t64 < 256 && s.K <= 1024)) return plan_few(s, ws_bytes, false, mn_a);
     const int nk = (s.K + 63) / 64;
     Plan p{Pick::T128x64, 1};
     if (s.K >= 16384 && t128 >= 256)
@@ -163,6 +169,17 @@ Plan plan(const GemmShape &s, size_t ws_bytes, bool mn_a = false) {
     return p;
 }
 
+// mn_a: the A operand is MN-major (the weight gradients).
+Plan plan(const GemmShape &s, const GemmWs &ws, bool mn_a = false) {
+    auto tiles = [&](int bm, int bn) { return (long)ceil_div(s.M, bm) * (long)ceil_div(s.N, bn); };
+    // few tiles: up to 96 of 128 x 64, and up to 255 where K is short (beyond, the
+    // two-group 128 x 64 blocks are as fast: 256 x 4096 x 4096 26.5 against 32.5 us)
+    const long t64 = tiles(128, 64);
+    if (t64 <= 96 || (t64 < 256 && s.K <= 1024))
+        return plan_few(s, ws, false, mn_a, plan_large(s, ~size_t(0)));
+    return plan_large(s, ws.p ? ws.bytes : 0);
+}
+
 // Whether the fused-epilogue forward kernels (8-wave 128 x 128 tiles only) take
 // the product: where plan() picks that tile, or, for a launch paired with one
 // of the same shape on a second stream (the forward's two half batches), where
@@ -170,7 +187,7 @@ Plan plan(const GemmShape &s, size_t ws_bytes, bool mn_a = false) {
 // step's q|k|v and gate/up halves: 256 + 256 and 384 + 384 tiles; the forward
 // as two concurrent half batches measured 18.58-18.59 against 18.85 ms).
 bool fused_tile_ok(const GemmShape &s, bool paired) {
-    const Plan p = plan(s, 0);
+    const Plan p = plan(s, GemmWs{nullptr, 0});
     if (p.tile == Pick::T128w8 && p.splits == 1) return true;
     return paired && s.M % 128 == 0 && 2L * (s.M / 128) * ceil_div(s.N, 128) >= 512;
 }
@@ -178,7 +195,7 @@ bool fused_tile_ok(const GemmShape &s, bool paired) {
 template <Lay LA, Lay LB, class Epi>
 hipError_t run16(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e, const GemmWs &ws,
                  hipStream_t st) {
-    const Plan p = plan(GemmShape{ws.plan_rows ? ws.plan_rows : s.M, s.N, s.K}, ws.p ? ws.bytes : 0, LA == Lay::MN);
+    const Plan p = plan(s, ws, LA == Lay::MN);
     const SplitK sk{p.splits, (f32x4 *)ws.p};
     const int g = p.column_order ? 0 : tile_group_rows<LA, LB>();
     switch (p.tile) {
@@ -215,21 +232,22 @@ hipError_t run16(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e,
 // Fewer than 256 tiles of 128 x 64, or fewer than 512 with a K of at most 1024:
 // plan_few (there the in-block split leaves CUs idle or its second group without
 // work: 2560-wide products of 512 rows 95 -> 64 us, 3072 x 1024 dW of 16 rows 15 -> 8).
-Plan plan32(const GemmShape &s, size_t ws_bytes, bool mn_a = false, bool two_halves = false) {
+Plan plan32(const GemmShape &s, const GemmWs &ws, bool mn_a = false) {
     auto tiles = [&](int bm, int bn) { return (long)ceil_div(s.M, bm) * (long)ceil_div(s.N, bn); };
     auto fill = [](long t) { return (double)t / (256.0 * (double)((t + 255) / 256)); };
     const long t128 = tiles(128, 128), t64 = tiles(128, 64);
     Plan p{Pick::T128x64, 1};
     if (t128 >= 256 && fill(t128) >= fill(t64)) p = Plan{Pick::T128w8, 1};
-    else if (t64 < 256 || (t64 < 512 && s.K <= 1024)) p = plan_few(s, ws_bytes, true, mn_a, two_halves);
     else if (t64 < 512) p = Plan{Pick::T128x64ks2, 1};
+    if ((p.tile == Pick::T128x64ks2 && (t64 < 256 || s.K <= 1024)) || ws.min_chains > 2)
+        return plan_few(s, ws, true, mn_a, p);
     return p;
 }
 
 template <Lay LA, Lay LB, class Epi>
 hipError_t run32(const Op16 &a, const Op16 &b, const GemmShape &s, const Epi &e, const GemmWs &ws,
                  hipStream_t st) {
-    const Plan p = plan32(s, ws.p ? ws.bytes : 0, LA == Lay::MN, ws.two_halves);
+    const Plan p = plan32(s, ws, LA == Lay::MN);
     const SplitK sk{p.splits, (f32x4 *)ws.p};
     const int g = p.column_order ? 0 : tile_group_rows<LA, LB>();
     switch (p.tile) {
@@ -540,7 +558,7 @@ hipError_t g16_qkv_norm_rope(const bf16 *x, long ldx, const bf16 *w, long ldw, f
         return hipErrorNotSupported;
     const GemmShape s{M, N, K};
     if (!fused_tile_ok(s, paired)) return hipErrorNotSupported;
-    const Plan p = plan(s, 0);  // its tile order where it is this tile
+    const Plan p = plan(s, GemmWs{nullptr, 0});  // its tile order where it is this tile
     if (((uintptr_t)out & 15u) || ld_out % 8 || (L.qk_norm && (((uintptr_t)wq | (uintptr_t)wk) & 15u)) ||
         (L.rotary_dim && ((uintptr_t)tab & 15u)))
         return hipErrorNotSupported;
@@ -563,7 +581,7 @@ hipError_t g32_qkv_norm_rope(const float *x, long ldx, const float *w, long ldw,
         L.rotary_dim > 128 || N != (L.n_q_heads + 2 * L.n_kv_heads) * 128)
         return hipErrorNotSupported;
     const GemmShape s{M, N, K};
-    const Plan p = plan32(s, 0);
+    const Plan p = plan32(s, GemmWs{nullptr, 0});
     if (p.tile != Pick::T128w8 || p.splits != 1) return hipErrorNotSupported;
     if (((uintptr_t)out & 15u) || ld_out % 4 || (L.qk_norm && (((uintptr_t)wq | (uintptr_t)wk) & 15u)) ||
         (L.rotary_dim && ((uintptr_t)tab & 15u)))
@@ -581,7 +599,7 @@ hipError_t g32_gate_up_swiglu(const float *x, long ldx, const float *w, long ldw
                               long ldgu, float *gated, long ldg, int M, int F, int K, hipStream_t st) {
     if (M <= 0 || F <= 0 || F % 64) return hipErrorNotSupported;
     const GemmShape s{M, 2 * F, K};
-    const Plan p = plan32(s, 0);
+    const Plan p = plan32(s, GemmWs{nullptr, 0});
     if (p.tile != Pick::T128w8 || p.splits != 1) return hipErrorNotSupported;
     Op16 a, b;
     if (!make_op32(x, ldx, M, K, a) || !make_op32(w, ldw, 2L * F, K, b)) return hipErrorNotSupported;
@@ -834,14 +852,18 @@ hipError_t lin_run(LinOp op, LinForm f, const void *a, const void *b, float *out
     return g16_tn(x, lda, y, ldb, out, K, M, N, K, 1.f, 0.f, rest, st);
 }
 
-size_t g32_ws_bytes_for(int M, int N, int K) {
+size_t g32_ws_bytes_for(int M, int N, int K, int min_chains) {
     const GemmShape s{M, N, K};
-    return std::max(ws_for(plan32(s, ~size_t(0)), s), ws_for(plan32(s, ~size_t(0), true), s));
+    GemmWs any{(void *)1, ~size_t(0)};  // (planned for, not used)
+    any.min_chains = min_chains;
+    return std::max(ws_for(plan32(s, any), s), ws_for(plan32(s, any, true), s));
 }
 
-size_t g16_ws_bytes_for(int M, int N, int K) {
+size_t g16_ws_bytes_for(int M, int N, int K, bool keep_sums) {
     const GemmShape s{M, N, K};
-    return std::max(ws_for(plan(s, ~size_t(0)), s), ws_for(plan(s, ~size_t(0), true), s));
+    GemmWs any{(void *)1, ~size_t(0)};
+    any.keep_sums = keep_sums;
+    return std::max(ws_for(plan(s, any), s), ws_for(plan(s, any, true), s));
 }
 
 }  // namespace vkh

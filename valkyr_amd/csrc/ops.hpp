@@ -37,14 +37,12 @@ hipError_t gemm_tn(Precision pr, Mat dy, Mat x, float *dw, long lddw, int M, int
 struct GemmWs {
     void *p;
     size_t bytes;
-    // rows to plan for instead of M (0: M): a product run as parts of one with more
-    // rows (the forward's half batches) takes the whole product's split over K, so
-    // its sums have the same bits either way
-    int plan_rows = 0;
-    // fp32 products keep the summation order of two halves of K whatever their tile:
-    // the training step's gradients, and with them its Adam trajectory, stay the same
-    // bits on every tile plan
-    bool two_halves = false;
+    // products of few tiles keep the large tiles' partial sums over K whatever their
+    // tile: the training step's gradients, and with them its Adam trajectory, stay the
+    // same bits on every tile plan
+    bool keep_sums = false;
+    // fp32 products run as at least this many partial sums over K (0: as the plan has it)
+    int min_chains = 0;
 };
 hipError_t g16_nt(const bf16 *x, long ldx, const bf16 *w, long ldw, float *y, long ldy, int M,
                   int N, int K, const float *R, long ldr, float alpha, float beta,
@@ -69,7 +67,7 @@ hipError_t g16_nn_bf16(const bf16 *dy, long lddy, const bf16 *w, long ldw, bf16 
 hipError_t g16_tn(const bf16 *dy, long lddy, const bf16 *x, long ldx, float *dw, long lddw, int M,
                   int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st,
                   bool padded = false);
-size_t g16_ws_bytes_for(int M, int N, int K);
+size_t g16_ws_bytes_for(int M, int N, int K, bool keep_sums = false);
 // fp32 operands on the same DMA-staged kernels (fp32 matrix cores); operands
 // the DMA path cannot take (alignment, ld or extent not a multiple of 4, over
 // 2 GiB) go to gemm_nt / gemm_nn / gemm_tn at Precision::FP32.
@@ -82,7 +80,7 @@ hipError_t g32_nn(const float *dy, long lddy, const float *w, long ldw, float *d
 hipError_t g32_tn(const float *dy, long lddy, const float *x, long ldx, float *dw, long lddw, int M,
                   int N, int K, float alpha, float beta, const GemmWs &ws, hipStream_t st,
                   bool padded = false);
-size_t g32_ws_bytes_for(int M, int N, int K);
+size_t g32_ws_bytes_for(int M, int N, int K, int min_chains = 0);
 // The three contractions of a linear layer on dense row-major operands of any
 // width and alignment: NT y = x W^T (a = x, b = W), NN dx = dy W, TN dW = dy^T x,
 // output overwritten.  F32: fp32 products; MIXED: fp32 operands rounded to bf16

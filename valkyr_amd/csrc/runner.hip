@@ -519,7 +519,7 @@ struct vkh_runner {
         // step keeps its sums in two halves of K, in one block each, and needs none
         size_t wsb = 0;
         auto need = [&](int m, int n, int k) {
-            if (b16()) wsb = std::max(wsb, g16_ws_bytes_for(m, n, k));
+            if (b16()) wsb = std::max(wsb, g16_ws_bytes_for(m, n, k, true));
         };
         for (const int t : {T, T / 2}) {
             need(t, qkvd, D); need(t, D, qd); need(t, 2 * F, D); need(t, D, F); need(t, V, D);
@@ -532,7 +532,7 @@ struct vkh_runner {
             VKH_TRY(alloc(w, wsb));
             gws = GemmWs{w, wsb};
         }
-        gws.two_halves = gws2.two_halves = !b16();
+        gws.keep_sums = gws2.keep_sums = true;
         if (concurrent) {
             // the side stream (weight gradients, Adam) and each layer's gradient
             // operands for it, in the step's precision
@@ -593,7 +593,7 @@ struct vkh_runner {
                 char *w = nullptr;
                 VKH_TRY(alloc(w, wsb));
                 gws2 = GemmWs{w, wsb};
-                gws2.two_halves = !b16();
+                gws2.keep_sums = true;
             }
         }
         VKH_TRY(alloc(ce_lse, T));
@@ -1109,7 +1109,6 @@ struct vkh_runner {
             for (int h = 0; h < 2 && st == VKH_OK; ++h) {
                 cur = h ? side : c0;
                 gws = h ? gws2 : w0;
-                gws.plan_rows = T0;
                 x_emb = x0 + h * th * D;
                 std::swap(acts, acts_h[h]);
                 st = layer_forward(l);
