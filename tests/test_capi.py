@@ -5,6 +5,7 @@ import ctypes as C
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -27,6 +28,14 @@ def test_header_compiles_as_c_and_cpp(tmp_path):
                             "-x", "c" if cc == "gcc" else "c++", str(src), "-o", str(out)],
                            capture_output=True, text=True)
         assert r.returncode == 0, r.stderr
+
+
+def test_library_loads_beside_torch():
+    """torch brings its own HIP runtime, which may be older than the one that the library
+    was linked with: a process that has torch in it already can load the library."""
+    r = subprocess.run([sys.executable, "-c", "import torch, valkyr_amd; valkyr_amd.lib()"], cwd=ROOT,
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
 
 
 def test_library_exports_every_declared_symbol():

@@ -80,6 +80,43 @@ def test_rmsnorm_backward_scratch_shared_across_streams():
         assert rel_l2(dw_ref, host(bdw)) < 1e-5
 
 
+def test_scratch_of_two_streams_beside_torch():
+    """The same, and LoRA (whose scratch holds packed operands), in a process that has
+    torch's own HIP runtime: where that has no stream identities, streams still do not
+    share scratch."""
+    import os
+    import subprocess
+    import sys
+
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = ("import torch; torch.zeros(1, device='cuda'); import test_gpu_kernels as t; "
+            "t.test_rmsnorm_backward_scratch_shared_across_streams(); t.run_lora_on_two_streams()")
+    r = subprocess.run([sys.executable, "-c", code], cwd=here, capture_output=True, text=True, timeout=100,
+                       env={**os.environ, "PYTHONPATH": os.pathsep.join([here, os.path.dirname(here)])})
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+def run_lora_on_two_streams():
+    from valkyr_amd import kernels as K
+    from valkyr_amd.device import Stream
+
+    M, N, Kd, r = 512, 768, 1024, 8
+    s1, s2 = Stream(), Stream()
+    runs = []
+    for i in range(6):
+        rng = np.random.default_rng(i)
+        x, w, a, b = (rng.standard_normal(s, dtype=np.float32) for s in ((M, Kd), (N, Kd), (r, Kd), (N, r)))
+        ref = O.round_bf16(x).astype(np.float64).reshape(M, Kd) @ O.round_bf16(w).reshape(N, Kd).T
+        ref += 0.5 * (x.astype(np.float64) @ a.T) @ b.T
+        runs.append((ref, zeros(M * N), [dev(t) for t in (x, w, a, b)], zeros(M * r)))
+    for i, (_, y, bufs, inter) in enumerate(runs):
+        K.lora_forward(*bufs, y, inter, M, N, Kd, r, 0.5, 1, stream=(s1 if i % 2 else s2))
+    s1.synchronize()
+    s2.synchronize()
+    for ref, y, _, _ in runs:
+        assert rel_l2(ref, host(y)) < 1e-5
+
+
 def test_swiglu_forward_backward():
     from valkyr_amd import kernels as K
 

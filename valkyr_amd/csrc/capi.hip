@@ -1,6 +1,7 @@
 // C ABI for the individual kernels plus the HIP plumbing (memory, streams,
 // events) a host without its own HIP bindings needs.  Every function checks
 // its arguments, enqueues, and reports launch errors as VKH_ERR_HIP.
+#include <dlfcn.h>
 #include <math.h>
 #include <stdio.h>
 #include <string.h>
@@ -68,14 +69,29 @@ static vkh_status rope_table_cached(int seq_len, int rot, float theta, const flo
 // different buffers, so no event is recorded or waited for per call (an
 // event record costs a few microseconds of device time).  Streams are told
 // apart by hipStreamGetId, which is unique for the life of the process, so a
-// stream created after another was destroyed never inherits its buffer.  A
+// stream created after another was destroyed never inherits its buffer.  The
+// runtime that a process has loaded may be older than that function (torch
+// brings its own), so it is looked up at run time; without it only the null
+// stream, which is never destroyed, keeps a buffer, and others take theirs in
+// stream order for the call, as calls of more than kLeaseMax do.  A
 // buffer is replaced only after its stream has drained; at most kMaxStreams
 // buffers are kept, and making room for another waits for the whole device.
 constexpr size_t kLeaseMax = 256ull << 20;  // the most that a call keeps here
 class ScratchLease {
   public:
+    ~ScratchLease() {
+        if (own_) (void)hipFreeAsync(own_, st_);
+    }
     vkh_status acquire(size_t bytes, hipStream_t st, void **out) {
         note_allocation();
+        static const auto stream_id =
+            (hipError_t(*)(hipStream_t, unsigned long long *))dlsym(RTLD_DEFAULT, "hipStreamGetId");
+        if (bytes > kLeaseMax || (!stream_id && st)) {
+            VKH_HIP(hipMallocAsync(&own_, bytes, st));
+            st_ = st;
+            *out = own_;
+            return VKH_OK;
+        }
         constexpr size_t kMaxStreams = 64;
         struct Buf {
             void *p = nullptr;
@@ -87,7 +103,7 @@ class ScratchLease {
         int dev = 0;
         VKH_HIP(hipGetDevice(&dev));
         unsigned long long sid = 0;
-        VKH_HIP(hipStreamGetId(st, &sid));
+        if (stream_id) VKH_HIP(stream_id(st, &sid));
         const auto key = std::make_pair(dev, sid);
         auto it = per_stream.find(key);
         if (it == per_stream.end()) {
@@ -122,6 +138,8 @@ class ScratchLease {
 
   private:
     std::unique_lock<std::mutex> lk_;
+    void *own_ = nullptr;  // of this call alone
+    hipStream_t st_ = nullptr;
 };
 
 }  // namespace vkh
@@ -391,22 +409,14 @@ vkh_status vkh_fa_backward_from_o(const vkh_attn_params *p, const void *q, const
 
 // ── GEMMs ──────────────────────────────────────────────────────────────
 
-// Workspace for one call.  Up to kLeaseMax it is the stream's kept scratch; more
-// is allocated in stream order and freed after the call's work.
+// Workspace for one call.
 extern "C++" {
 template <class F>
 static vkh_status with_ws(size_t bytes, hipStream_t st, const char *what, F &&f) {
     GemmWs ws{nullptr, bytes};
     ScratchLease lease;
-    const bool own = bytes > kLeaseMax;
-    if (own) {
-        note_allocation();
-        VKH_HIP(hipMallocAsync(&ws.p, bytes, st));
-    } else if (bytes) {
-        VKH_TRY(lease.acquire(bytes, st, &ws.p));
-    }
+    if (bytes) VKH_TRY(lease.acquire(bytes, st, &ws.p));
     const hipError_t e = f(ws);
-    if (own) (void)hipFreeAsync(ws.p, st);
     if (e != hipSuccess) return hip_fail(e, what);
     return VKH_OK;
 }
@@ -524,33 +534,6 @@ vkh_status vkh_linear_backward_dw_bf16(const void *dy, const void *x, float *dw,
     return linear(LinOp::TN, LinForm::BF16, dy, x, dw, M, N, K, "linear_backward_dw_bf16", S(stream));
 }
 
-// Scratch of a LoRA call: the stream's kept buffer, or stream-ordered memory where it is
-// larger than that keeps.
-extern "C++" {
-namespace {
-class LoraScratch {
-  public:
-    vkh_status acquire(size_t bytes, hipStream_t st) {
-        st_ = st;
-        if (bytes <= kLeaseMax) return lease_.acquire(bytes, st, (void **)&p);
-        note_allocation();
-        VKH_HIP(hipMallocAsync((void **)&p, bytes, st));
-        own_ = true;
-        return VKH_OK;
-    }
-    ~LoraScratch() {
-        if (own_) (void)hipFreeAsync(p, st_);
-    }
-    char *p = nullptr;
-
-  private:
-    ScratchLease lease_;
-    hipStream_t st_ = nullptr;
-    bool own_ = false;
-};
-}  // namespace
-}
-
 // The rank-r products go through the fp32 GEMMs (their few-tile plans split the long
 // sum; one block per column group walked it alone before, dA and dB 21 us each at 2048
 // tokens and 2560 columns), and the rank-r update rides in the base product's epilogue
@@ -580,9 +563,10 @@ vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, cons
             return VKH_OK;
         }
         const size_t wsb = std::max(lin_ws_bytes(LinOp::NT, form, x, w, M, N, K), g32_ws_bytes_for(M, r, K, kLoraChains));
-        LoraScratch sc;
-        if (wsb) VKH_TRY(sc.acquire(wsb, st));
-        const GemmWs ws{sc.p, wsb}, rows{sc.p, wsb, false, kLoraChains};
+        ScratchLease lease;
+        void *sc = nullptr;
+        if (wsb) VKH_TRY(lease.acquire(wsb, st, &sc));
+        const GemmWs ws{sc, wsb}, rows{sc, wsb, false, kLoraChains};
         VKH_HIP(g32_nt(x, K, a, K, inter, r, M, r, K, nullptr, 0, 1.f, 0.f, rows, st));
         VKH_HIP(lin_run(LinOp::NT, form, x, w, y, M, N, K, ws, st, &sb, (int)r, aor));
         return VKH_OK;
@@ -616,10 +600,11 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
         // fp32 factors and products
         size_t wsb = std::max({g32_ws_bytes_for(M, r, N, kLoraChains), g32_ws_bytes_for(r, K, M), g32_ws_bytes_for(N, r, M)});
         if (dx) wsb = std::max(wsb, lin_ws_bytes(LinOp::NN, form, dy, w, M, N, K));
-        LoraScratch sc;
-        VKH_TRY(sc.acquire(dyb_bytes + wsb, st));
-        float *dyB = (float *)sc.p;
-        const GemmWs ws{wsb ? sc.p + dyb_bytes : nullptr, wsb}, rows{ws.p, wsb, false, kLoraChains};
+        ScratchLease lease;
+        void *sc = nullptr;
+        VKH_TRY(lease.acquire(dyb_bytes + wsb, st, &sc));
+        float *dyB = (float *)sc;
+        const GemmWs ws{wsb ? (char *)sc + dyb_bytes : nullptr, wsb}, rows{ws.p, wsb, false, kLoraChains};
         sa.s[0].u = dyB;
         VKH_HIP(g32_nn(dy, N, b, r, dyB, r, M, N, r, 1.f, 0.f, rows, st));
         if (dx) VKH_HIP(lin_run(LinOp::NN, form, dy, w, dx, M, N, K, ws, st, &sa, (int)r, aor));
