@@ -80,6 +80,78 @@ def test_rmsnorm_backward_scratch_shared_across_streams():
         assert rel_l2(dw_ref, host(bdw)) < 1e-5
 
 
+def test_scratch_settles_and_is_bounded():
+    """Calls of slowly growing shapes replace their stream's scratch a few times, not at
+    every call; and however many streams ask, at most 1 GiB stays with them (the rest is
+    freed after its call), with right results past that bound too."""
+    import ctypes
+
+    import valkyr_amd as v
+    from valkyr_amd import kernels as K
+    from valkyr_amd.device import Stream, synchronize
+
+    note("scratch growth and bound")
+    N, Kd = 256, 256  # mixed products: the scratch holds the operands' packed copies
+    x, w = O.normal(40000 * Kd, 71), O.normal(N * Kd, 72)
+    bx, bw, y, st = dev(x), dev(w), zeros(40000 * N), Stream()
+    before = v.lib().vkh_allocation_count()
+    steps = range(4000, 40000, 1000)
+    for m in steps:
+        K.matmul_nt(bx, bw, y, m, N, Kd, 1, stream=st)
+    st.synchronize()
+    assert v.lib().vkh_allocation_count() - before <= len(steps) + 6  # a lease each, 2 -> 32 MiB
+    hip, free, total = v.lib(), ctypes.c_size_t(), ctypes.c_size_t()
+    M = 390000  # 200 MB of packed rows
+    big, out = zeros(M * Kd), zeros(M * N)
+    rows = dev(x[:64 * Kd])
+    used = []
+    streams = [Stream() for _ in range(9)]
+    for s in streams:
+        K.matmul_nt(big, bw, out, M, N, Kd, 1, stream=s)
+        K.matmul_nt(rows, bw, y, 64, N, Kd, 1, stream=s)
+        s.synchronize()
+        synchronize()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        used.append(total.value - free.value)
+        xr, wr = (O.round_bf16(t).reshape(-1, Kd).astype(np.float64) for t in (x[:64 * Kd], w))
+        assert rel_l2(xr @ wr.T, host(y, 64 * N)) < 1e-5
+        assert not np.any(host(out, 4096))
+    assert used[-1] - used[0] <= 1 << 30
+
+
+def test_scratch_of_threads_on_their_own_streams():
+    """Threads that call on streams of their own, each growing its scratch at its own pace."""
+    import threading
+
+    from valkyr_amd import kernels as K
+    from valkyr_amd.device import Stream
+
+    note("scratch of threads")
+    N, Kd = 192, 320
+    w = O.normal(N * Kd, 74)
+    bw, wr = dev(w), O.round_bf16(w).reshape(N, Kd).astype(np.float64)
+    bad = []
+
+    def work(i):
+        try:
+            st, rng = Stream(), np.random.default_rng(i)
+            for m in rng.integers(1, 6000, 12):
+                x = rng.standard_normal((m, Kd), dtype=np.float32)
+                bx, y = dev(x), zeros(m * N)
+                K.matmul_nt(bx, bw, y, int(m), N, Kd, 1, stream=st)
+                st.synchronize()
+                e = rel_l2(O.round_bf16(x).reshape(m, Kd).astype(np.float64) @ wr.T, y.to_numpy(np.float32))
+                if not e < 1e-5:
+                    bad.append((i, m, e))
+        except Exception as e:  # noqa: BLE001 - reported below
+            bad.append((i, e))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad, bad[:3]
+
+
 def test_scratch_of_two_streams_beside_torch():
     """The same, and LoRA (whose scratch holds packed operands), in a process that has
     torch's own HIP runtime: where that has no stream identities, streams still do not

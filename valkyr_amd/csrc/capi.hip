@@ -10,6 +10,7 @@
 #include <atomic>
 #include <iterator>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
 #include <vector>
@@ -63,20 +64,24 @@ static vkh_status rope_table_cached(int seq_len, int rot, float theta, const flo
 }
 
 // Scratch memory of the standalone entry points (gain partials, split-K
-// partials): one buffer per (device, stream), grown on demand and reused, so
-// a call does not allocate once its stream's buffer is large enough.  Calls
-// on one stream are ordered by the stream; calls on different streams use
-// different buffers, so no event is recorded or waited for per call (an
-// event record costs a few microseconds of device time).  Streams are told
-// apart by hipStreamGetId, which is unique for the life of the process, so a
-// stream created after another was destroyed never inherits its buffer.  The
-// runtime that a process has loaded may be older than that function (torch
-// brings its own), so it is looked up at run time; without it only the null
-// stream, which is never destroyed, keeps a buffer, and others take theirs in
-// stream order for the call, as calls of more than kLeaseMax do.  A
-// buffer is replaced only after its stream has drained; at most kMaxStreams
-// buffers are kept, and making room for another waits for the whole device.
-constexpr size_t kLeaseMax = 256ull << 20;  // the most that a call keeps here
+// partials, packed operands, parts of a split dK / dV): one buffer per (device,
+// stream), grown on demand and reused, so a call does not allocate once its
+// stream's buffer is large enough.  Calls on one stream are ordered by the stream;
+// calls on different streams use different buffers, so no event is recorded or
+// waited for per call (an event record costs a few microseconds of device time).
+// Streams are told apart by hipStreamGetId, which is unique for the life of the
+// process, so a stream created after another was destroyed never inherits its
+// buffer.  The runtime that a process has loaded may be older than that function
+// (torch brings its own), so it is looked up at run time; without it only the null
+// stream, which is never destroyed, keeps a buffer.
+//   * A buffer is replaced by one of at least twice its size (calls of varying
+//     shapes settle) after its stream has drained; only calls on that stream wait.
+//   * At most kMaxStreams buffers and kKeptTotal bytes are kept; room for another
+//     stream is made by freeing the buffers that no call holds, after the device
+//     has drained.
+//   * What is not kept (calls of more than kLeaseMax, calls past kKeptTotal, streams
+//     without an identity) is allocated in stream order and freed after the call.
+constexpr size_t kLeaseMax = 256ull << 20, kKeptTotal = 1ull << 30;
 class ScratchLease {
   public:
     ~ScratchLease() {
@@ -84,61 +89,115 @@ class ScratchLease {
     }
     vkh_status acquire(size_t bytes, hipStream_t st, void **out) {
         note_allocation();
-        static const auto stream_id =
-            (hipError_t(*)(hipStream_t, unsigned long long *))dlsym(RTLD_DEFAULT, "hipStreamGetId");
-        if (bytes > kLeaseMax || (!stream_id && st)) {
-            VKH_HIP(hipMallocAsync(&own_, bytes, st));
-            st_ = st;
-            *out = own_;
-            return VKH_OK;
+        const vkh_status s = get(bytes, st, out);
+        if (s != VKH_OK) (void)hipGetLastError();  // (an allocation's: the caller may do without)
+        if (s != VKH_OK || own_) {
+            lk_ = std::unique_lock<std::mutex>();
+            buf_.reset();
         }
-        constexpr size_t kMaxStreams = 64;
-        struct Buf {
-            void *p = nullptr;
-            size_t bytes = 0;
-        };
-        static std::mutex mu;
-        static std::map<std::pair<int, unsigned long long>, Buf> per_stream;
-        lk_ = std::unique_lock<std::mutex>(mu);  // held until the call has enqueued its work
-        int dev = 0;
-        VKH_HIP(hipGetDevice(&dev));
-        unsigned long long sid = 0;
-        if (stream_id) VKH_HIP(stream_id(st, &sid));
-        const auto key = std::make_pair(dev, sid);
-        auto it = per_stream.find(key);
-        if (it == per_stream.end()) {
-            if (per_stream.size() >= kMaxStreams) {
-                // every stream's work done: any kept buffer may go
-                VKH_HIP(hipDeviceSynchronize());
-                for (auto &kv : per_stream) {
-                    if (kv.first.first != dev) continue;
-                    VKH_HIP(hipFree(kv.second.p));
-                }
-                for (auto i = per_stream.begin(); i != per_stream.end();)
-                    i = i->first.first == dev ? per_stream.erase(i) : std::next(i);
-            }
-            it = per_stream.emplace(key, Buf{}).first;
-        }
-        Buf &b = it->second;
-        if (b.bytes < bytes) {
-            if (b.p) {
-                VKH_HIP(hipStreamSynchronize(st));  // its earlier uses are done
-                VKH_HIP(hipFree(b.p));
-                b.p = nullptr;
-                b.bytes = 0;
-            }
-            const size_t nb = std::max(bytes, (size_t)1 << 20);
-            note_allocation();
-            VKH_HIP(hipMalloc(&b.p, nb));
-            b.bytes = nb;
-        }
-        *out = b.p;
-        return VKH_OK;
+        return s;
     }
 
   private:
-    std::unique_lock<std::mutex> lk_;
-    void *own_ = nullptr;  // of this call alone
+    struct Buf {
+        std::mutex mu;  // held by a call until it has enqueued its work
+        void *p = nullptr;
+        size_t bytes = 0;
+    };
+    typedef std::pair<int, unsigned long long> Key;
+    struct Kept {
+        std::mutex mu;
+        std::map<Key, std::shared_ptr<Buf>> per_stream;
+        size_t total = 0;
+    };
+    static Kept &kept() {
+        static Kept k;
+        return k;
+    }
+
+    vkh_status get(size_t bytes, hipStream_t st, void **out) {
+        static const auto stream_id =
+            (hipError_t(*)(hipStream_t, unsigned long long *))dlsym(RTLD_DEFAULT, "hipStreamGetId");
+        if (bytes > kLeaseMax || (!stream_id && st)) return in_order(bytes, st, out);
+        Key key(0, 0);
+        VKH_HIP(hipGetDevice(&key.first));
+        if (stream_id) VKH_HIP(stream_id(st, &key.second));
+        VKH_TRY(find(key));
+        lk_ = std::unique_lock<std::mutex>(buf_->mu);
+        if (buf_->bytes < bytes) {
+            size_t nb = std::max({bytes, 2 * buf_->bytes, (size_t)1 << 20});
+            nb = std::min(nb, kLeaseMax);
+            if (!reserve(nb - buf_->bytes)) return in_order(bytes, st, out);
+            hipError_t e = buf_->p ? hipStreamSynchronize(st) : hipSuccess;  // its earlier uses are done
+            if (e == hipSuccess && buf_->p) e = hipFree(buf_->p);
+            buf_->p = nullptr;
+            note_allocation();
+            if (e == hipSuccess) e = hipMalloc(&buf_->p, nb);
+            if (e != hipSuccess) buf_->p = nullptr, give_back(nb);
+            buf_->bytes = buf_->p ? nb : 0;
+            if (e != hipSuccess) return hip_fail(e, "scratch");
+        }
+        *out = buf_->p;
+        return VKH_OK;
+    }
+
+    vkh_status in_order(size_t bytes, hipStream_t st, void **out) {
+        note_allocation();
+        VKH_HIP(hipMallocAsync(&own_, bytes, st));
+        st_ = st;
+        *out = own_;
+        return VKH_OK;
+    }
+
+    // buf_ = the stream's buffer (a new one is empty)
+    vkh_status find(const Key &key) {
+        constexpr size_t kMaxStreams = 64;
+        std::vector<std::shared_ptr<Buf>> idle;
+        {
+            Kept &k = kept();
+            std::lock_guard<std::mutex> lk(k.mu);
+            auto it = k.per_stream.find(key);
+            if (it == k.per_stream.end()) {
+                if (k.per_stream.size() >= kMaxStreams)
+                    for (auto i = k.per_stream.begin(); i != k.per_stream.end();) {
+                        // no call holds it, and none can find it from here on
+                        if (i->first.first == key.first && i->second.use_count() == 1) {
+                            idle.push_back(i->second);
+                            i = k.per_stream.erase(i);
+                        } else {
+                            ++i;
+                        }
+                    }
+                it = k.per_stream.emplace(key, std::make_shared<Buf>()).first;
+            }
+            buf_ = it->second;
+        }
+        if (idle.empty()) return VKH_OK;
+        const hipError_t e = hipDeviceSynchronize();
+        for (auto &b : idle) {
+            if (b->p) (void)hipFree(b->p);
+            give_back(b->bytes);
+        }
+        VKH_HIP(e);
+        return VKH_OK;
+    }
+
+    static bool reserve(size_t bytes) {
+        Kept &k = kept();
+        std::lock_guard<std::mutex> lk(k.mu);
+        if (k.total + bytes > kKeptTotal) return false;
+        k.total += bytes;
+        return true;
+    }
+    static void give_back(size_t bytes) {
+        Kept &k = kept();
+        std::lock_guard<std::mutex> lk(k.mu);
+        k.total -= bytes;
+    }
+
+    std::shared_ptr<Buf> buf_;
+    std::unique_lock<std::mutex> lk_;  // (released before buf_ is)
+    void *own_ = nullptr;              // of this call alone
     hipStream_t st_ = nullptr;
 };
 
@@ -299,14 +358,17 @@ vkh_status vkh_fa_bw_dq(const vkh_attn_params *p, const void *q, const void *k, 
     return VKH_OK;
 }
 
-// Scratch of a split dK / dV launch, where the grid asks for one (not under capture).
+// Scratch of a split dK / dV launch, where the grid asks for one (not under capture, nor
+// where there is no memory for it).
 static bool capturing(hipStream_t st);
 static vkh_status attn_parts(const AttnShape &s, AttnPtrs &a, ScratchLease &lease, hipStream_t st) {
     const int parts = fa_bw_parts(s, a.dt);
     const size_t b = fa_bw_parts_ws_bytes(s, parts);
     if (!b || b > kLeaseMax || capturing(st)) return VKH_OK;
     void *w = nullptr;
-    VKH_TRY(lease.acquire(b, st, &w));
+    const vkh_status got = lease.acquire(b, st, &w);
+    if (got == VKH_ERR_OUT_OF_MEMORY) return VKH_OK;
+    VKH_TRY(got);
     a.split_ws = (float *)w;
     a.split_parts = parts;
     return VKH_OK;
@@ -409,19 +471,6 @@ vkh_status vkh_fa_backward_from_o(const vkh_attn_params *p, const void *q, const
 
 // ── GEMMs ──────────────────────────────────────────────────────────────
 
-// Workspace for one call.
-extern "C++" {
-template <class F>
-static vkh_status with_ws(size_t bytes, hipStream_t st, const char *what, F &&f) {
-    GemmWs ws{nullptr, bytes};
-    ScratchLease lease;
-    if (bytes) VKH_TRY(lease.acquire(bytes, st, &ws.p));
-    const hipError_t e = f(ws);
-    if (e != hipSuccess) return hip_fail(e, what);
-    return VKH_OK;
-}
-}
-
 static bool capturing(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
@@ -434,17 +483,25 @@ static bool capturing(hipStream_t st) {
 // One contraction of a linear layer.  Operands that need a packed copy (fp32
 // operands in the bf16 precision; rows that are not whole 16-byte chunks) go
 // through the workspace to the DMA-staged kernels; while the stream is being
-// captured they take the generic kernel, and the others a plan without a split:
-// a graph outlives the call, so it holds no pointer into the stream's scratch
-// (which a later call may replace).  Against the generic
-// kernel, forward / dx / dW: 2048 tokens, 2560 x 2560, fp32 operands in bf16
-// products 55 / 55 / 63 us (645 / 443 / 351); bf16 operands of 2000 x 4100 x 4099
-// 156 / 143 / 117 us (455 / 638 / 533); fp32 of 1000 x 1500 x 3001 131 / 130 /
-// 117 us (205 / 156 / 211); 16 tokens, 1024 x 1024 mixed 15 / 15 / 8 us (41 / 29 / 7).
+// captured, or where there is no memory for the workspace, they take the generic
+// kernel, and the others a plan without a split: a graph outlives the call, so it
+// holds no pointer into the stream's scratch (which a later call may replace).
+// Against the generic kernel, forward / dx / dW: 2048 tokens, 2560 x 2560, fp32
+// operands in bf16 products 55 / 55 / 63 us (645 / 443 / 351); bf16 operands of
+// 2000 x 4100 x 4099 156 / 143 / 117 us (455 / 638 / 533); fp32 of 1000 x 1500 x 3001
+// 131 / 130 / 117 us (205 / 156 / 211); 16 tokens, 1024 x 1024 mixed 15 / 15 / 8 us
+// (41 / 29 / 7).
 static vkh_status linear(LinOp op, LinForm f, const void *a, const void *b, float *out, uint32_t M,
                          uint32_t N, uint32_t K, const char *what, hipStream_t st) {
-    const bool captured = capturing(st);
-    if (!M || !N || !K || (captured && lin_packs(op, f, a, b, M, N, K))) {
+    ScratchLease lease;
+    GemmWs ws{nullptr, 0};
+    if (M && N && K && !capturing(st)) {
+        ws.bytes = lin_ws_bytes(op, f, a, b, M, N, K);
+        const vkh_status got = ws.bytes ? lease.acquire(ws.bytes, st, &ws.p) : VKH_OK;
+        if (got == VKH_ERR_OUT_OF_MEMORY) ws = GemmWs{nullptr, 0};
+        else VKH_TRY(got);
+    }
+    if (!M || !N || !K || (!ws.p && lin_packs(op, f, a, b, M, N, K))) {
         const Precision pr = f == LinForm::F32 ? Precision::FP32 : Precision::BF16;
         const DType dt = f == LinForm::BF16 ? DType::BF16 : DType::F32;
         const Mat ma{a, (long)(op == LinOp::NT ? K : N), dt}, mb{b, (long)K, dt};
@@ -453,9 +510,9 @@ static vkh_status linear(LinOp op, LinForm f, const void *a, const void *b, floa
         else VKH_HIP(gemm_tn(pr, ma, mb, out, K, M, N, K, 1.f, 0.f, st));
         return VKH_OK;
     }
-    return with_ws(captured ? 0 : lin_ws_bytes(op, f, a, b, M, N, K), st, what, [&](const GemmWs &ws) {
-        return lin_run(op, f, a, b, out, M, N, K, ws, st);
-    });
+    const hipError_t e = lin_run(op, f, a, b, out, M, N, K, ws, st);
+    if (e != hipSuccess) return hip_fail(e, what);
+    return VKH_OK;
 }
 static inline LinForm form_of(uint32_t precision) {
     return PR(precision) == Precision::FP32 ? LinForm::F32 : LinForm::MIXED;
@@ -538,8 +595,8 @@ vkh_status vkh_linear_backward_dw_bf16(const void *dy, const void *x, float *dw,
 // sum; one block per column group walked it alone before, dA and dB 21 us each at 2048
 // tokens and 2560 columns), and the rank-r update rides in the base product's epilogue
 // instead of reading the output back (16 and 14 us): that layer, forward and backward
-// at rank 16, 213 -> 157 us.  A captured stream (no scratch) and operands of 2 GiB keep
-// the row and update kernels, with fp32 factors and products as well.  x A^T and dy B
+// at rank 16, 213 -> 157 us.  A captured stream (no scratch), no memory for the scratch and
+// operands of 2 GiB keep the row and update kernels, with fp32 factors and products as well.  x A^T and dy B
 // sum in at least the row kernel's eight partial sums.
 constexpr int kLoraChains = 8;
 vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, const float *b,
@@ -556,16 +613,21 @@ vkh_status vkh_lora_forward(const float *x, const float *w, const float *a, cons
     sb.s[0] = LoraSeg{0, (int)N, b, (long)r, 1, inter, (long)r};
     // fp32 factors and products where the shape allows
     if (lora_fast_ok(DType::F32, x, K, (int)r, sa) && lora_update_ok(y, N, (int)r, sb) && M) {
-        if (capturing(st) || !lin_lora_ok(LinOp::NT, form, M, N, K, sb, (int)r)) {
+        const size_t wsb = std::max(lin_ws_bytes(LinOp::NT, form, x, w, M, N, K), g32_ws_bytes_for(M, r, K, kLoraChains));
+        ScratchLease lease;
+        void *sc = nullptr;
+        bool tiled = !capturing(st) && lin_lora_ok(LinOp::NT, form, M, N, K, sb, (int)r);
+        if (tiled && wsb) {
+            const vkh_status got = lease.acquire(wsb, st, &sc);
+            if (got == VKH_ERR_OUT_OF_MEMORY) tiled = false;
+            else VKH_TRY(got);
+        }
+        if (!tiled) {
             VKH_TRY(linear(LinOp::NT, form, x, w, y, M, N, K, "lora_forward", st));
             VKH_HIP(lora_rows(DType::F32, x, K, (int)M, (int)r, sa, 1.f, st));
             VKH_HIP(lora_update(y, N, (int)M, (int)r, sb, aor, st));
             return VKH_OK;
         }
-        const size_t wsb = std::max(lin_ws_bytes(LinOp::NT, form, x, w, M, N, K), g32_ws_bytes_for(M, r, K, kLoraChains));
-        ScratchLease lease;
-        void *sc = nullptr;
-        if (wsb) VKH_TRY(lease.acquire(wsb, st, &sc));
         const GemmWs ws{sc, wsb}, rows{sc, wsb, false, kLoraChains};
         VKH_HIP(g32_nt(x, K, a, K, inter, r, M, r, K, nullptr, 0, 1.f, 0.f, rows, st));
         VKH_HIP(lin_run(LinOp::NT, form, x, w, y, M, N, K, ws, st, &sb, (int)r, aor));
@@ -596,13 +658,18 @@ vkh_status vkh_lora_backward(const float *dy, const float *x, const float *w, co
     const bool fast = lora_fast_ok(DType::F32, dy, N, (int)r, sb) && lora_fast_ok(DType::F32, x, K, (int)r, sdA) &&
                       lora_fast_ok(DType::F32, dy, N, (int)r, sdB) && M &&
                       (!dx || lora_update_ok(dx, K, (int)r, sa));
-    if (fast && !capturing(st) && (!dx || lin_lora_ok(LinOp::NN, form, M, N, K, sa, (int)r))) {
-        // fp32 factors and products
-        size_t wsb = std::max({g32_ws_bytes_for(M, r, N, kLoraChains), g32_ws_bytes_for(r, K, M), g32_ws_bytes_for(N, r, M)});
+    bool tiled = fast && !capturing(st) && (!dx || lin_lora_ok(LinOp::NN, form, M, N, K, sa, (int)r));
+    ScratchLease lease;
+    void *sc = nullptr;
+    size_t wsb = 0;
+    if (tiled) {
+        wsb = std::max({g32_ws_bytes_for(M, r, N, kLoraChains), g32_ws_bytes_for(r, K, M), g32_ws_bytes_for(N, r, M)});
         if (dx) wsb = std::max(wsb, lin_ws_bytes(LinOp::NN, form, dy, w, M, N, K));
-        ScratchLease lease;
-        void *sc = nullptr;
-        VKH_TRY(lease.acquire(dyb_bytes + wsb, st, &sc));
+        const vkh_status got = lease.acquire(dyb_bytes + wsb, st, &sc);
+        if (got == VKH_ERR_OUT_OF_MEMORY) tiled = false;
+        else VKH_TRY(got);
+    }
+    if (tiled) {  // fp32 factors and products
         float *dyB = (float *)sc;
         const GemmWs ws{wsb ? (char *)sc + dyb_bytes : nullptr, wsb}, rows{ws.p, wsb, false, kLoraChains};
         sa.s[0].u = dyB;
