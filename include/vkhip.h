@@ -523,16 +523,19 @@ vkh_status vkh_fa_bw_dkv(const vkh_attn_params *p, const void *q, const void *k,
 
 /* The FA-2 backward of one attention call after vkh_fa_bw_d (the
  * fa_bw_dkv.comp + fa_bw_dq.comp pair of the reference's attention
- * backward): dK, dV, dQ fp32 (overwrite).  With bf16 operands (head_dim 64 or
- * 128, n_q and n_kv multiples of 64, self-attention when causal):
- *   - head_dim 128, an even number of query heads per KV head and n_kv a
- *     multiple of 128: a dK/dV kernel and a dQ kernel that each form S and
- *     dP themselves (no workspace: vkh_fa_backward_workspace_bytes is 0);
- *   - otherwise dK/dV write dS = P (dP - D) once as bf16 into `workspace` and
- *     dQ = dS K is a GEMM.
- * Other shapes run the two kernels above.  `workspace` may be NULL (allocated
- * per call on the stream when needed) or hold
- * vkh_fa_backward_workspace_bytes(p) bytes. */
+ * backward): dK, dV, dQ fp32 (overwrite).  A dK/dV kernel and a dQ kernel that
+ * each form S and dP themselves; with bf16 operands they take head_dim 64 and 128,
+ * any lengths (n_q == n_kv when causal) and any head group, where rows are 16-byte
+ * aligned and a sequence's views stay under 1 GiB.  Elsewhere bf16 calls whose n_q
+ * and n_kv are multiples of 64 (self-attention when causal) write dS = P (dP - D)
+ * once as bf16 into a workspace and form dQ = dS K as a GEMM, and others take
+ * general kernels.  `workspace` may be NULL or hold
+ * vkh_fa_backward_workspace_bytes(p) bytes, what a call with aligned operands
+ * needs (0 wherever the first pair takes it); a call that needs more allocates it
+ * on the stream.  Where key blocks are too few for the chip, this call,
+ * vkh_fa_bw_dkv and vkh_fa_backward_from_o also use up to 256 MiB of the library's
+ * per-stream scratch for the parts of a split dK/dV (not while the stream is being
+ * captured, nor where there is no memory for it: then they run unsplit). */
 size_t vkh_fa_backward_workspace_bytes(const vkh_attn_params *p);
 vkh_status vkh_fa_backward(const vkh_attn_params *p, const void *q, const void *k, const void *v,
                            const void *dout, const float *lse, const float *d, float *dq,

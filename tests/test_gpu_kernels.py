@@ -1107,18 +1107,19 @@ def test_flash_attention_bf16_mfma(case):
     note(f"  vs the bf16-operand oracle dQ={e16[0]:.2e} dK={e16[1]:.2e} dV={e16[2]:.2e}")
     # same roundings at the same points: only fp32 summation order differs
     assert all(x < 1e-4 for x in e16), e16
-    # the fused backward (bf16 dS workspace + dQ GEMM where the shape allows)
+    # the one-call backward: the two kernels above, or the fused form's own pair of them
+    # (its dS form is test_flash_attention_bf16_ds_workspace's)
     ws_bytes = K.fa_backward_workspace_bytes(p)
-    note(f"  fused path: workspace {ws_bytes} bytes")
+    assert ws_bytes == 0  # aligned operands recompute dS on every shape
     bdq, bdk, bdv = zeros(dq.size), zeros(dk.size), zeros(dv.size)
-    ws = zeros(ws_bytes // 4 + 1) if ws_bytes else None
+    ws = None
     K.fa_backward(p, qb, kb, vb, dob16, dev(lse_r), dev(d), bdq, bdk, bdv, ws)
     f = [rel_l2(dq_r, host(bdq)), rel_l2(dk_r, host(bdk)), rel_l2(dv_r, host(bdv))]
     g = [rel_l2(dq, host(bdq)), rel_l2(dk, host(bdk)), rel_l2(dv, host(bdv))]
-    note(f"  fused vs oracle dQ={f[0]:.2e} dK={f[1]:.2e} dV={f[2]:.2e}; "
+    note(f"  one call vs oracle dQ={f[0]:.2e} dK={f[1]:.2e} dV={f[2]:.2e}; "
          f"vs two-kernel dQ={g[0]:.2e} dK={g[1]:.2e} dV={g[2]:.2e}")
     assert all(x < BF16_TOL for x in f), f
-    # same dS values and products, only the dQ summation order differs
+    # same dS values and products, only summation orders differ
     assert all(x < 1e-5 for x in g), g
     _check_from_o(p, qb, kb, vb, o, dob16, lse_r, dO.size, ws)
 
@@ -1224,6 +1225,48 @@ def test_flash_attention_bf16_rows_without_gradient(n, H, Hkv, hd):
     _, _, dq2, _, dv2 = run(q, do, lse, d)
     assert np.all(dq2[7] == 0) and np.array_equal(np.delete(dq2, 7, 0), np.delete(dq, 7, 0))
     assert rel_l2(dv, dv2) < 1e-6
+
+
+@pytest.mark.parametrize("case", [  # (n, H, Hkv, hd, causal, B)
+    (64, 2, 2, 64, True, 1), (256, 4, 2, 64, True, 2), (192, 3, 1, 64, False, 1),
+    (192, 4, 4, 128, True, 2), (320, 6, 2, 128, True, 1), (128, 5, 5, 128, False, 1)])
+def test_flash_attention_bf16_ds_workspace(case):
+    """The backward that keeps dS in a workspace (the training step's on 64-wide heads, odd
+    head groups and few key blocks; standalone where dQ is not 16-byte aligned, as here):
+    against the oracle's bf16-operand model and the recompute kernels.  A caller's
+    workspace of the size asked for, which is none, is not written."""
+    import valkyr_amd as v
+    from valkyr_amd import kernels as K
+
+    n, H, Hkv, hd, causal, B = case
+    note(f"fa bf16 dS workspace {case}")
+    (qb, q), (kb, k), (vb, vv) = (bf16_dev(O.normal(B * n * h * hd, s)) for h, s in ((H, 51), (Hkv, 52), (Hkv, 53)))
+    dob, do = bf16_dev(O.normal(B * n * H * hd, 54, 0.1))
+    o, lse, *_ = _fa_oracle(q, k, vv, do, B, n, n, H, Hkv, hd, causal)
+    d = O.fa_bw_d(o, do, B * n, H, hd)
+    p = K.attn_params(n, n, H, Hkv, hd, causal, B, K.BF16)
+    assert K.fa_backward_workspace_bytes(p) == 0
+    got, count = [], []
+    ws = dev(np.full(4096, 7, np.uint8))
+    for skew in (0, 4):
+        bdq, bdk, bdv = zeros(q.size + 1), zeros(k.size), zeros(k.size)
+        before = v.lib().vkh_allocation_count()
+        K.fa_backward(p, qb, kb, vb, dob, dev(lse), dev(d), bdq.offset(skew), bdk, bdv, ws.offset(64))
+        count.append(v.lib().vkh_allocation_count() - before)
+        got.append([host(bdq)[skew // 4:][:q.size], host(bdk), host(bdv)])
+    assert count[1] > count[0]  # the dS memory: the other path ran
+    assert np.all(host(ws, 4096, np.uint8) == 7)
+    m16 = []
+    for b in range(B):
+        sq, sk, sr = (slice(b * n * w, (b + 1) * n * w) for w in (H * hd, Hkv * hd, H))
+        m16.append(O.flash_backward(q[sq], k[sk], vv[sk], o[sq], do[sq], lse[sr], n, n, H, Hkv, hd, causal,
+                                    bf16_ops=True))
+    for i, name in enumerate(("dQ", "dK", "dV")):
+        ref = np.concatenate([x[i] for x in m16])
+        e = rel_l2(ref, got[1][i]), rel_l2(got[0][i], got[1][i])
+        note(f"  {name} vs the bf16-operand oracle {e[0]:.1e}, vs the recompute kernels {e[1]:.1e}")
+        # the bounds of test_flash_attention_bf16_mfma
+        assert e[0] < 1e-4 and e[1] < 1e-5, (name, e)
 
 
 # n_q != n_kv in bf16 (the reference's causal limit k <= q + (n_kv - n_q),

@@ -398,7 +398,12 @@ vkh_status vkh_fa_bw_dkv(const vkh_attn_params *p, const void *q, const void *k,
 size_t vkh_fa_backward_workspace_bytes(const vkh_attn_params *p) {
     if (!p || check_attn(p) != VKH_OK) return 0;
     const AttnShape s = attn_shape(p);
-    return p->dtype == VKH_BF16 && fa_bw_fused_ok(s) ? fa_bw_ws_bytes(s, fa_bw_v4_ok(s)) : 0;
+    // aligned operands of this shape (others allocate for their call)
+    const float *al = (const float *)256;
+    AttnPtrs a = attn_ptrs(p, al, al, al, al, al, al);
+    a.dq = a.dk = a.dv = (float *)al;
+    if (p->dtype != VKH_BF16 || !fa_bw_fused_ok(s) || attn_general(s, a)) return 0;
+    return fa_bw_ws_bytes(s, fa_bw_v4_ok(s));
 }
 
 vkh_status vkh_fa_backward(const vkh_attn_params *p, const void *q, const void *k, const void *v,
@@ -419,16 +424,19 @@ vkh_status vkh_fa_backward(const vkh_attn_params *p, const void *q, const void *
         VKH_HIP(fa_bw_dq(s, a, st));
         return VKH_OK;
     }
-    void *ws = workspace;
-    // the recompute kernels whenever the shape allows (they need no workspace)
+    // the fused form's own recompute kernels, or dS in a workspace (the caller's holds it
+    // only where vkh_fa_backward_workspace_bytes says so)
     const bool v4 = fa_bw_v4_ok(s);
     const size_t wsb = fa_bw_ws_bytes(s, v4);
-    if (!ws && wsb) {
+    const bool own = wsb && (!workspace || vkh_fa_backward_workspace_bytes(p) < wsb);
+    void *ws = workspace;
+    a.split_ws = nullptr;
+    if (own) {
         note_allocation();
         VKH_HIP(hipMallocAsync(&ws, wsb, st));
     }
     const hipError_t e = fa_bw_fused(s, a, (bf16 *)ws, v4, st);
-    if (!workspace && wsb) (void)hipFreeAsync(ws, st);
+    if (own) (void)hipFreeAsync(ws, st);
     if (e != hipSuccess) return hip_fail(e, "fa_backward");
     return VKH_OK;
 }

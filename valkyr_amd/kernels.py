@@ -65,9 +65,9 @@ def fa_backward_workspace_bytes(p):
 
 
 def fa_backward(p, q, k, v, dout, lse, d, dq, dk, dv, workspace=None, stream=None):
-    """dK, dV and dQ of one attention call (after fa_bw_d); bf16 shapes take
-    the fused dS path (workspace of fa_backward_workspace_bytes(p) bytes, or
-    None to allocate per call)."""
+    """dK, dV and dQ of one attention call (after fa_bw_d).  workspace:
+    fa_backward_workspace_bytes(p) bytes, or None to allocate per call what the
+    call needs."""
     check(lib().vkh_fa_backward(C.byref(p), _p(q), _p(k), _p(v), _p(dout), _p(lse), _p(d),
                                 _p(dq), _p(dk), _p(dv), _p(workspace), _s(stream)))
 
