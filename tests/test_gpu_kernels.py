@@ -7,6 +7,7 @@ bf16-operand contractions (compared with the oracle run on the same
 bf16-rounded inputs).  Elementwise kernels that restate the reference formula
 with identical fp32 rounding are held to much tighter bounds where that holds.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -84,8 +85,6 @@ def test_scratch_settles_and_is_bounded():
     """Calls of slowly growing shapes replace their stream's scratch a few times, not at
     every call; and however many streams ask, at most 1 GiB stays with them (the rest is
     freed after its call), with right results past that bound too."""
-    import ctypes
-
     import valkyr_amd as v
     from valkyr_amd import kernels as K
     from valkyr_amd.device import Stream, synchronize
@@ -1487,20 +1486,36 @@ def test_flash_attention_bf16_full_size_invariants():
             assert rel_l2(dk_ref[i], dk5[b, j, kv]) < 1e-2, ("dK", b, kv, j)
 
 
-@pytest.mark.parametrize("call", ["fp32", "mixed", "bf16", "lora fp32", "lora mixed"])
-def test_linear_products_on_a_captured_stream(call):
-    """A few-tile product and a LoRA layer recorded into a graph on a stream that has run
-    nothing yet: the recording succeeds (no scratch of the stream is taken), and each
-    replay gives the eager call's values up to the order of fp32 sums (2 sqrt(K) 2^-23,
-    both sides in different splits), also after a larger eager call on that stream."""
-    import ctypes
+def _replays(hip, st, record, check, between, n=3):
+    """Records `record()` on `st` into a graph and replays it n times: check() after each,
+    between() (eager work on that stream) before the next."""
+    graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(st.handle, 0) == 0
+    record()
+    assert hip.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(n):
+        assert hip.hipGraphLaunch(ex, st.handle) == 0
+        st.synchronize()
+        check()
+        between()
+        st.synchronize()
+    assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
 
+
+@pytest.mark.parametrize("used", [False, True], ids=["new-stream", "used-stream"])
+@pytest.mark.parametrize("call", ["fp32", "mixed", "bf16", "lora fp32", "lora mixed"])
+def test_linear_products_on_a_captured_stream(call, used):
+    """A few-tile product and a LoRA layer recorded into a graph, on a stream that has run
+    nothing yet and on one that keeps scratch already: the recording succeeds, and each
+    replay gives the eager call's values up to the order of fp32 sums (2 sqrt(K) 2^-23,
+    both sides in different splits), also after eager calls on that stream whose larger
+    scratch has replaced the one that was there at the recording."""
     from valkyr_amd import kernels as K
     from valkyr_amd import lib
     from valkyr_amd.device import Stream
 
-    note(f"captured {call}")
-    hip = lib()  # the runtime that the library is linked with
+    note(f"captured {call} {used}")
     M, N, Kd, r = 16, 1024, 3072, 16
     rng = np.random.default_rng(5)
     x, w, a, b = (rng.standard_normal(s, dtype=np.float32) for s in ((M, Kd), (N, Kd), (r, Kd), (N, r)))
@@ -1510,27 +1525,108 @@ def test_linear_products_on_a_captured_stream(call):
         bx, bw, ba, bb = dev(x), dev(w), dev(a), dev(b)
     inter, st = zeros(M * r), Stream()
 
-    def run(y, stream, n=N):
+    def run(y, stream):
         if call == "bf16":
-            K.matmul_nt_bf16(bx, bw, y, M, n, Kd, stream=stream)
+            K.matmul_nt_bf16(bx, bw, y, M, N, Kd, stream=stream)
         elif call.startswith("lora"):
-            K.lora_forward(bx, bw, ba, bb, y, inter, M, n, Kd, r, 0.5, int(call == "lora mixed"), stream=stream)
+            K.lora_forward(bx, bw, ba, bb, y, inter, M, N, Kd, r, 0.5, int(call == "lora mixed"), stream=stream)
         else:
-            K.matmul_nt(bx, bw, y, M, n, Kd, int(call == "mixed"), stream=stream)
+            K.matmul_nt(bx, bw, y, M, N, Kd, int(call == "mixed"), stream=stream)
 
-    eager, y, other = zeros(M * N), zeros(M * N), zeros(M * N)
-    run(eager, Stream())
-    ref = host(eager)
-    graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
-    assert hip.hipStreamBeginCapture(st.handle, 0) == 0
-    run(y, st)
-    assert hip.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0
-    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
-    for _ in range(3):
-        y.upload(np.zeros(M * N, np.float32))
-        assert hip.hipGraphLaunch(ex, st.handle) == 0
-        st.synchronize()
+    eager, y = zeros(M * N), zeros(M * N)
+    run(eager, st if used else Stream())
+    ref, rows = host(eager), [4096]
+    big = zeros(16384 * 1024), zeros(64 * 1024), zeros(16384 * 64)
+
+    def check():
         assert rel_l2(ref, host(y)) < 2 * math.sqrt(Kd) * 2.0 ** -23
-        run(other, st, N - 64)
-        st.synchronize()
-    assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
+        y.upload(np.zeros(M * N, np.float32))
+
+    def between():  # packed copies of 8, 16, 32 MiB, past the 1 MiB and what the call took
+        rows[0] = min(2 * rows[0], 16384)
+        K.matmul_nt(*big, rows[0], 64, 1024, 1, stream=st)
+
+    _replays(lib(), st, lambda: run(y, st), check, between)
+
+
+@pytest.mark.parametrize("form,n,H,Hkv,hd", [("bf16", 1000, 4, 2, 128), ("bf16", 640, 2, 2, 64),
+                                             ("fp32", 500, 4, 2, 64)])
+def test_attention_backward_on_a_captured_stream(form, n, H, Hkv, hd):
+    """The attention backward whose dK/dV is split between blocks when called eagerly, and
+    is not in a graph: dQ has the eager call's bits, dK and dV its values up to the order
+    of fp32 sums of n H / Hkv terms (all of one size here: 2 sqrt(terms) 2^-23 of the norm),
+    at every replay, also after a larger eager call has replaced the stream's scratch."""
+    from valkyr_amd import kernels as K
+    from valkyr_amd import lib
+    from valkyr_amd.device import Stream
+
+    note(f"captured attention backward {form} n={n} {H}/{Hkv} hd={hd}")
+    up = (lambda t: bf16_dev(t)[0]) if form == "bf16" else dev
+    q, do = (O.normal(n * H * hd, s) for s in (81, 82))
+    k, vv = (O.normal(n * Hkv * hd, s) for s in (83, 84))
+    p = K.attn_params(n, n, H, Hkv, hd, True, 1, K.BF16 if form == "bf16" else K.F32)
+    bq, bk, bv, bdo = up(q), up(k), up(vv), up(do)
+    o, lse, d = zeros(q.size), zeros(n * H), zeros(n * H)
+    K.fa_forward(p, bq, bk, bv, o, lse)
+    K.fa_bw_d(p, o, dev(do), d)
+    st, out = Stream(), [zeros(q.size), zeros(k.size), zeros(k.size)]
+    eager = [zeros(q.size), zeros(k.size), zeros(k.size)]
+    K.fa_backward(p, bq, bk, bv, bdo, lse, d, *eager, stream=st)
+    ref = [host(t) for t in eager]
+    big = zeros(16384 * 1024), zeros(64 * 1024), zeros(16384 * 64)
+
+    def check():
+        got = [host(t) for t in out]
+        assert np.array_equal(ref[0], got[0])
+        bound = 2 * math.sqrt(n * H / Hkv) * 2.0 ** -23
+        assert rel_l2(ref[1], got[1]) < bound and rel_l2(ref[2], got[2]) < bound
+        for t in out:
+            t.fill_zero()
+
+    _replays(lib(), st, lambda: K.fa_backward(p, bq, bk, bv, bdo, lse, d, *out, stream=st), check,
+             lambda: K.matmul_nt(*big, 16384, 64, 1024, 1, stream=st))
+
+
+def test_linear_product_of_packed_operands_of_2_gib():
+    """A mixed product whose packed copy reaches 2 GiB (row chunks of the DMA-staged
+    kernels): rows at both ends and around the chunk's edge."""
+    from valkyr_amd import kernels as K
+
+    M, N, Kd = (1 << 27) + 200, 8, 8
+    note(f"packed operand of {M * Kd * 2} bytes")
+    rng = np.random.default_rng(7)
+    spots = {0: 300, (1 << 27) - 40: 240, 77777777: 64}
+    bx, by = zeros(M * Kd), zeros(M * N)
+    w = rng.standard_normal((N, Kd), dtype=np.float32)
+    bw, rows = dev(w), {}
+    from valkyr_amd._lib import check, lib
+
+    for at, cnt in spots.items():
+        rows[at] = rng.standard_normal((cnt, Kd), dtype=np.float32)
+        check(lib().vkh_memcpy_h2d(bx.offset(at * Kd * 4), rows[at].ctypes.data_as(ctypes.c_void_p), rows[at].nbytes))
+    K.matmul_nt(bx, bw, by, M, N, Kd, 1)
+    wr = O.round_bf16(w).reshape(N, Kd).astype(np.float64)
+    for at, x in rows.items():
+        got = np.empty((len(x), N), np.float32)
+        host(by, 1)
+        check(lib().vkh_memcpy_d2h(got.ctypes.data_as(ctypes.c_void_p), by.offset(at * N * 4), got.nbytes))
+        assert rel_l2(O.round_bf16(x).reshape(-1, Kd).astype(np.float64) @ wr.T, got) < 1e-6
+
+
+def test_lora_layer_whose_scratch_is_not_kept():
+    """A LoRA layer whose packed operands are over the 256 MiB that a stream keeps."""
+    from valkyr_amd import kernels as K
+
+    M, N, Kd, r = 70000, 64, 2048, 16
+    note("lora scratch of 287 MB")
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((M, Kd), dtype=np.float32)
+    w, a, b = (0.1 * rng.standard_normal(s, dtype=np.float32) for s in ((N, Kd), (r, Kd), (N, r)))
+    bufs, y, inter = [dev(t) for t in (x, w, a, b)], zeros(M * N), zeros(M * r)
+    K.lora_forward(*bufs, y, inter, M, N, Kd, r, 0.5, 1)
+    at = rng.integers(0, M, 500)
+    xs = x[at]
+    ref = O.round_bf16(xs).reshape(-1, Kd).astype(np.float64) @ O.round_bf16(w).reshape(N, Kd).T
+    ref += 0.5 * (xs.astype(np.float64) @ a.T) @ b.T
+    assert rel_l2(ref, host(y).reshape(M, N)[at]) < 1e-5
+    assert rel_l2(xs.astype(np.float64) @ a.T, host(inter).reshape(M, r)[at]) < 1e-6

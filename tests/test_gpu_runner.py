@@ -231,6 +231,23 @@ def test_step_parity_bf16(variant):
         assert rel_l2(m.tensor(0, *k), r.get(0, *k)) < 1e-2
 
 
+ODD_GROUP = dict(n_heads=3, n_kv_heads=1)
+
+
+@pytest.mark.parametrize("variant", [
+    dict(vocab_size=1003), dict(vocab_size=1003, tied_embeddings=1, n_seqs=2, seq_len=64),
+    dict(HD128, vocab_size=4099, n_seqs=2), dict(seq_len=100), dict(seq_len=161, n_seqs=2),
+    dict(HD128, seq_len=100, n_seqs=2), dict(HD128, seq_len=161, vocab_size=1001),
+    dict(ODD_GROUP, seq_len=161), dict(HD128, **{**ODD_GROUP, "seq_len": 100, "n_seqs": 2}),
+    dict(ODD_GROUP, seq_len=1, n_seqs=3)],
+    ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()))
+def test_step_parity_bf16_odd_sizes(variant):
+    """The bf16 step where rows of the vocabulary are no whole 16-byte chunks (padded dz and
+    kept logits) and where sequences are no whole tiles (the recompute backward's general
+    form on the step's strided gradient rows), as test_step_parity_bf16."""
+    test_step_parity_bf16(dict({"n_layers": 1}, **variant))
+
+
 # Per-layer activation recompute (config 5's mode) at 5 layers, so that the
 # two shared activation sets, the two gradient-copy sets and the three-deep
 # dy ring are all reused: the same kernels run on the same inputs, so every
