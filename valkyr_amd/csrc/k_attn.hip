@@ -26,7 +26,9 @@
 // visits every key tile, fa_bw_dq.comp:114).  dQ is produced by its own
 // kernel, so no atomics and the result is deterministic.
 //
-// fp32 path (precision = fp32, parity mode): one wave per query (or key) row,
+// fp32 path (precision = fp32, parity mode): the tile kernels of k_attn_f32.hip where
+// fa_f32m_ok holds; otherwise (other head widths, unaligned rows, a training step's
+// sequences that are no whole tiles) the kernels here, one wave per query (or key) row,
 // scalar FMAs with wave reductions, structured like the reference shaders.
 #include "gemm16.hpp"
 #include "ops.hpp"
@@ -1065,7 +1067,9 @@ __global__ __launch_bounds__(dkv3::NT3, 1) void fa_bwd_dkv3_k(AttnShape s, AttnP
     }
 }
 
-// ── backward v4 (head_dim 128, an even number of query heads per KV head) ──
+// ── backward v4: the recompute kernels ─────────────────────────────────────
+// head_dim 128, an even number of query heads per KV head and whole 128-key blocks; the
+// general form (RAG, HDR below) takes 64-wide heads, odd head groups and any lengths.
 //
 // Two kernels that each form S and dP themselves (seven score-sized products
 // per (query, key) pair instead of five), so nothing of size
@@ -1172,7 +1176,8 @@ __global__ __launch_bounds__(NWV * 64, 1) void fa_bwd_dkv4_k(AttnShape s, AttnPt
     const float c2 = s.inv_sqrt_dim * LOG2E;
 
     // K and V of the slice as B operands: lane (g, c16) holds key 16 ks + c16,
-    // d = 32 ds + 8 g .. + 7 (n_kv is a multiple of 128: no edge)
+    // d = 32 ds + 8 g .. + 7 (RAG: keys past the end read the last one's row; without it
+    // n_kv is a multiple of 128)
     bf16x8 kr[KS][DSR];
     {
         const bf16 *kb = (const bf16 *)p.k + ((long)b * s.n_kv + kw0 + c16) * p.ldk + kvh * HDR + 8 * g;
@@ -1568,8 +1573,8 @@ constexpr int TILE = BN * HD * 2;  // 8 KB: one K or V tile
 constexpr int NBUF = 3;
 }  // namespace dq4
 
-// dQ.  Block = BQ (256 or 128) queries of one (sequence, head) on NWV waves
-// (8: two per SIMD, BQ / 8 queries each); wave w owns
+// dQ.  Block = BQ (256, 128 or 64) queries of one (sequence, head) on NWV waves
+// (8: two per SIMD, BQ / 8 queries each; 4 for 64); wave w owns
 // the 16-row query sub-tiles Q0 + 16 (NWV j + w), interleaved so that under a
 // causal mask every wave has work until the block's last key tile.  Q and dO
 // of those rows sit in VGPRs as B operands; per 32-key tile (K and V by DMA,
@@ -2310,8 +2315,8 @@ void launch_dkv4_ragged(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
     if (parts > 1) dkv_sum(s, q, st);
 }
 
-// dQ blocks of 256 queries (8 waves), of 128 (8 waves) or of 64 (4 waves): of 128 where 256 would leave fewer blocks than
-// CUs: there a causal grid is also short of work at its end, since a block's
+// dQ blocks of 256 queries (8 waves), of 128 (8 waves) or of 64 (4 waves): of 128 where
+// 256 would leave fewer blocks than CUs: there a causal grid is also short of work at its end, since a block's
 // work grows with its last query (config 3, 4 x 512: 128 blocks of 256 rows,
 // the later block of each sequence twice the earlier); with 256-query blocks
 // filling the chip, 128 loses (config 2: 0.268 against 0.250 ms per call)
@@ -2347,7 +2352,7 @@ void launch_dq4(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
 
 // The recompute kernels on lengths that are not whole tiles, or with an odd head
 // group: head_dim 64 or 128, n_q == n_kv under a causal mask, 16-byte aligned rows under
-// 2 GiB a sequence.
+// 1 GiB a sequence (the DMA offsets are 32-bit and run on past the last row's tile).
 static bool v4_ragged_ok(const AttnShape &s, const AttnPtrs &p) {
     auto al = [](const void *x, long ld) { return ((uintptr_t)x & 15) == 0 && ld % 8 == 0; };
     return p.dt == DType::BF16 && bf16_ok(s) && (!s.causal || s.n_q == s.n_kv) && s.n_kv > 0 &&

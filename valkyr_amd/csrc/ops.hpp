@@ -388,9 +388,12 @@ hipError_t fa_bw_d_bf16(const AttnShape &s, const bf16 *o, long ldo, const bf16 
                         float *d, hipStream_t st);
 hipError_t fa_bw_dq(const AttnShape &s, const AttnPtrs &p, hipStream_t st);
 hipError_t fa_bw_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st);
-// The whole bf16 backward from bf16 O (p.o16; D is written) on shapes the fused form
-// does not take, with the recompute kernels' ragged form; false, launching nothing,
-// where they do not apply (fa_bw_dkv and fa_bw_dq pick it by the same rule).
+// The recompute kernels' general form, of lengths, head groups and widths that the fused
+// form's own pair does not take (fa_bw_dkv and fa_bw_dq pick it by the same rule, for the
+// training step's sequences of no whole tiles too).  fa_bw_ragged: the whole bf16 backward
+// from bf16 O (p.o16; D is written); false, launching nothing, where it does not apply.
+// fa_bw_parts: blocks per key block of a split dK / dV, whose sums take
+// fa_bw_parts_ws_bytes in split_ws.
 int fa_bw_parts(const AttnShape &s, DType dt);
 void fa_dkv_sum(const AttnShape &s, const AttnPtrs &p, hipStream_t st);  // adds the parts
 bool fa_bw_ragged_ok(const AttnShape &s, const AttnPtrs &p);
