@@ -130,7 +130,12 @@ Plan plan_few(const GemmShape &s, const GemmWs &ws, bool f32, bool mn_a, const P
     };
     tile(Pick::T128x64, Pick::T128x64ks2, 128, 64);
     tile(Pick::T64, Pick::T64ks2, 64, 64);
-    if (f32 || !mn_a) tile(Pick::T32x64, Pick::T32x64ks2, 32, 64);
+    // In bf16 up to one 32 x 64 tile per CU: beyond, several of them on a CU are bound by
+    // their operand traffic, which the model does not see (128 x 8200 over K = 1016, 516
+    // tiles: 21.7 us against 14.4 on 64 x 64 and 14.6 on 128 x 64; of 260 drawn products
+    // the most that one lost to 128 x 64 was 24 %, and 7 % with this line).
+    if (f32 || (!mn_a && (long)ceil_div(s.M, 32) * ceil_div(s.N, 64) <= 256))
+        tile(Pick::T32x64, Pick::T32x64ks2, 32, 64);
     if (f32) tile(Pick::T32, Pick::T32ks2, 32, 32);
     return best;
 }
