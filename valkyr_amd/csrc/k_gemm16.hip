@@ -75,12 +75,13 @@ size_t ws_for(const Plan &p, const GemmShape &s) {
 // bf16, 0.36 in fp32, where the matrix cores are the slower part).  The tile and
 // the split over K come from a model of the launch: its fixed cost, the slower of
 // the slab chain, the CU's matrix time when blocks share it, operand traffic and
-// output traffic, and the reduce launch of a split.  Fitted (least squares on the
-// logarithm, 11-15 % rms) to 2800 timings of 16-512 rows over widths 256-32000 in
-// the three layouts; the pick is 4-6 % above the best of the table on average, and
-// against the 128 x 64 tiles before it: fp32 16 x 1024 x 3072 107 -> 9.7 us,
-// 128 x 512 x 512 22 -> 7.3, 512 x 1024 x 1024 39 -> 16; bf16 16 x 1024 x 3072
-// 18.8 -> 7.3 us, 128 x 1024 x 1024 10.6 -> 6.5, 512 x 768 x 32000 95 -> 55.
+// output traffic, and the reduce launch of a split.  Fitted by least squares on the
+// logarithm to timings of 16-512 rows over widths 256-32000 in the three layouts; of
+// the 5668 in profiles/gemm_few_tiles.csv it is off by 12 % (fp32) and 17 % (bf16) rms
+// with no bias, and the pick is 4 % above the best of a product's on average.  Against
+// the 128 x 64 tiles before it: fp32 16 x 1024 x 3072 107 -> 9.7 us, 128 x 512 x 512
+// 22 -> 7.3, 512 x 1024 x 1024 39 -> 16; bf16 16 x 1024 x 3072 18.8 -> 7.3 us,
+// 128 x 1024 x 1024 10.6 -> 6.5, 512 x 768 x 32000 95 -> 55.
 // fp32 also has the in-block split (two wave groups on the halves of K, no reduce
 // launch).  `base` is the plan of the large tiles, whose number of partial sums over K
 // is the least that the pick may have: fewer, longer chains would round worse (one
