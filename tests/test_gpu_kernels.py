@@ -957,7 +957,7 @@ def _fa_f32_all(p, n, H, q, k, v, do, lse=None, d=None):
     return [t.reshape(n, H) if i in (1, 2) else t.reshape(-1, H, hd) for i, t in enumerate(out)]
 
 
-@pytest.mark.parametrize("n,hd", [(37, 64), (100, 128)])
+@pytest.mark.parametrize("n,hd", [(37, 64), (100, 128), (8, 128)])
 def test_flash_attention_fp32_ragged_masked_rows(n, hd):
     """A query whose scores are all -inf (keys of -inf against a positive query, as an
     additive mask leaves them) gets O = 0, LSE = -inf and dQ = 0, and no gradient flows

@@ -2100,7 +2100,7 @@ __global__ void fa_fwd_f32_k(AttnShape s, const float *q, long ldq, const float 
         const float sc = dot_wave(qr, kr) * s.inv_sqrt_dim;
         const float mn = fmaxf(m, sc);
         const float so = m == -INFINITY ? 0.f : expf(m - mn);
-        const float pv = expf(sc - mn);
+        const float pv = sc == -INFINITY ? 0.f : expf(sc - mn);  // (also where every score so far is)
         load_row(vr, v + kt * ldv + kvh * hd, hd, lane);
 #pragma unroll
         for (int i = 0; i < MAXE; ++i) orow[i] = orow[i] * so + pv * vr[i];

@@ -649,10 +649,27 @@ bool fa_f32m_ok(const AttnShape &s) {
            s.n_kv_heads > 0 && s.n_heads % s.n_kv_heads == 0;
 }
 
+// Ragged calls of a few steps a row on at most 4096 rows (16 waves a CU) stay on the
+// per-row kernels (a wave a row): a tile launch is mostly empty tiles there.  8 tokens,
+// 16 / 8 heads of 128: forward 6.2 us there against 7.0, dQ 6.1 against 8.3, dK/dV 12
+// against 18; 24 tokens: 14.1, 13.3 and 32 against 7.3, 9.0 and 19.  One or two queries
+// against many keys: 1 x 4000, dK/dV 21 against 33 us (64-wide: 16 against 29 in groups of
+// four heads; 19 against 19 in groups of two, 15 against 13 without).
+static bool few_steps(const AttnShape &s, int n_kv_max) {
+    return !whole_tiles(s) && s.n_kv <= n_kv_max && (long)s.n_batch * s.n_q * s.n_heads <= 4096;
+}
+static bool few_steps_dkv(const AttnShape &s) {
+    if (whole_tiles(s)) return false;
+    const int w = s.head_dim / 64, hpk = s.n_heads / s.n_kv_heads;
+    if ((long)s.n_batch * s.n_kv * s.n_kv_heads <= 4096 && s.n_q <= 6 * w && s.n_q * hpk <= 8 + 8 * w)
+        return true;
+    return s.n_q <= w && hpk <= 8 && (w == 2 || hpk >= 4);
+}
+
 bool fa_f32m_fwd(const AttnShape &s, const float *q, long ldq, const float *k, long ldk,
                  const float *v, long ldv, float *o, long ldo, float *lse, hipStream_t st) {
     if (!fa_f32m_ok(s) || !al16(q) || !al16(k) || !al16(v) || !al16(o) || ldq % 4 || ldk % 4 ||
-        ldv % 4 || ldo % 4)
+        ldv % 4 || ldo % 4 || few_steps(s, s.head_dim / 16))
         return false;
     const dim3 grid(s.n_heads * s.n_batch, (s.n_q + 63) / 64);
     const bool zz = fits_two_per_cu((long)grid.x * grid.y);
@@ -670,7 +687,8 @@ static bool ptrs_ok(const AttnPtrs &p) {
 }
 
 bool fa_f32m_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
-    if (!fa_f32m_ok(s) || !ptrs_ok(p) || !al16(p.dk) || !al16(p.dv) || p.lddk % 4 || p.lddv % 4)
+    if (!fa_f32m_ok(s) || !ptrs_ok(p) || !al16(p.dk) || !al16(p.dv) || p.lddk % 4 || p.lddv % 4 ||
+        few_steps_dkv(s))
         return false;
     if (p.qk_fp32 && !fa_f32m_qk_ok(s, p)) return false;
     AttnPtrs q = p;
@@ -691,7 +709,7 @@ bool fa_f32m_dkv(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
 }
 
 bool fa_f32m_dq(const AttnShape &s, const AttnPtrs &p, hipStream_t st) {
-    if (!fa_f32m_ok(s) || !ptrs_ok(p) || !al16(p.dq) || p.lddq % 4) return false;
+    if (!fa_f32m_ok(s) || !ptrs_ok(p) || !al16(p.dq) || p.lddq % 4 || few_steps(s, 3 * s.head_dim / 32)) return false;
     if (p.qk_fp32 && !fa_f32m_qk_ok(s, p)) return false;
     const dim3 grid(s.n_heads * s.n_batch, (s.n_q + 63) / 64);
     const bool zz = fits_two_per_cu((long)grid.x * grid.y);
