@@ -499,17 +499,34 @@ static bool capturing(hipStream_t st) {
 // 2000 x 4100 x 4099 156 / 143 / 117 us (455 / 638 / 533); fp32 of 1000 x 1500 x 3001
 // 131 / 130 / 117 us (205 / 156 / 211); 16 tokens, 1024 x 1024 mixed 15 / 15 / 8 us
 // (41 / 29 / 7).
+//
+// Products of so few terms that the packing launch is most of the call stay on the
+// generic kernel: sums of up to 64 terms onto 1.25 M outputs, of 32 onto 2.5 M, and of
+// 128 where its 128 x 128 tiles fill the chip (mixed dW of 16 to 64 tokens, 1000 x 1000:
+// 6.7 us against 8.1; 16 x 30000 over 96: 7.9 to 9.5 against 10.7 to 11.8).  Beyond,
+// the packed form is: 2048 x 1024 over 64 8.8 against 11.3, 2048 x 4096 over 64 the same
+// way; over 472 timed products of 1 to 300 terms this line is 1 % above the better form.
+static bool few_terms(LinOp op, uint32_t M, uint32_t N, uint32_t K) {
+    const uint32_t rows = op == LinOp::TN ? N : M, cols = op == LinOp::NT ? N : K,
+                   terms = op == LinOp::NT ? K : op == LinOp::NN ? N : M;
+    const double out = (double)rows * cols;
+    return (terms <= 64 && out <= 1.25e6) || (terms <= 32 && out <= 2.5e6) ||
+           (terms <= 128 && out <= 2.5e6 && (uint64_t)ceil_div(rows, 128) * ceil_div(cols, 128) >= 192);
+}
+
 static vkh_status linear(LinOp op, LinForm f, const void *a, const void *b, float *out, uint32_t M,
                          uint32_t N, uint32_t K, const char *what, hipStream_t st) {
     ScratchLease lease;
     GemmWs ws{nullptr, 0};
-    if (M && N && K && !capturing(st)) {
+    const bool any = M && N && K, packs = any && lin_packs(op, f, a, b, M, N, K);
+    const bool generic = !any || (packs && few_terms(op, M, N, K));
+    if (!generic && !capturing(st)) {
         ws.bytes = lin_ws_bytes(op, f, a, b, M, N, K);
         const vkh_status got = ws.bytes ? lease.acquire(ws.bytes, st, &ws.p) : VKH_OK;
         if (got == VKH_ERR_OUT_OF_MEMORY) ws = GemmWs{nullptr, 0};
         else VKH_TRY(got);
     }
-    if (!M || !N || !K || (!ws.p && lin_packs(op, f, a, b, M, N, K))) {
+    if (generic || (packs && !ws.p)) {
         const Precision pr = f == LinForm::F32 ? Precision::FP32 : Precision::BF16;
         const DType dt = f == LinForm::BF16 ? DType::BF16 : DType::F32;
         const Mat ma{a, (long)(op == LinOp::NT ? K : N), dt}, mb{b, (long)K, dt};
