@@ -93,6 +93,7 @@ def test_scratch_settles_and_is_bounded():
     N, Kd = 256, 256  # mixed products: the scratch holds the operands' packed copies
     x, w = O.normal(40000 * Kd, 71), O.normal(N * Kd, 72)
     bx, bw, y, st = dev(x), dev(w), zeros(40000 * N), Stream()
+    synchronize()
     before = v.lib().vkh_allocation_count()
     steps = range(4000, 40000, 1000)
     for m in steps:
@@ -123,7 +124,7 @@ def test_scratch_of_threads_on_their_own_streams():
     import threading
 
     from valkyr_amd import kernels as K
-    from valkyr_amd.device import Stream
+    from valkyr_amd.device import DeviceBuffer, Stream
 
     note("scratch of threads")
     N, Kd = 192, 320
@@ -136,7 +137,7 @@ def test_scratch_of_threads_on_their_own_streams():
             st, rng = Stream(), np.random.default_rng(i)
             for m in rng.integers(1, 6000, 12):
                 x = rng.standard_normal((m, Kd), dtype=np.float32)
-                bx, y = dev(x), zeros(m * N)
+                bx, y = dev(x), DeviceBuffer(int(m) * N * 4)
                 K.matmul_nt(bx, bw, y, int(m), N, Kd, 1, stream=st)
                 st.synchronize()
                 e = rel_l2(O.round_bf16(x).reshape(m, Kd).astype(np.float64) @ wr.T, y.to_numpy(np.float32))
@@ -169,7 +170,7 @@ def test_scratch_of_two_streams_beside_torch():
 
 def run_lora_on_two_streams():
     from valkyr_amd import kernels as K
-    from valkyr_amd.device import Stream
+    from valkyr_amd.device import Stream, synchronize
 
     M, N, Kd, r = 512, 768, 1024, 8
     s1, s2 = Stream(), Stream()
@@ -180,6 +181,7 @@ def run_lora_on_two_streams():
         ref = O.round_bf16(x).astype(np.float64).reshape(M, Kd) @ O.round_bf16(w).reshape(N, Kd).T
         ref += 0.5 * (x.astype(np.float64) @ a.T) @ b.T
         runs.append((ref, zeros(M * N), [dev(t) for t in (x, w, a, b)], zeros(M * r)))
+    synchronize()  # (the buffers' memset is on the null stream)
     for i, (_, y, bufs, inter) in enumerate(runs):
         K.lora_forward(*bufs, y, inter, M, N, Kd, r, 0.5, 1, stream=(s1 if i % 2 else s2))
     s1.synchronize()
@@ -1489,17 +1491,20 @@ def test_flash_attention_bf16_full_size_invariants():
 def _replays(hip, st, record, check, between, n=3):
     """Records `record()` on `st` into a graph and replays it n times: check() after each,
     between() (eager work on that stream) before the next."""
+    from valkyr_amd.device import synchronize
+
     graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
     assert hip.hipStreamBeginCapture(st.handle, 0) == 0
     record()
     assert hip.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0
     assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
     for _ in range(n):
+        synchronize()  # (memsets are on the null stream)
         assert hip.hipGraphLaunch(ex, st.handle) == 0
         st.synchronize()
         check()
+        synchronize()
         between()
-        st.synchronize()
     assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
@@ -1513,7 +1518,7 @@ def test_linear_products_on_a_captured_stream(call, used):
     scratch has replaced the one that was there at the recording."""
     from valkyr_amd import kernels as K
     from valkyr_amd import lib
-    from valkyr_amd.device import Stream
+    from valkyr_amd.device import Stream, synchronize
 
     note(f"captured {call} {used}")
     M, N, Kd, r = 16, 1024, 3072, 16
@@ -1534,6 +1539,7 @@ def test_linear_products_on_a_captured_stream(call, used):
             K.matmul_nt(bx, bw, y, M, N, Kd, int(call == "mixed"), stream=stream)
 
     eager, y = zeros(M * N), zeros(M * N)
+    synchronize()
     run(eager, st if used else Stream())
     ref, rows = host(eager), [4096]
     big = zeros(16384 * 1024), zeros(64 * 1024), zeros(16384 * 64)
@@ -1558,7 +1564,7 @@ def test_attention_backward_on_a_captured_stream(form, n, H, Hkv, hd):
     at every replay, also after a larger eager call has replaced the stream's scratch."""
     from valkyr_amd import kernels as K
     from valkyr_amd import lib
-    from valkyr_amd.device import Stream
+    from valkyr_amd.device import Stream, synchronize
 
     note(f"captured attention backward {form} n={n} {H}/{Hkv} hd={hd}")
     up = (lambda t: bf16_dev(t)[0]) if form == "bf16" else dev
@@ -1571,6 +1577,7 @@ def test_attention_backward_on_a_captured_stream(form, n, H, Hkv, hd):
     K.fa_bw_d(p, o, dev(do), d)
     st, out = Stream(), [zeros(q.size), zeros(k.size), zeros(k.size)]
     eager = [zeros(q.size), zeros(k.size), zeros(k.size)]
+    synchronize()
     K.fa_backward(p, bq, bk, bv, bdo, lse, d, *eager, stream=st)
     ref = [host(t) for t in eager]
     big = zeros(16384 * 1024), zeros(64 * 1024), zeros(16384 * 64)
