@@ -546,6 +546,15 @@ def test_linear_products_of_any_width_and_alignment(form, shape, skew):
         assert rel_l2(ref, host(got)) < 1e-6 + 4 * math.sqrt(n) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("form", ["fp32", "mixed", "bf16"])
+@pytest.mark.parametrize("shape", [(64, 1001, 1001), (65, 1001, 1001), (32, 2049, 1025), (33, 2049, 1025),
+                                   (1001, 1001, 64), (16, 24583, 30)])
+def test_linear_products_of_few_terms(form, shape):
+    """Either side of the lines between the generic kernel and packed operands, held to the
+    bounds of test_linear_products_of_any_width_and_alignment."""
+    test_linear_products_of_any_width_and_alignment(form, shape, 0)
+
+
 @pytest.mark.parametrize("shape", [(2048, 3072, 1024), (2000, 3072, 1000), (256, 192, 128),
                                    (130, 100, 72)])
 def test_gate_up_swiglu_matches_two_passes(shape):
@@ -938,6 +947,17 @@ def test_flash_attention_fp32_ragged_lengths(case):
     """The fp32 matrix-core kernels on lengths that are not whole tiles (one row, a row
     past a tile, causal with more keys than queries, either side longer without a mask),
     held to test_flash_attention_fp32's bounds."""
+    test_flash_attention_fp32(case)
+
+
+@pytest.mark.parametrize("case", [  # (n_q, n_kv, H, Hkv, hd, causal, B)
+    (4, 4, 4, 2, 64, True, 2), (5, 5, 4, 2, 64, True, 2), (7, 7, 4, 2, 64, True, 1), (8, 8, 4, 2, 128, True, 3),
+    (9, 9, 4, 2, 128, True, 1), (12, 12, 4, 4, 128, True, 1), (13, 13, 4, 4, 128, True, 1),
+    (1, 300, 8, 2, 64, True, 1), (1, 300, 8, 4, 64, False, 1), (2, 300, 8, 2, 128, True, 1),
+    (3, 300, 8, 2, 128, False, 1), (600, 3, 8, 2, 128, False, 1), (1, 1, 32, 2, 128, True, 1)])
+def test_flash_attention_fp32_few_tokens(case):
+    """Either side of the lines between the per-row and the tile kernels, held to
+    test_flash_attention_fp32's bounds."""
     test_flash_attention_fp32(case)
 
 
