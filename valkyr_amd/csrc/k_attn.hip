@@ -1096,7 +1096,7 @@ VKH_DEV void st_row_bf16(bf16 *row, const float (&v)[8][4], int g) {
 
 namespace dkv4 {
 constexpr int HD = 128, BM = 32, BN = 128;
-constexpr int DS = HD / 32, DSUB = HD / 16, QS = BM / 16;
+constexpr int QS = BM / 16;
 constexpr int TILE = BM * HD * 2;           // 8 KB: one Q or dO tile
 constexpr int NBUF = 3;                     // tile buffers (two DMA batches in flight)
 constexpr int STREAM = NBUF * 2 * TILE;     // 48 KB: one head group's Q / dO tiles
@@ -1568,7 +1568,7 @@ __global__ __launch_bounds__(256) void fa_dkv_combine_k(AttnShape s, AttnPtrs p)
 
 namespace dq4 {
 constexpr int HD = 128, BN = 32;
-constexpr int KS = BN / 16, DS = HD / 32, DSUB = HD / 16;
+constexpr int KS = BN / 16;
 constexpr int TILE = BN * HD * 2;  // 8 KB: one K or V tile
 constexpr int NBUF = 3;
 }  // namespace dq4
